@@ -5,7 +5,7 @@
 // I of the rebuild list.  One wave64 owns a chunk: both 32-lane halves hold
 // the 32 i-atoms of block I in registers, so i-forces accumulate without
 // any cross-lane or memory traffic, and no j-side force is ever written
-// (every pair is visited from both sides; energies take half per visit).
+// (every pair is visited from both sides; energies are taken on one).
 //
 // Per tile and step: the tile is skipped when the current block boxes are
 // farther apart than rcut; otherwise the j-atoms within rcut of the current
@@ -145,50 +145,109 @@ __device__ __forceinline__ void pair_ef(const NbConst &c, float qq, float c12, f
   }
 }
 
-// FP64 pair energy at effective distance r (energy steps only): the total
-// potential is a small difference of large pair sums, so the sum is built
-// from FP64 pair energies (same pair set and parameters as the forces).
+// ---- FP64 pair energies of energy steps ----------------------------------
+// The total potential is a small difference of large pair sums, so the sum
+// is built from FP64 pair energies.  1/x and 1/sqrt(x) are the hardware
+// approximation refined by Newton steps, and erfc is the fit of
+// fit_erfc.py times exp by range reduction and its Taylor series: about 90
+// FP64 instructions a pair without a branch, where the library's erfc walks
+// through three ranges, of which a wave takes all.  Relative error of erfc
+// below 4e-14 on [0, 6] (tests/test_erfc64.py).
+__device__ __forceinline__ double rcp_d(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  y = fma(fma(-x, y, 1.0), y, y);
+  return fma(fma(-x, y, 1.0), y, y);
+}
+__device__ __forceinline__ double rsqrt_d(double x) {
+  double y = __builtin_amdgcn_rsq(x);
+  y = fma(y, fma(-0.5 * x * y, y, 0.5), y);
+  return fma(y, fma(-0.5 * x * y, y, 0.5), y);
+}
+// (polynomial coefficients in constant memory: read into scalar registers;
+// as literals they are kept in two vector registers each)
+__constant__ double c_exp[13] = {1.0,        1.0,         1.0 / 2,      1.0 / 6,       1.0 / 24,       1.0 / 120,      1.0 / 720,
+                                 1.0 / 5040, 1.0 / 40320, 1.0 / 362880, 1.0 / 3628800, 1.0 / 39916800, 1.0 / 479001600};
+__constant__ double c_erfc[BM_ERFCD_DEG + 1] = {BM_ERFCD_COEF};
+__device__ __forceinline__ double exp_d(double v) {
+  const double n = rint(v * 1.4426950408889634);
+  // ln 2 as its float value and the rest
+  double r = fma(n, -(double)0.693147182464599609375f, v);
+  r = fma(n, 1.904654299957767878541823e-09, r);
+  double p = c_exp[12];   // sum r^k / k!, |r| <= ln 2 / 2
+#pragma unroll
+  for (int k = 11; k >= 0; k--) p = fma(p, r, c_exp[k]);
+  return ldexp(p, (int)n);
+}
+__device__ __forceinline__ double erfc_d(double x) {
+  const double xc = fmin(x, BM_ERFCD_XMAX);
+  const double y = fma(-2.0 * BM_ERFCD_A, rcp_d(xc + BM_ERFCD_A), 1.0);
+  double p = c_erfc[BM_ERFCD_DEG];
+#pragma unroll
+  for (int k = BM_ERFCD_DEG - 1; k >= 0; k--) p = fma(p, y, c_erfc[k]);
+  return p * exp_d(-x * x);
+}
+
+struct EnConst {
+  double rc, rs, beta, rcinv;
+  double rc3i, rc6i, k6, k12, dv6, dv12;   // VFSWITCH
+  double A, B, C, D, dvc, roff2;           // FSWITCH
+  double rul3i;                            // VSWITCH
+};
+
+__device__ __forceinline__ EnConst make_energy_const(const Dev &d) {
+  EnConst c;
+  c.rc = d.rcd; c.rs = d.rsd; c.beta = d.betad;
+  c.rcinv = 1.0 / c.rc;
+  const double rc3 = c.rc * c.rc * c.rc, rs3 = c.rs * c.rs * c.rs;
+  c.rc3i = 1 / rc3;
+  c.rc6i = c.rc3i * c.rc3i;
+  c.k6 = rc3 / (rc3 - rs3);
+  c.k12 = rc3 * rc3 / (rc3 * rc3 - rs3 * rs3);
+  c.dv6 = 1 / (rc3 * rs3);
+  c.dv12 = c.dv6 * c.dv6;
+  const double roff2 = c.rc * c.rc, ron2 = c.rs * c.rs;
+  const double g = 1 / ((roff2 - ron2) * (roff2 - ron2) * (roff2 - ron2));
+  c.roff2 = roff2;
+  c.rul3i = g;
+  c.A = roff2 * roff2 * (roff2 - 3 * ron2) * g;
+  c.B = 6 * roff2 * ron2 * g;
+  c.C = -(ron2 + roff2) * g;
+  c.D = 0.4 * g;
+  c.dvc = 8 * (ron2 * roff2 * (c.rc - c.rs) - (roff2 * roff2 * c.rc - ron2 * ron2 * c.rs) / 5) * g;
+  return c;
+}
+
+// energy of a pair at effective distance r (rinv = 1/r)
 template <int ELEC, int VDW>
-__device__ double pair_energy_d(const Dev &d, double qq, double c12, double c6, double r) {
-  const double rc = d.rcd, rs = d.rsd, rinv = 1.0 / r;
+__device__ __forceinline__ double pair_energy_sum(const EnConst &c, double qq, double c12, double c6, double r,
+                                                double rinv) {
+  const double r2 = r * r;
   double e;
   if (ELEC == BM_PME) {
-    e = qq * erfc(d.betad * r) * rinv;
+    e = qq * erfc_d(c.beta * r) * rinv;
   } else if (ELEC == BM_FSWITCH) {
-    const double roff2 = rc * rc, ron2 = rs * rs;
-    const double ginv = 1 / ((roff2 - ron2) * (roff2 - ron2) * (roff2 - ron2));
-    const double A = roff2 * roff2 * (roff2 - 3 * ron2) * ginv, B = 6 * roff2 * ron2 * ginv;
-    const double C = -(ron2 + roff2) * ginv, D = 2 * ginv / 5;
-    const double dvc = 8 * (ron2 * roff2 * (rc - rs) - (roff2 * roff2 * rc - ron2 * ron2 * rs) / 5) * ginv;
-    const double r3 = r * r * r, r5 = r3 * r * r;
-    e = (r <= rs) ? qq * (rinv + dvc)
-                  : qq * (A * (rinv - 1 / rc) + B * (rc - r) + C * (roff2 * rc - r3) + D * (roff2 * roff2 * rc - r5));
+    const double r3 = r2 * r, r5 = r3 * r2;
+    const double in = rinv + c.dvc;
+    const double out = c.A * (rinv - c.rcinv) + c.B * (c.rc - r) + c.C * (c.roff2 * c.rc - r3) +
+                       c.D * (c.roff2 * c.roff2 * c.rc - r5);
+    e = qq * (r <= c.rs ? in : out);
   } else {
-    e = qq * (rinv - 2 / rc + r / (rc * rc));
+    e = qq * (rinv - 2 * c.rcinv + r * (c.rcinv * c.rcinv));
   }
   const double rinv3 = rinv * rinv * rinv, rinv6 = rinv3 * rinv3;
   if (VDW == BM_VFSWITCH) {
-    const double rc3 = rc * rc * rc, rs3 = rs * rs * rs;
-    if (r < rs) {
-      const double dv6 = 1 / (rc3 * rs3);
-      e += c12 * (rinv6 * rinv6 - dv6 * dv6) - c6 * (rinv6 - dv6);
-    } else {
-      const double k6 = rc3 / (rc3 - rs3), k12 = rc3 * rc3 / (rc3 * rc3 - rs3 * rs3);
-      const double a3 = rinv3 - 1 / rc3, a6 = rinv6 - 1 / (rc3 * rc3);
-      e += c12 * k12 * a6 * a6 - c6 * k6 * a3 * a3;
-    }
+    const bool in = r < c.rs;
+    const double a3 = rinv3 - c.rc3i, a6 = rinv6 - c.rc6i;
+    const double rep = in ? rinv6 * rinv6 - c.dv12 : c.k12 * a6 * a6;
+    const double att = in ? rinv6 - c.dv6 : c.k6 * a3 * a3;
+    e += c12 * rep - c6 * att;
   } else if (VDW == BM_VSWITCH) {
-    if (r < rs) {
-      e += c12 * rinv6 * rinv6 - c6 * rinv6;
-    } else {
-      const double c2of = rc * rc, c2on = rs * rs;
-      const double rul3 = (c2of - c2on) * (c2of - c2on) * (c2of - c2on);
-      const double rijl = c2on - r * r, riju = c2of - r * r;
-      e += riju * riju * (riju - 3 * rijl) / rul3 * (c12 * rinv6 - c6) * rinv6;
-    }
+    const double rijl = c.rs * c.rs - r2, riju = c.roff2 - r2;
+    const double sw = r < c.rs ? 1.0 : riju * riju * (riju - 3 * rijl) * c.rul3i;
+    e += sw * (c12 * rinv6 - c6) * rinv6;
   } else {
-    const double r6 = r * r * r * r * r * r, rc6 = rc * rc * rc * rc * rc * rc;
-    e += c12 * (rinv6 * rinv6 + 2 * r6 / (rc6 * rc6 * rc6) - 3 / (rc6 * rc6)) - c6 * (rinv6 + r6 / (rc6 * rc6) - 2 / rc6);
+    const double r6 = r2 * r2 * r2, rc12i = c.rc6i * c.rc6i;
+    e += c12 * (rinv6 * rinv6 + 2 * r6 * rc12i * c.rc6i - 3 * rc12i) - c6 * (rinv6 + r6 * rc12i - 2 * c.rc6i);
   }
   return e;
 }
@@ -238,6 +297,15 @@ __device__ __forceinline__ bool near_box(const Dev &d, uint4 ci, uint4 hi, uint4
   return g2 <= rc2 * 1.0001f;
 }
 
+// an atom within rcut of the current box of block J
+__device__ __forceinline__ bool atom_near_block(const Dev &d, uint4 p, int J, float rc2) {
+  const uint4 c = d.bbc[J], h = d.bbh[J];
+  const float gx = fmaxf((fabsf((float)(int)(p.x - c.x)) - (float)h.x) * d.fracscale[0], 0.f);
+  const float gy = fmaxf((fabsf((float)(int)(p.y - c.y)) - (float)h.y) * d.fracscale[1], 0.f);
+  const float gz = fmaxf((fabsf((float)(int)(p.z - c.z)) - (float)h.z) * d.fracscale[2], 0.f);
+  return fmaf(gx, gx, fmaf(gy, gy, gz * gz)) <= rc2 * 1.0001f;
+}
+
 // i-atom of a lane, held for a whole chunk
 struct IAtom {
   uint4 p;       // fractional coordinates, charge bits
@@ -257,7 +325,7 @@ constexpr int kVdwLdsMax = 6144;
 // entries 1, 3, ...).  CHK: the tile has exclusions or is the diagonal
 // tile (I == J), so the exclusion bit and j == i are tested.
 template <int ELEC, int VDW, bool ENERGY, bool ALCH, bool SOFT, bool CHK>
-__device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const IAtom &ia, int li,
+__device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const EnConst &ec, const IAtom &ia, int li,
                                            int half, const uint4 *sp, const int2 *spr, const float *slo,
                                            const unsigned char *sjx, const float2 *svdw, int nj,
                                            unsigned em, bool self, float &fx, float &fy, float &fz,
@@ -305,13 +373,14 @@ __device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const
     if (ALCH) f *= s;
     if (ENERGY) {
       // FP64 pair energy from the exact integer displacement and FP64
-      // charges / LJ parameters; half per visit
+      // charges / LJ parameters
       const double2 ljd = d.vdwd[vi];
       const double qjd = (double)__uint_as_float(pj.w) + (double)slo[jl];
       const double ddx = (double)(int)(ia.p.x - pj.x) * d.ddscale[0];
       const double ddy = (double)(int)(ia.p.y - pj.y) * d.ddscale[1];
       const double ddz = (double)(int)(ia.p.z - pj.z) * d.ddscale[2];
-      double rd = sqrt(ddx * ddx + ddy * ddy + ddz * ddz);
+      const double dd2 = ddx * ddx + ddy * ddy + ddz * ddz;
+      double rid = rsqrt_d(dd2), rd = dd2 * rid;
       double sd = 1.0;
       if (ALCH && alchPair) {
         const double li_d = (bi & 0xFFFF) ? d.lambda[bi & 0xFFFF] : 1.0;
@@ -323,10 +392,11 @@ __device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const
           if (rd < rSoft) {
             const double q = rd / rSoft;
             rd = ((1.0 - 0.5 * q) * q * q * q + 0.5) * rSoft;
+            rid = rcp_d(rd);
           }
         }
       }
-      etile += 0.5 * sd * pair_energy_d<ELEC, VDW>(d, ia.qd * qjd, ljd.x, ljd.y, rd);
+      etile += sd * pair_energy_sum<ELEC, VDW>(ec, ia.qd * qjd, ljd.x, ljd.y, rd, rid);
     }
     (void)eq; (void)eA; (void)eB;
     float fr;
@@ -347,7 +417,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 // One chunk of the list: the tiles of row I it holds, against the 32
 // i-atoms in registers; the i-force partials go to the chunk's slot.
 template <int ELEC, int VDW, bool ENERGY, bool ALCH, bool SOFT>
-__device__ __forceinline__ void chunk_pairs(const Dev &d, const NbConst &c, const float2 *s_vdw, int ch, int lane,
+__device__ __forceinline__ void chunk_pairs(const Dev &d, const NbConst &c, const EnConst &ec, const float2 *s_vdw, int ch, int lane,
                                             int half, int li, uint4 *sp, int2 *spr, float *slo,
                                             unsigned char *sjx, double &eacc) {
   const int4 cr = d.chunk[ch];
@@ -422,18 +492,27 @@ __device__ __forceinline__ void chunk_pairs(const Dev &d, const NbConst &c, cons
     double etile = 0.0;
     const bool alchTile = ALCH && (hi.w | alchJc);
     const bool self = I == Jc, chk = self || ex >= 0;
-#define BM_TILE(AL, SO, CK)                                                                        \
-tile_pairs<ELEC, VDW, ENERGY, AL, SO, CK>(d, c, ia, li, half, sp, spr, slo, sjx, s_vdw, nj, emc, \
-                                          self, fx, fy, fz, etile)
-    if (alchTile) {
-      if (chk) BM_TILE(ALCH, SOFT, true);
-      else BM_TILE(ALCH, SOFT, false);
+#define BM_TILE(EN, AL, SO, CK)                                                                       \
+  tile_pairs<ELEC, VDW, EN, AL, SO, CK>(d, c, ec, ia, li, half, sp, spr, slo, sjx, s_vdw, nj, emc, self, \
+                                        fx, fy, fz, etile)
+#define BM_TILE_CHK(EN)                  \
+  if (alchTile) {                        \
+    if (chk) BM_TILE(EN, ALCH, SOFT, true); \
+    else BM_TILE(EN, ALCH, SOFT, false); \
+  } else {                               \
+    if (chk) BM_TILE(EN, false, false, true); \
+    else BM_TILE(EN, false, false, false); \
+  }
+    // energies from the tiles with J >= I only (a pair of blocks is in the
+    // list both ways), those of the diagonal tile in halves
+    if (ENERGY && Jc >= I) {
+      BM_TILE_CHK(ENERGY)
     } else {
-      if (chk) BM_TILE(false, false, true);
-      else BM_TILE(false, false, false);
+      BM_TILE_CHK(false)
     }
+#undef BM_TILE_CHK
 #undef BM_TILE
-    if (ENERGY) eacc += etile;
+    if (ENERGY) eacc += self ? 0.5 * etile : etile;
     wave_lds_sync();
     k = kn;
   }
@@ -467,6 +546,8 @@ __device__ __forceinline__ void nbdirect_kernel_body(const Dev &d, int bid, int 
   }
   const float2 *s_vdw = GTABLE ? d.vdw : s_vdw_dyn;
   const NbConst c = make_const(d);
+  EnConst ec;
+  if (ENERGY) ec = make_energy_const(d);
   const bool fits = *d.ntiles <= d.maxtiles && *d.nchunks <= d.maxchunks;
   const int nchunks = fits ? *d.nchunks : 0;
   double eacc = 0.0;
@@ -479,7 +560,7 @@ __device__ __forceinline__ void nbdirect_kernel_body(const Dev &d, int bid, int 
   // one chunk per wave; waves past this step's chunk count exit
   const int k = bid * 4 + w;
   if (k >= nchunks) return;
-  chunk_pairs<ELEC, VDW, ENERGY, ALCH, SOFT>(d, c, s_vdw, k, lane, half, li, sp, spr, slo, sjx, eacc);
+  chunk_pairs<ELEC, VDW, ENERGY, ALCH, SOFT>(d, c, ec, s_vdw, k, lane, half, li, sp, spr, slo, sjx, eacc);
   if (ENERGY) {
     long long v = (long long)__double2ll_rn(eacc * kFixScaleD);
     wave_atomic_fix(&d.energy[BM_ENBDIRECT], v);
@@ -496,22 +577,73 @@ __global__ void __launch_bounds__(256) nbdirect_kernel_multi(Multi m) {
   nbdirect_kernel_body<ELEC, VDW, ENERGY, ALCH, SOFT, GTABLE>(d, b.bid, b.nblk);
 }
 
+// FP64 energy of a pair at effective distance r, for dU/dlambda.  (The form
+// of pair_energy_sum would differ in the last bits; dU/dlambda drives theta,
+// and a trajectory or a restart is to go on as before, to the bit.)
+template <int ELEC, int VDW>
+__device__ double pair_energy_d(const Dev &d, double qq, double c12, double c6, double r) {
+  const double rc = d.rcd, rs = d.rsd, rinv = 1.0 / r;
+  double e;
+  if (ELEC == BM_PME) {
+    e = qq * erfc(d.betad * r) * rinv;
+  } else if (ELEC == BM_FSWITCH) {
+    const double roff2 = rc * rc, ron2 = rs * rs;
+    const double ginv = 1 / ((roff2 - ron2) * (roff2 - ron2) * (roff2 - ron2));
+    const double A = roff2 * roff2 * (roff2 - 3 * ron2) * ginv, B = 6 * roff2 * ron2 * ginv;
+    const double C = -(ron2 + roff2) * ginv, D = 2 * ginv / 5;
+    const double dvc = 8 * (ron2 * roff2 * (rc - rs) - (roff2 * roff2 * rc - ron2 * ron2 * rs) / 5) * ginv;
+    const double r3 = r * r * r, r5 = r3 * r * r;
+    e = (r <= rs) ? qq * (rinv + dvc)
+                  : qq * (A * (rinv - 1 / rc) + B * (rc - r) + C * (roff2 * rc - r3) + D * (roff2 * roff2 * rc - r5));
+  } else {
+    e = qq * (rinv - 2 / rc + r / (rc * rc));
+  }
+  const double rinv3 = rinv * rinv * rinv, rinv6 = rinv3 * rinv3;
+  if (VDW == BM_VFSWITCH) {
+    const double rc3 = rc * rc * rc, rs3 = rs * rs * rs;
+    if (r < rs) {
+      const double dv6 = 1 / (rc3 * rs3);
+      e += c12 * (rinv6 * rinv6 - dv6 * dv6) - c6 * (rinv6 - dv6);
+    } else {
+      const double k6 = rc3 / (rc3 - rs3), k12 = rc3 * rc3 / (rc3 * rc3 - rs3 * rs3);
+      const double a3 = rinv3 - 1 / rc3, a6 = rinv6 - 1 / (rc3 * rc3);
+      e += c12 * k12 * a6 * a6 - c6 * k6 * a3 * a3;
+    }
+  } else if (VDW == BM_VSWITCH) {
+    if (r < rs) {
+      e += c12 * rinv6 * rinv6 - c6 * rinv6;
+    } else {
+      const double c2of = rc * rc, c2on = rs * rs;
+      const double rul3 = (c2of - c2on) * (c2of - c2on) * (c2of - c2on);
+      const double rijl = c2on - r * r, riju = c2of - r * r;
+      e += riju * riju * (riju - 3 * rijl) / rul3 * (c12 * rinv6 - c6) * rinv6;
+    }
+  } else {
+    const double r6 = r * r * r * r * r * r, rc6 = rc * rc * rc * rc * rc * rc;
+    e += c12 * (rinv6 * rinv6 + 2 * r6 / (rc6 * rc6 * rc6) - 3 / (rc6 * rc6)) - c6 * (rinv6 + r6 / (rc6 * rc6) - 2 / rc6);
+  }
+  return e;
+}
+
 // dU/dlambda of the nonbonded pairs (the lambda derivative of
 // nbdirect/nbdirect.cu:244-275,400-415) in FP64, by alchemical atom: the
 // tile kernels leave it out, since FP32 pair energies summed over a site's
-// thousands of pairs drift past the 1e-3 kcal/mol dU/dlambda bar.  Wave w
-// takes atom alchat[w / kDudlWaves] and every kDudlWaves-th pair of tiles
-// of its block's row (a half-wave per tile, a lane per j slot); each pair
+// thousands of pairs drift past the 1e-3 kcal/mol dU/dlambda bar.  An atom's
+// row of tiles is dealt in pairs to kDudlParts sums, each rounded to fixed
+// point by itself; wave w takes every kDudlWaves-th sum of atom
+// alchat[w / kDudlWaves], a half-wave per tile, a lane per j slot.  Tiles
+// whose current box is beyond rcut of the atom are passed over (four in
+// five).  Each pair
 // within rcut that is not excluded gives d(s E)/ds (E in FP64 at the FP64
 // effective distance; the soft-core term s dE/dr dr/ds with dE/dr in FP32)
 // times the lambda of the other block, or half of it within one block
 // (the pair is met again from the other atom), to the atom's block.
-constexpr int kDudlWaves = 32;
+constexpr int kDudlParts = 32, kDudlWaves = 16;
 template <int ELEC, int VDW, bool SOFT>
 __device__ __forceinline__ void nb_dudl_body(const Dev &d, int bid) {
   const int lane = threadIdx.x & 63, half = lane >> 5, lj = lane & 31;
   const int wv = bid * 4 + (threadIdx.x >> 6);
-  const int ai = wv / kDudlWaves, sub = wv % kDudlWaves;
+  const int ai = wv / kDudlWaves;
   if (ai >= d.nalchat) return;
   if (*d.ntiles > d.maxtiles || *d.nchunks > d.maxchunks) return;
   const int a = d.alchat[ai], sa = d.g2s[a], I = sa / kBlockAtoms, li = sa % kBlockAtoms;
@@ -521,10 +653,13 @@ __device__ __forceinline__ void nb_dudl_body(const Dev &d, int bid) {
   const double qa = kElectricD * ((double)__uint_as_float(pa.w) + (double)d.slo[sa]);
   const double la = d.lambda[ba & 0xFFFF];
   const NbConst c = make_const(d);
-  double acc = 0.0;
   const int t1 = d.tstart[I + 1];
-  for (int t = d.tstart[I] + 2 * sub + half; t < t1; t += 2 * kDudlWaves) {
+  long long sum = 0;
+  for (int part = wv % kDudlWaves; part < kDudlParts; part += kDudlWaves) {
+   double acc = 0.0;
+   for (int t = d.tstart[I] + 2 * part + half; t < t1; t += 2 * kDudlParts) {
     const int J = d.tile_j[t], ex = d.tile_ex[t];
+    if (!atom_near_block(d, pa, J, d.rc2)) continue;
     const int sj = J * kBlockAtoms + lj;
     const int2 prj = d.spar[sj];
     if (prj.x < 0 || sj == sa) continue;
@@ -559,9 +694,11 @@ __device__ __forceinline__ void nb_dudl_body(const Dev &d, int bid) {
       fl += sd * (double)f * dredll;
     }
     acc += same ? 0.5 * fl : lo * fl;
+   }
+   for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+   sum += fix_d(acc);
   }
-  for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-  if (lane == 0 && acc != 0.0) atomic_fix(&d.dudl[ba & 0xFFFF], fix_d(acc));
+  if (lane == 0 && sum) atomic_fix(&d.dudl[ba & 0xFFFF], sum);
 }
 
 template <int ELEC, int VDW, bool SOFT>
