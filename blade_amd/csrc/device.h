@@ -65,7 +65,8 @@ struct Dev {
   int ncx, ncy, ncol, maxblocks;
   long long maxtiles;
   unsigned *ufrac;               // [3][N] fractional coordinates at rebuild
-  int *colcount, *colstart, *colfill, *bucket;   // [ncol],[ncol+1],[ncol],[N]
+  int *colcount, *colstart, *bucket;   // [ncol],[ncol+1],[N]
+  int *colrank;                  // [N] place of an atom in its column's bucket
   int *blkstart;                 // [ncol+1] first block of each column
   int *nblocks;                  // [1]
   int *l2g;                      // [32*maxB] slot -> atom (-1 empty)
@@ -78,8 +79,7 @@ struct Dev {
   int *tcount, *tstart;          // [maxB],[maxB+1] directed tiles per row
   int *ntiles;                   // [1]
   int *tile_i, *tile_j, *tile_ex;// [maxtiles]
-  int *tile_flag;                // [maxtiles]
-  int *ccount, *cstart;          // [maxB],[maxB+1] chunks per row
+  int *cstart;                   // [maxB+1] chunks before each row
   int *nchunks;                  // [1]
   int maxchunks;
   int4 *chunk;                   // [maxchunks] (I, first tile, tiles, 0)
@@ -87,12 +87,9 @@ struct Dev {
                                  // order); the force assembly converts them to fixed point
   int nalchat;                   // atoms of lambda blocks (site block != 0)
   int *alchat;                   // [nalchat] their indices
-  int *ecount, *estart;          // [maxB],[maxB+1] tiles with exclusions per row
-  int *nexcltiles;               // [1]
+  int *nexcltiles;               // [1] tiles with exclusions
   unsigned *emask;               // [32*2*n_excl]
-  int *excl_tile;                // [2*n_excl] tiles (I,J) and (J,I) of each pair
-  int nexcl;
-  int *excl;                     // [2*n_excl]
+  int *exstart, *exadj;          // [N+1],[2*n_excl] atoms excluded from each atom
   int *workctr;                  // [4] dynamic work counters
   int *errflag;                  // [1] overflow / capacity errors
   double rlist2;                 // (rcut+pad)^2, as the oracle computes it

@@ -4,10 +4,14 @@
 // fractional coordinates; orc_domdec in the oracle is the same rule set).
 //
 // Rebuild sequence (no host synchronisation, fixed grids, graph-capturable):
-//   dd_wrap_count -> dd_scan_columns -> dd_scatter -> dd_sort_columns ->
-//   dd_tile_count -> dd_scan_tiles -> dd_tile_write -> dd_excl_mark ->
-//   dd_excl_rows -> dd_scan_excl -> dd_excl_assign -> dd_excl_clear ->
-//   dd_excl_set
+//   dd_wrap_count -> dd_scatter -> dd_sort_columns -> dd_tile_count ->
+//   dd_tile_write
+// Five dependent launches: each one costs about 5 us beside its own work
+// (start-up, drain, a dependent load chain), which is most of a rebuild at
+// any size this list serves, so prefix sums over columns and rows are
+// formed by every workgroup that needs them (a few KB from L2) instead of
+// in kernels of their own, and the exclusion masks are made by the wave
+// that writes the row.
 // Every step: dd_pack (slot positions, block boxes, accumulator reset).
 //
 // The tile list is directed: row I holds every block J (J == I included)
@@ -26,52 +30,47 @@
 
 namespace blade {
 
-// One workgroup of 1024 threads: exclusive scan of in[0..n) into out,
-// out[n] = total.  Deterministic integer arithmetic.
-__device__ void block_scan_1024(const int *in, int *out, int n, int *total) {
-  __shared__ int part[1024];
-  const int tid = threadIdx.x;
-  const int per = (n + 1023) / 1024;
-  const int b = tid * per, e = min(n, b + per);
-  int s = 0;
-  for (int i = b; i < e; i++) s += in[i];
-  part[tid] = s;
+// Sum of v over the 256 threads of a workgroup, for all of them (every
+// thread must call it; s_sum: four ints of LDS, free again on return).
+__device__ __forceinline__ int wg_sum256(int v, int *s_sum) {
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = v;
   __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    int v = tid >= off ? part[tid - off] : 0;
-    __syncthreads();
-    part[tid] += v;
-    __syncthreads();
-  }
-  int run = part[tid] - s;
-  for (int i = b; i < e; i++) {
-    int v = in[i];
-    out[i] = run;
-    run += v;
-  }
-  if (tid == 1023) {
-    out[n] = part[1023];
-    if (total) *total = part[1023];
-  }
+  const int t = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
+  __syncthreads();
+  return t;
 }
 
-__device__ __forceinline__ void dd_zero_columns_body(const Dev &d, int bid, int nblk) {
-  if (halted_wg(d)) return;   // a halted step leaves the list as it is
-  int c = bid * blockDim.x + threadIdx.x;
-  if (c < d.ncol) {
-    d.colcount[c] = 0;
-    d.colfill[c] = 0;
+// Exclusive prefix sum of f(0..n) into out[0..n], out[n] the total, by the
+// 256 threads of a workgroup; out may be in LDS or global memory.
+template <class F>
+__device__ __forceinline__ void wg_scan256(int n, F f, int *out, int *s_sum) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int run = 0;
+  for (int i0 = 0; i0 < n; i0 += 256) {
+    const int i = i0 + threadIdx.x;
+    const int v = i < n ? f(i) : 0;
+    int x = v;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    if (lane == 63) s_sum[w] = x;
+    __syncthreads();
+    int pre = run;
+    for (int k = 0; k < 4; k++) {
+      if (k < w) pre += s_sum[k];
+      run += s_sum[k];
+    }
+    if (i < n) out[i] = pre + x - v;
+    __syncthreads();
   }
-}
-__global__ void __launch_bounds__(256) dd_zero_columns(Dev d) { dd_zero_columns_body(d, blockIdx.x, gridDim.x); }
-__global__ void __launch_bounds__(256) dd_zero_columns_multi(Multi m) {
-  const MultiBlk b = multi_block(m);
-  const Dev d = m.devs[b.sys];
-  dd_zero_columns_body(d, b.bid, b.nblk);
+  if (threadIdx.x == 0) out[n] = run;
 }
 
-// wrap every atom into the box, fractional coordinates, column counts
-// (one thread per slot of the previous rebuild; every atom has one slot)
+// wrap every atom into the box, fractional coordinates, column counts and
+// each atom's place in its column's bucket (one thread per slot of the
+// previous rebuild; every atom has one slot; the pack clears the counts)
 __device__ __forceinline__ void dd_wrap_count_body(const Dev &d, int bid, int nblk) {
   if (halted_wg(d)) return;   // a halted step leaves the list as it is
   const int s = bid * blockDim.x + threadIdx.x;
@@ -92,7 +91,8 @@ __device__ __forceinline__ void dd_wrap_count_body(const Dev &d, int bid, int nb
     unsigned cy = (unsigned)(((unsigned long long)u[1] * (unsigned)d.ncy) >> 32);
     col = cx * d.ncy + cy;
   }
-  wave_claim(d.colcount, col, i >= 0);
+  const int f = wave_claim(d.colcount, col, i >= 0);
+  if (i >= 0) d.colrank[i] = f;
 }
 __global__ void __launch_bounds__(256) dd_wrap_count(Dev d) { dd_wrap_count_body(d, blockIdx.x, gridDim.x); }
 __global__ void __launch_bounds__(256) dd_wrap_count_multi(Multi m) {
@@ -101,48 +101,37 @@ __global__ void __launch_bounds__(256) dd_wrap_count_multi(Multi m) {
   dd_wrap_count_body(d, b.bid, b.nblk);
 }
 
-// blocks per column = ceil(count/32); block starts by exclusive scan
-__device__ __forceinline__ void dd_scan_columns_body(const Dev &d, int bid, int nblk) {
+// Atoms into column buckets (bucket order is arbitrary; the column sort
+// fixes the final order).  Every workgroup scans the column counts into LDS
+// (ncol+1 ints); the first also stores the column starts and, with
+// ceil(count/32) blocks to a column, the block starts.
+__device__ __forceinline__ void dd_scatter_body(const Dev &d, int bid) {
   if (halted_wg(d)) return;   // a halted step leaves the list as it is
-  __shared__ int nb[4096];
-  int *tmp = d.bucket;  // not yet used this rebuild: scratch for ncol > 4096
-  const bool big = d.ncol > 4096;
-  for (int c = threadIdx.x; c < d.ncol; c += 1024) {
-    int v = (d.colcount[c] + kBlockAtoms - 1) / kBlockAtoms;
-    if (big) tmp[c] = v; else nb[c] = v;
-  }
+  extern __shared__ int s_start[];
+  __shared__ int s_sum[4];
+  wg_scan256(d.ncol, [&](int c) { return d.colcount[c]; }, s_start, s_sum);
   __syncthreads();
-  block_scan_1024(d.colcount, d.colstart, d.ncol, nullptr);
-  __syncthreads();
-  block_scan_1024(big ? tmp : nb, d.blkstart, d.ncol, d.nblocks);
-}
-__global__ void __launch_bounds__(1024) dd_scan_columns(Dev d) { dd_scan_columns_body(d, blockIdx.x, gridDim.x); }
-__global__ void __launch_bounds__(1024) dd_scan_columns_multi(Multi m) {
-  const MultiBlk b = multi_block(m);
-  const Dev d = m.devs[b.sys];
-  dd_scan_columns_body(d, b.bid, b.nblk);
-}
-
-// atoms into column buckets (bucket order is arbitrary; the column sort
-// fixes the final order)
-__device__ __forceinline__ void dd_scatter_body(const Dev &d, int bid, int nblk) {
-  if (halted_wg(d)) return;   // a halted step leaves the list as it is
   const int s = bid * blockDim.x + threadIdx.x;
   const int i = s < 32 * d.maxblocks ? d.l2g[s] : -1;
-  int c = 0;
   if (i >= 0) {
-    unsigned cx = (unsigned)(((unsigned long long)d.ufrac[i] * (unsigned)d.ncx) >> 32);
-    unsigned cy = (unsigned)(((unsigned long long)d.ufrac[d.n + i] * (unsigned)d.ncy) >> 32);
-    c = cx * d.ncy + cy;
+    const unsigned cx = (unsigned)(((unsigned long long)d.ufrac[i] * (unsigned)d.ncx) >> 32);
+    const unsigned cy = (unsigned)(((unsigned long long)d.ufrac[d.n + i] * (unsigned)d.ncy) >> 32);
+    d.bucket[s_start[cx * d.ncy + cy] + d.colrank[i]] = i;
   }
-  const int f = wave_claim(d.colfill, c, i >= 0);
-  if (i >= 0) d.bucket[d.colstart[c] + f] = i;
+  if (bid == 0) {
+    for (int c = threadIdx.x; c <= d.ncol; c += blockDim.x) d.colstart[c] = s_start[c];
+    wg_scan256(d.ncol, [&](int c) { return (d.colcount[c] + kBlockAtoms - 1) / kBlockAtoms; }, d.blkstart, s_sum);
+    if (threadIdx.x == 0) {
+      *d.nblocks = d.blkstart[d.ncol];   // this thread's own store
+      *d.nexcltiles = 0;
+    }
+  }
 }
-__global__ void __launch_bounds__(256) dd_scatter(Dev d) { dd_scatter_body(d, blockIdx.x, gridDim.x); }
+__global__ void __launch_bounds__(256) dd_scatter(Dev d) { dd_scatter_body(d, blockIdx.x); }
 __global__ void __launch_bounds__(256) dd_scatter_multi(Multi m) {
   const MultiBlk b = multi_block(m);
   const Dev d = m.devs[b.sys];
-  dd_scatter_body(d, b.bid, b.nblk);
+  dd_scatter_body(d, b.bid);
 }
 
 // One workgroup per column: rank atoms by (z fraction, atom index), place
@@ -216,21 +205,35 @@ __global__ void __launch_bounds__(256) dd_sort_columns_multi(Multi m) {
 
 // Periodic gap between two rebuild boxes (fractional counts), squared, in
 // A^2, against (rcut+pad)^2; rounding as in the oracle (no contraction).
+// The gap to either side is a difference modulo 2^32.  Pairs clearly inside
+// or outside in FP32 (whose error is below 1e-6 relative) are settled
+// there; the rest in the oracle's FP64 arithmetic.
 __device__ __forceinline__ bool dd_close(const Dev &d, const unsigned (&aLo)[3], const unsigned (&aHi)[3],
                                          const unsigned (&bLo)[3], const unsigned (&bHi)[3]) {
-  const unsigned long long P = 1ull << 32;
-  double g[3];
+  unsigned gap[3];
+  float sf = 0.f;
 #pragma unroll
   for (int k = 0; k < 3; k++) {
-    unsigned long long aL = aLo[k], aH = aHi[k], bL = bLo[k], bH = bHi[k];
-    unsigned long long gap = 0;
-    if (aH < bL) gap = min(bL - aH, aL + P - bH);
-    else if (bH < aL) gap = min(aL - bH, bL + P - aH);
-    g[k] = __dmul_rn((double)gap, d.ddscale[k]);
+    const bool apart = aHi[k] < bLo[k] || bHi[k] < aLo[k];
+    gap[k] = apart ? min(bLo[k] - aHi[k], aLo[k] - bHi[k]) : 0u;
+    const float g = (float)gap[k] * d.fracscale[k];
+    sf += g * g;
   }
+  const float r2 = (float)d.rlist2;
+  if (sf < r2 * 0.99999f) return true;
+  if (sf > r2 * 1.00001f) return false;
+  double g[3];
+#pragma unroll
+  for (int k = 0; k < 3; k++) g[k] = __dmul_rn((double)gap[k], d.ddscale[k]);
   double s = __dadd_rn(__dmul_rn(g[0], g[0]), __dmul_rn(g[1], g[1]));
   s = __dadd_rn(s, __dmul_rn(g[2], g[2]));
   return s <= d.rlist2;
+}
+
+__device__ __forceinline__ void dd_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 constexpr int kBoxLds = 2048;   // block boxes staged in LDS by the tile kernels
@@ -279,10 +282,7 @@ __device__ __forceinline__ void dd_tile_count_body(const Dev &d, int bid, int nb
     const bool keep = J < nb && dd_tile_keep(d, s_lo, s_hi, I, aLo, aHi, J);
     cnt += __popcll(__ballot(keep));
   }
-  if (lane == 0) {
-    d.tcount[I] = cnt;
-    d.ccount[I] = (cnt + d.tchunk - 1) / d.tchunk;
-  }
+  if (lane == 0) d.tcount[I] = cnt;
 }
 __global__ void __launch_bounds__(256) dd_tile_count(Dev d) { dd_tile_count_body(d, blockIdx.x, gridDim.x); }
 __global__ void __launch_bounds__(256) dd_tile_count_multi(Multi m) {
@@ -291,182 +291,137 @@ __global__ void __launch_bounds__(256) dd_tile_count_multi(Multi m) {
   dd_tile_count_body(d, b.bid, b.nblk);
 }
 
-// row starts of tiles and chunks; flags a list that outgrows its buffers
-__device__ __forceinline__ void dd_scan_tiles_body(const Dev &d, int bid, int nblk) {
-  if (halted_wg(d)) return;   // a halted step leaves the list as it is
-  const int nb = *d.nblocks;
-  block_scan_1024(d.tcount, d.tstart, nb, d.ntiles);
-  __syncthreads();
-  block_scan_1024(d.ccount, d.cstart, nb, d.nchunks);
-  __syncthreads();
-  if (threadIdx.x == 0 && (*d.ntiles > d.maxtiles || *d.nchunks > d.maxchunks)) atomicOr(d.errflag, 4);
-}
-__global__ void __launch_bounds__(1024) dd_scan_tiles(Dev d) { dd_scan_tiles_body(d, blockIdx.x, gridDim.x); }
-__global__ void __launch_bounds__(1024) dd_scan_tiles_multi(Multi m) {
-  const MultiBlk b = multi_block(m);
-  const Dev d = m.devs[b.sys];
-  dd_scan_tiles_body(d, b.bid, b.nblk);
-}
+// LDS of one row in dd_tile_write: the bitmap of its blocks J (64-bit
+// words), the tiles before each word, and a bit per tile for exclusions
+__host__ __device__ inline int dd_row_words(int maxblocks) { return (maxblocks + 63) / 64; }
+static size_t lds_tile_write(const Dev &d) { return (size_t)4 * dd_row_words(d.maxblocks) * (8 + 8 + 4); }
 
-__device__ __forceinline__ void dd_tile_write_body(const Dev &d, int bid, int nblk) {
+// One wave per row I (four to a workgroup): row starts of
+// tiles and chunks (sums of the counts of the rows before; flags a list that
+// outgrows its buffers), the row's tiles in ascending J and its chunks, then
+// the exclusions of the row's atoms: tiles holding one get 32 mask words
+// (bit j of word i: slots (I,i) and (J,j) are excluded), numbered by a claim
+// on the number of such tiles, -1 in tile_ex for the others.  Lane l makes
+// word l of every mask of its row, so no other thread writes it.
+__device__ __forceinline__ void dd_tile_write_body(const Dev &d, int bid) {
   if (halted_wg(d)) return;   // a halted step leaves the list as it is
   __shared__ unsigned s_lo[3 * kBoxLds], s_hi[3 * kBoxLds];
-  const int nb = *d.nblocks;
-  if (*d.ntiles > d.maxtiles || *d.nchunks > d.maxchunks) return;
+  __shared__ int s_sum[4];
+  extern __shared__ unsigned long long s_row[];
+  const int nb = *d.nblocks, rows = 4;
+  const int tc = d.tchunk, I0 = bid * rows;
+  if (I0 >= nb) return;
+  // (32-bit sums: a list of 2^31 tiles is beyond any capacity of its arrays)
+  int before = 0, cbefore = 0, all = 0, call = 0;
+  for (int k = threadIdx.x; k < nb; k += blockDim.x) {
+    const int t = d.tcount[k], c = (t + tc - 1) / tc;
+    all += t;
+    call += c;
+    if (k < I0) {
+      before += t;
+      cbefore += c;
+    }
+  }
+  all = wg_sum256(all, s_sum);
+  call = wg_sum256(call, s_sum);
+  if (bid == 0 && threadIdx.x == 0) {
+    *d.ntiles = all;
+    *d.nchunks = call;
+    if (all > d.maxtiles || call > d.maxchunks) atomicOr(d.errflag, 4);
+  }
+  if (all > d.maxtiles || call > d.maxchunks) return;
+  before = wg_sum256(before, s_sum);
+  cbefore = wg_sum256(cbefore, s_sum);
   dd_stage_boxes(d, nb, s_lo, s_hi);
-  const int I = (bid * blockDim.x + threadIdx.x) >> 6;
+  const int w = threadIdx.x >> 6, I = I0 + w;
   const int lane = threadIdx.x & 63;
   if (I >= nb) return;
+  for (int k = I0; k < I; k++) {
+    const int t = d.tcount[k];
+    before += t;
+    cbefore += (t + tc - 1) / tc;
+  }
+  const int cnt = d.tcount[I], nchunk = (cnt + tc - 1) / tc;
+  if (lane == 0) {
+    d.tstart[I] = before;
+    d.cstart[I] = cbefore;
+    if (I == nb - 1) {
+      d.tstart[nb] = before + cnt;
+      d.cstart[nb] = cbefore + nchunk;
+    }
+  }
   unsigned aLo[3], aHi[3];
 #pragma unroll
   for (int k = 0; k < 3; k++) {
     aLo[k] = d.bblo[3 * I + k];
     aHi[k] = d.bbhi[3 * I + k];
   }
-  int base = d.tstart[I];
+  const int nw = dd_row_words(d.maxblocks);
+  unsigned long long *bits = s_row + w * nw;                                     // kept blocks
+  unsigned long long *ebits = s_row + (rows + w) * nw;                           // tiles with exclusions
+  int *pre = reinterpret_cast<int *>(s_row + 2 * rows * nw) + w * nw;            // tiles before a word
   const unsigned long long below = (1ull << lane) - 1;
+  int run = 0;
   for (int J0 = 0; J0 < nb; J0 += 64) {
     const int J = J0 + lane;
     const bool keep = J < nb && dd_tile_keep(d, s_lo, s_hi, I, aLo, aHi, J);
     const unsigned long long m = __ballot(keep);
     if (keep) {
-      int t = base + __popcll(m & below);
+      const int t = before + run + __popcll(m & below);
       d.tile_i[t] = I;
       d.tile_j[t] = J;
-      d.tile_flag[t] = 0;
     }
-    base += __popcll(m);
+    if (lane == 0) {
+      bits[J0 >> 6] = m;
+      pre[J0 >> 6] = run;
+      ebits[J0 >> 6] = 0;
+    }
+    run += __popcll(m);
   }
-  const int t0 = d.tstart[I], cnt = d.tcount[I], c0 = d.cstart[I];
-  const int tc = d.tchunk;
-  for (int k = lane; k * tc < cnt; k += 64) d.chunk[c0 + k] = make_int4(I, t0 + k * tc, min(tc, cnt - k * tc), 0);
+  for (int k = lane; k < nchunk; k += 64)
+    d.chunk[cbefore + k] = make_int4(I, before + k * tc, min(tc, cnt - k * tc), 0);
+  dd_wave_sync();
+  // place in the row of the tile to block J, -1 if the row has none
+  auto place = [&](int J) {
+    const unsigned long long m = bits[J >> 6], bit = 1ull << (J & 63);
+    return m & bit ? pre[J >> 6] + __popcll(m & (bit - 1)) : -1;
+  };
+  const int a = lane < kBlockAtoms ? d.l2g[I * kBlockAtoms + lane] : -1;
+  const int x0 = a >= 0 ? d.exstart[a] : 0, x1 = a >= 0 ? d.exstart[a + 1] : 0;
+  for (int x = x0; x < x1; x++) {
+    const int q = place(d.g2s[d.exadj[x]] / kBlockAtoms);
+    if (q >= 0) atomicOr(&ebits[q >> 6], 1ull << (q & 63));
+  }
+  dd_wave_sync();
+  const int tw = (cnt + 63) / 64;   // words of ebits in use
+  int flagged = 0;
+  for (int k = 0; k < tw; k++) flagged += __popcll(ebits[k]);
+  int base = 0;
+  if (lane == 0 && flagged) base = atomicAdd(d.nexcltiles, flagged);
+  base = __shfl(base, 0, 64);
+  int e0 = base;
+  for (int k = 0; k < tw; k++) {
+    const unsigned long long m = ebits[k];
+    const int t = k * 64 + lane;
+    if (t < cnt) d.tile_ex[before + t] = (m >> lane) & 1ull ? e0 + __popcll(m & below) : -1;
+    e0 += __popcll(m);
+  }
+  if (lane < kBlockAtoms)
+    for (int k = 0; k < flagged; k++) d.emask[(long long)(base + k) * kBlockAtoms + lane] = 0u;
+  for (int x = x0; x < x1; x++) {
+    const int sb = d.g2s[d.exadj[x]];
+    const int q = place(sb / kBlockAtoms);
+    if (q < 0) continue;
+    int e = base + __popcll(ebits[q >> 6] & ((1ull << (q & 63)) - 1));
+    for (int k = 0; k < q >> 6; k++) e += __popcll(ebits[k]);
+    atomicOr(&d.emask[(long long)e * kBlockAtoms + lane], 1u << (sb % kBlockAtoms));
+  }
 }
-__global__ void __launch_bounds__(256) dd_tile_write(Dev d) { dd_tile_write_body(d, blockIdx.x, gridDim.x); }
+__global__ void __launch_bounds__(256) dd_tile_write(Dev d) { dd_tile_write_body(d, blockIdx.x); }
 __global__ void __launch_bounds__(256) dd_tile_write_multi(Multi m) {
   const MultiBlk b = multi_block(m);
   const Dev d = m.devs[b.sys];
-  dd_tile_write_body(d, b.bid, b.nblk);
-}
-
-// tile (I,J) by binary search in row I's ascending J list, -1 if absent
-__device__ __forceinline__ int dd_find_tile(const Dev &d, int I, int J) {
-  int lo = d.tstart[I], hi = d.tstart[I + 1];
-  const int end = hi;
-  while (lo < hi) {
-    int mid = (lo + hi) >> 1;
-    if (d.tile_j[mid] < J) lo = mid + 1; else hi = mid;
-  }
-  return (lo < end && d.tile_j[lo] == J) ? lo : -1;
-}
-
-// exclusion pair -> the tiles (I,J) and (J,I) holding it
-__device__ __forceinline__ void dd_excl_mark_body(const Dev &d, int bid, int nblk) {
-  if (halted_wg(d)) return;   // a halted step leaves the list as it is
-  const int e = bid * blockDim.x + threadIdx.x;
-  if (e >= d.nexcl) return;
-  if (*d.ntiles > d.maxtiles) return;
-  const int sa = d.g2s[d.excl[2 * e]], sb = d.g2s[d.excl[2 * e + 1]];
-  const int I = sa / kBlockAtoms, J = sb / kBlockAtoms;
-  const int ta = dd_find_tile(d, I, J);
-  const int tb = ta < 0 ? -1 : (I == J ? ta : dd_find_tile(d, J, I));
-  d.excl_tile[2 * e] = ta;
-  d.excl_tile[2 * e + 1] = tb;
-  if (ta >= 0) d.tile_flag[ta] = 1;
-  if (tb >= 0) d.tile_flag[tb] = 1;
-}
-__global__ void __launch_bounds__(256) dd_excl_mark(Dev d) { dd_excl_mark_body(d, blockIdx.x, gridDim.x); }
-__global__ void __launch_bounds__(256) dd_excl_mark_multi(Multi m) {
-  const MultiBlk b = multi_block(m);
-  const Dev d = m.devs[b.sys];
-  dd_excl_mark_body(d, b.bid, b.nblk);
-}
-
-// one wave per row: tiles of the row holding exclusions
-__device__ __forceinline__ void dd_excl_rows_body(const Dev &d, int bid, int nblk) {
-  if (halted_wg(d)) return;   // a halted step leaves the list as it is
-  const int I = (bid * blockDim.x + threadIdx.x) >> 6;
-  const int lane = threadIdx.x & 63;
-  if (I >= *d.nblocks) return;
-  int cnt = 0;
-  if (*d.ntiles <= d.maxtiles)
-    for (int t = d.tstart[I] + lane; t - lane < d.tstart[I + 1]; t += 64)
-      cnt += __popcll(__ballot(t < d.tstart[I + 1] && d.tile_flag[t]));
-  if (lane == 0) d.ecount[I] = cnt;
-}
-__global__ void __launch_bounds__(256) dd_excl_rows(Dev d) { dd_excl_rows_body(d, blockIdx.x, gridDim.x); }
-__global__ void __launch_bounds__(256) dd_excl_rows_multi(Multi m) {
-  const MultiBlk b = multi_block(m);
-  const Dev d = m.devs[b.sys];
-  dd_excl_rows_body(d, b.bid, b.nblk);
-}
-
-__device__ __forceinline__ void dd_scan_excl_body(const Dev &d, int bid, int nblk) {
-  if (halted_wg(d)) return;   // a halted step leaves the list as it is
-  block_scan_1024(d.ecount, d.estart, *d.nblocks, d.nexcltiles);
-}
-__global__ void __launch_bounds__(1024) dd_scan_excl(Dev d) { dd_scan_excl_body(d, blockIdx.x, gridDim.x); }
-__global__ void __launch_bounds__(1024) dd_scan_excl_multi(Multi m) {
-  const MultiBlk b = multi_block(m);
-  const Dev d = m.devs[b.sys];
-  dd_scan_excl_body(d, b.bid, b.nblk);
-}
-
-// one wave per row: compact mask index of every flagged tile, -1 otherwise
-__device__ __forceinline__ void dd_excl_assign_body(const Dev &d, int bid, int nblk) {
-  if (halted_wg(d)) return;   // a halted step leaves the list as it is
-  const int I = (bid * blockDim.x + threadIdx.x) >> 6;
-  const int lane = threadIdx.x & 63;
-  if (I >= *d.nblocks || *d.ntiles > d.maxtiles) return;
-  int base = d.estart[I];
-  const unsigned long long below = (1ull << lane) - 1;
-  const int t1 = d.tstart[I + 1];
-  for (int t0 = d.tstart[I]; t0 < t1; t0 += 64) {
-    const int t = t0 + lane;
-    const bool f = t < t1 && d.tile_flag[t];
-    const unsigned long long m = __ballot(f);
-    if (t < t1) d.tile_ex[t] = f ? base + __popcll(m & below) : -1;
-    base += __popcll(m);
-  }
-}
-__global__ void __launch_bounds__(256) dd_excl_assign(Dev d) { dd_excl_assign_body(d, blockIdx.x, gridDim.x); }
-__global__ void __launch_bounds__(256) dd_excl_assign_multi(Multi m) {
-  const MultiBlk b = multi_block(m);
-  const Dev d = m.devs[b.sys];
-  dd_excl_assign_body(d, b.bid, b.nblk);
-}
-
-__device__ __forceinline__ void dd_excl_clear_body(const Dev &d, int bid, int nblk) {
-  if (halted_wg(d)) return;   // a halted step leaves the list as it is
-  const long long n = (long long)(*d.nexcltiles) * kBlockAtoms;
-  for (long long i = bid * (long long)blockDim.x + threadIdx.x; i < n;
-       i += (long long)nblk * blockDim.x)
-    d.emask[i] = 0u;
-}
-__global__ void __launch_bounds__(256) dd_excl_clear(Dev d) { dd_excl_clear_body(d, blockIdx.x, gridDim.x); }
-__global__ void __launch_bounds__(256) dd_excl_clear_multi(Multi m) {
-  const MultiBlk b = multi_block(m);
-  const Dev d = m.devs[b.sys];
-  dd_excl_clear_body(d, b.bid, b.nblk);
-}
-
-// bit j of word i of tile (I,J): slots (I,i) and (J,j) are excluded
-__device__ __forceinline__ void dd_excl_set_body(const Dev &d, int bid, int nblk) {
-  if (halted_wg(d)) return;   // a halted step leaves the list as it is
-  const int e = bid * blockDim.x + threadIdx.x;
-  if (e >= d.nexcl) return;
-  if (*d.ntiles > d.maxtiles) return;
-  const int ta = d.excl_tile[2 * e], tb = d.excl_tile[2 * e + 1];
-  if (ta < 0) return;
-  const int sa = d.g2s[d.excl[2 * e]], sb = d.g2s[d.excl[2 * e + 1]];
-  const int la = sa % kBlockAtoms, lb = sb % kBlockAtoms;
-  atomicOr(&d.emask[d.tile_ex[ta] * kBlockAtoms + la], 1u << lb);
-  if (tb >= 0) atomicOr(&d.emask[d.tile_ex[tb] * kBlockAtoms + lb], 1u << la);
-}
-__global__ void __launch_bounds__(256) dd_excl_set(Dev d) { dd_excl_set_body(d, blockIdx.x, gridDim.x); }
-__global__ void __launch_bounds__(256) dd_excl_set_multi(Multi m) {
-  const MultiBlk b = multi_block(m);
-  const Dev d = m.devs[b.sys];
-  dd_excl_set_body(d, b.bid, b.nblk);
+  dd_tile_write_body(d, b.bid);
 }
 
 // Every step: slot coordinates, per-block box centre/half-extent for the
@@ -481,6 +436,7 @@ __device__ __forceinline__ void dd_pack_body(const Dev &d, int bid) {
     d.dtheta[s] = 0;
   }
   if (s < BM_NTERMS) d.energy[s] = 0;
+  if (s < d.ncol) d.colcount[s] = 0;   // for the next rebuild
   if (s == 0) {
     d.workctr[0] = 0;
     d.workctr[1] = 0;
@@ -537,69 +493,39 @@ __global__ void __launch_bounds__(256) dd_pack_multi(Multi m) {
 // launchers
 // ---------------------------------------------------------------------
 void launch_domdec_rebuild(const Dev &d, int maxBlocks, hipStream_t st) {
-  const int n = d.n;
-  const unsigned slots = (unsigned)((32LL * maxBlocks + 255) / 256);
-  const unsigned rows = (unsigned)((maxBlocks + 3) / 4);   // a wave per block
-  (void)n;
-  dd_zero_columns<<<(d.ncol + 255) / 256, 256, 0, st>>>(d);
-  dd_wrap_count<<<slots, 256, 0, st>>>(d);
-  dd_scan_columns<<<1, 1024, 0, st>>>(d);
-  dd_scatter<<<slots, 256, 0, st>>>(d);
-  dd_sort_columns<<<d.ncol, 256, 0, st>>>(d);
-  dd_tile_count<<<rows, 256, 0, st>>>(d);
-  dd_scan_tiles<<<1, 1024, 0, st>>>(d);
-  dd_tile_write<<<rows, 256, 0, st>>>(d);
-  if (d.nexcl) dd_excl_mark<<<(d.nexcl + 255) / 256, 256, 0, st>>>(d);
-  dd_excl_rows<<<rows, 256, 0, st>>>(d);
-  dd_scan_excl<<<1, 1024, 0, st>>>(d);
-  dd_excl_assign<<<rows, 256, 0, st>>>(d);
-  if (d.nexcl) {
-    dd_excl_clear<<<256, 256, 0, st>>>(d);
-    dd_excl_set<<<(d.nexcl + 255) / 256, 256, 0, st>>>(d);
-  }
+  (void)maxBlocks;
+  dd_wrap_count<<<grid_rebuild(d, 0), 256, 0, st>>>(d);
+  dd_scatter<<<grid_rebuild(d, 1), 256, lds_rebuild(d, 1), st>>>(d);
+  dd_sort_columns<<<grid_rebuild(d, 2), 256, 0, st>>>(d);
+  dd_tile_count<<<grid_rebuild(d, 3), 256, 0, st>>>(d);
+  dd_tile_write<<<grid_rebuild(d, 4), 256, lds_rebuild(d, 4), st>>>(d);
 }
 
 // The rebuild's kernels in order, for one launch each over several
-// systems: workgroups of kernel k for system d (0 leaves d out of that
-// launch), and the launches over the per-kernel plans m[kRebuildKernels].
+// systems: workgroups and dynamic LDS of kernel k for system d, and the
+// launches over the per-kernel plans m[kRebuildKernels] (lds: the largest
+// of their systems).
 int grid_rebuild(const Dev &d, int k) {
   const int slots = (int)((32LL * d.maxblocks + 255) / 256), rows = (d.maxblocks + 3) / 4;
   switch (k) {
-    case 0: return (d.ncol + 255) / 256;                // dd_zero_columns
-    case 1: return slots;                               // dd_wrap_count
-    case 2: return 1;                                   // dd_scan_columns
-    case 3: return slots;                               // dd_scatter
-    case 4: return d.ncol;                              // dd_sort_columns
-    case 5: return rows;                                // dd_tile_count
-    case 6: return 1;                                   // dd_scan_tiles
-    case 7: return rows;                                // dd_tile_write
-    case 8: return d.nexcl ? (d.nexcl + 255) / 256 : 0; // dd_excl_mark
-    case 9: return rows;                                // dd_excl_rows
-    case 10: return 1;                                  // dd_scan_excl
-    case 11: return rows;                               // dd_excl_assign
-    case 12: return d.nexcl ? 256 : 0;                  // dd_excl_clear
-    default: return d.nexcl ? (d.nexcl + 255) / 256 : 0;  // dd_excl_set
+    case 0: return slots;   // dd_wrap_count
+    case 1: return slots;   // dd_scatter
+    case 2: return d.ncol;  // dd_sort_columns
+    default: return rows;   // dd_tile_count, dd_tile_write: a wave per block
   }
 }
 
-void launch_domdec_rebuild_multi(const Multi *m, hipStream_t st) {
-#define BM_RB(K, KER, TH) \
-  if (m[K].nwg) KER##_multi<<<m[K].nwg, TH, 0, st>>>(m[K]);
-  BM_RB(0, dd_zero_columns, 256)
-  BM_RB(1, dd_wrap_count, 256)
-  BM_RB(2, dd_scan_columns, 1024)
-  BM_RB(3, dd_scatter, 256)
-  BM_RB(4, dd_sort_columns, 256)
-  BM_RB(5, dd_tile_count, 256)
-  BM_RB(6, dd_scan_tiles, 1024)
-  BM_RB(7, dd_tile_write, 256)
-  BM_RB(8, dd_excl_mark, 256)
-  BM_RB(9, dd_excl_rows, 256)
-  BM_RB(10, dd_scan_excl, 1024)
-  BM_RB(11, dd_excl_assign, 256)
-  BM_RB(12, dd_excl_clear, 256)
-  BM_RB(13, dd_excl_set, 256)
-#undef BM_RB
+size_t lds_rebuild(const Dev &d, int k) {
+  if (k == 1) return ((size_t)d.ncol + 1) * sizeof(int);
+  return k == 4 ? lds_tile_write(d) : 0;
+}
+
+void launch_domdec_rebuild_multi(const Multi *m, const size_t *lds, hipStream_t st) {
+  dd_wrap_count_multi<<<m[0].nwg, 256, 0, st>>>(m[0]);
+  dd_scatter_multi<<<m[1].nwg, 256, lds[1], st>>>(m[1]);
+  dd_sort_columns_multi<<<m[2].nwg, 256, 0, st>>>(m[2]);
+  dd_tile_count_multi<<<m[3].nwg, 256, 0, st>>>(m[3]);
+  dd_tile_write_multi<<<m[4].nwg, 256, lds[4], st>>>(m[4]);
 }
 
 int grid_pack(const Dev &d) {

@@ -403,8 +403,8 @@ int bm_system_create(int device, const bm_topology *t, const bm_runparams *rp, c
   ALLOC(d.ufrac, 3 * (size_t)n);
   ALLOC(d.colcount, d.ncol);
   ALLOC(d.colstart, d.ncol + 1);
-  ALLOC(d.colfill, d.ncol);
-  ALLOC(d.bucket, std::max(n, d.ncol));
+  ALLOC(d.bucket, n);
+  ALLOC(d.colrank, n);
   ALLOC(d.blkstart, d.ncol + 1);
   ALLOC(d.nblocks, 1);
   {
@@ -425,25 +425,28 @@ int bm_system_create(int device, const bm_topology *t, const bm_runparams *rp, c
   ALLOC(d.tcount, MB);
   ALLOC(d.tstart, MB + 1);
   ALLOC(d.ntiles, 1);
-  // +1: the exclusive scans also write the total at index n
   ALLOC(d.tile_i, s->maxTiles + 1);
   ALLOC(d.tile_j, s->maxTiles + 1);
   ALLOC(d.tile_ex, s->maxTiles + 1);
-  ALLOC(d.tile_flag, s->maxTiles + 1);
-  ALLOC(d.ccount, MB);
   ALLOC(d.cstart, MB + 1);
   ALLOC(d.nchunks, 1);
   ALLOC(d.chunk, d.maxchunks);
   ALLOC(d.ichunk, (size_t)d.maxchunks * 3 * kBlockAtoms);
-  ALLOC(d.ecount, MB);
-  ALLOC(d.estart, MB + 1);
   ALLOC(d.nexcltiles, 1);
-  d.nexcl = t->n_excl;
   ALLOC(d.emask, 2 * (size_t)std::max(1, t->n_excl) * kBlockAtoms);
-  ALLOC(d.excl_tile, 2 * (size_t)t->n_excl);
   {
-    std::vector<int> ex(t->excl_idx, t->excl_idx + 2 * (size_t)t->n_excl);
-    UPLOAD(d.excl, ex);
+    // both directions of every excluded pair, by atom
+    std::vector<int> start(n + 1, 0), adj(2 * (size_t)t->n_excl);
+    for (size_t k = 0; k < adj.size(); k++) start[t->excl_idx[k] + 1]++;
+    for (int i = 0; i < n; i++) start[i + 1] += start[i];
+    std::vector<int> fill(start.begin(), start.end() - 1);
+    for (int e = 0; e < t->n_excl; e++) {
+      const int a = t->excl_idx[2 * e], b = t->excl_idx[2 * e + 1];
+      adj[fill[a]++] = b;
+      adj[fill[b]++] = a;
+    }
+    UPLOAD(d.exstart, start);
+    UPLOAD(d.exadj, adj);
   }
   ALLOC(d.workctr, 4);
   ALLOC(d.errflag, 1);
@@ -1066,7 +1069,7 @@ static int set_tile_capacity(bm_system *s, long long maxTiles) {
   d.maxchunks = (int)(maxTiles / d.tchunk + s->maxBlocks + 1);
   const size_t T = (size_t)maxTiles + 1;
   if ((rc = s->realloc_dev(d.tile_i, T)) || (rc = s->realloc_dev(d.tile_j, T)) ||
-      (rc = s->realloc_dev(d.tile_ex, T)) || (rc = s->realloc_dev(d.tile_flag, T)) ||
+      (rc = s->realloc_dev(d.tile_ex, T)) ||
       (rc = s->realloc_dev(d.chunk, (size_t)d.maxchunks)) ||
       (rc = s->realloc_dev(d.ichunk, (size_t)d.maxchunks * 3 * blade::kBlockAtoms)))
     return rc;
@@ -1281,8 +1284,12 @@ struct bm_batch {
     if (rebuild) {
       // the list rebuild of every member, one launch per rebuild kernel
       blade::Multi rm[blade::kRebuildKernels];
-      for (int k = 0; k < blade::kRebuildKernels; k++) rm[k] = this->rebuild[k].m;
-      blade::launch_domdec_rebuild_multi(rm, st);
+      size_t lds[blade::kRebuildKernels];
+      for (int k = 0; k < blade::kRebuildKernels; k++) {
+        rm[k] = this->rebuild[k].m;
+        lds[k] = this->rebuild[k].lds;
+      }
+      blade::launch_domdec_rebuild_multi(rm, lds, st);
     }
     blade::launch_pack_multi(pack.m, st);
     (void)hipEventRecord(fork2, st);
@@ -1370,8 +1377,10 @@ static int build_plans(bm_batch *b) {
   if ((rc = make_plan(b, b->normals, all, blade::grid_normals))) return rc;
   if ((rc = make_plan(b, b->bonded, all, blade::grid_bonded))) return rc;
   if ((rc = make_plan(b, b->tail, all, blade::grid_tail))) return rc;
-  for (int r = 0; r < blade::kRebuildKernels; r++)
+  for (int r = 0; r < blade::kRebuildKernels; r++) {
     if ((rc = make_plan(b, b->rebuild[r], all, [r](const Dev &d) { return blade::grid_rebuild(d, r); }))) return rc;
+    for (int k : all) b->rebuild[r].lds = std::max(b->rebuild[r].lds, blade::lds_rebuild(D(k), r));
+  }
   if ((rc = make_groups(b, b->bin, pme, [&](int k) { return D(k).order; }, blade::grid_pme_bin))) return rc;
   if ((rc = make_groups(b, b->spread, pme, [&](int k) { return D(k).order; }, blade::grid_pme_spread))) return rc;
   for (size_t g = 0; g < b->bin.size(); g++) {
