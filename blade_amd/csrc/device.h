@@ -33,6 +33,7 @@ constexpr unsigned kFamBond = 1u << 0, kFamAngle = 1u << 1, kFamDihe = 1u << 2, 
 // tile list capacity helpers
 constexpr int kBlockAtoms = 32;      // atoms per block (one half-wave)
 constexpr int kTileChunk = 16;       // most directed tiles in one nonbonded work unit
+constexpr int kClusterAtoms = 8;     // atoms of a pair-kernel cluster (four clusters to a block)
 constexpr int kMaxColumnAtoms = 2048;
 
 // Device view of one system.
@@ -74,6 +75,10 @@ struct Dev {
   unsigned *bblo, *bbhi;         // [3*maxB] rebuild boxes (exact intervals)
   uint4 *bbc;                    // [maxB] per-step box centre (frac counts)
   uint4 *bbh;                    // [maxB] per-step half extent (frac counts), .w = alch flag
+  int clusters;                  // the list is short enough for the pair kernel's clusters
+  unsigned char *sperm;          // [32*maxB] slots of a block by cluster of eight (dd_sort_columns)
+  uint4 *sbc;                    // [4*maxB] per-step cluster box centre (frac counts), .w = alch flag
+  float4 *sbh;                   // [4*maxB] per-step cluster half extent (A; hugely negative: empty)
   uint4 *spos;                   // [32*maxB] slot (ux,uy,uz,q bits)
   int2 *spar;                    // [32*maxB] slot (type or -1, siteBlock)
   int *tcount, *tstart;          // [maxB],[maxB+1] directed tiles per row

@@ -190,6 +190,24 @@ __device__ __forceinline__ void dd_sort_columns_body(const Dev &d, int bid, int 
         lo[q] = min(lo[q], (unsigned)__shfl_xor((int)lo[q], o, 32));
         hi[q] = max(hi[q], (unsigned)__shfl_xor((int)hi[q], o, 32));
       }
+    // clusters of eight for the pair kernel: the block's atoms in two halves
+    // by x, each half in two by y (a block is a z slice of its column, so
+    // the clusters are prisms half as wide as the column); empty slots last
+    if (d.clusters) {
+      const unsigned kx = in ? sx[sorted[r]] : 0xFFFFFFFFu, ky = in ? sy[sorted[r]] : 0xFFFFFFFFu;
+      int rx = 0;
+      for (int o = 0; o < kBlockAtoms; o++) {
+        const unsigned v = (unsigned)__shfl((int)kx, o, 32);
+        rx += v < kx || (v == kx && o < l);
+      }
+      int ry = 0;
+      for (int o = 0; o < kBlockAtoms; o++) {
+        const unsigned v = (unsigned)__shfl((int)ky, o, 32);
+        const int ox = __shfl(rx, o, 32);
+        ry += (ox >> 4) == (rx >> 4) && (v < ky || (v == ky && o < l));
+      }
+      if (bb < nbc) d.sperm[(b0 + bb) * kBlockAtoms + (rx & 16) + ry] = (unsigned char)l;
+    }
     if (bb < nbc && l < 3) {
       d.bblo[3 * (b0 + bb) + l] = l == 0 ? lo[0] : l == 1 ? lo[1] : lo[2];
       d.bbhi[3 * (b0 + bb) + l] = l == 0 ? hi[0] : l == 1 ? hi[1] : hi[2];
@@ -459,21 +477,43 @@ __device__ __forceinline__ void dd_pack_body(const Dev &d, int bid) {
     d.spar[s] = make_int2(-1, 0);
     d.slo[s] = 0.f;
   }
-  // box of the 32-slot block (a half wave); slot 0 of a block is occupied
-  unsigned c[3], h[3];
+  // boxes of the block (a half wave; its slot 0 is occupied) and of its four
+  // clusters: lane l takes the slot at place l of the cluster order, so
+  // eight neighbouring lanes hold one cluster
+  const int l = threadIdx.x & (kBlockAtoms - 1);
+  const int pl = in && d.clusters ? d.sperm[s] : l;
+  const bool occ = __shfl(a, pl, 32) >= 0;
+  int alch = (a >= 0 && d.sb[a] != 0) ? 1 : 0;
+  alch = __shfl(alch, pl, 32);
+  for (int o = 4; o > 0; o >>= 1) alch |= __shfl_xor(alch, o, 32);
+  const int calch = alch;
+  for (int o = 16; o > 4; o >>= 1) alch |= __shfl_xor(alch, o, 32);
+  const unsigned long long om = __ballot(occ);
+  const bool cocc = (om >> (threadIdx.x & 56)) & 0xFFull;
+  unsigned c[3], h[3], cc[3];
+  float ch[3];
   for (int k = 0; k < 3; k++) {
-    unsigned ref = __shfl(u[k], 0, 32);
-    int off = (int)(u[k] - ref);
-    int mn = a >= 0 ? off : 0x7FFFFFFF, mx = a >= 0 ? off : (int)0x80000000;
-    for (int o = 16; o > 0; o >>= 1) {
+    const unsigned ref = __shfl(u[k], 0, 32);
+    const int off = __shfl((int)(u[k] - ref), pl, 32);
+    int mn = occ ? off : 0x7FFFFFFF, mx = occ ? off : (int)0x80000000;
+    for (int o = 4; o > 0; o >>= 1) {
+      mn = min(mn, __shfl_xor(mn, o, 32));
+      mx = max(mx, __shfl_xor(mx, o, 32));
+    }
+    // (mn + mx may pass 2^31: slot 0 need not be in the cluster)
+    cc[k] = cocc ? ref + (unsigned)mn + ((unsigned)(mx - mn) >> 1) : ref;
+    ch[k] = cocc ? (float)((unsigned)(mx - mn + 1) >> 1) * d.fracscale[k] : -1e15f;
+    for (int o = 16; o > 4; o >>= 1) {
       mn = min(mn, __shfl_xor(mn, o, 32));
       mx = max(mx, __shfl_xor(mx, o, 32));
     }
     c[k] = ref + (unsigned)((mn + mx) >> 1);
     h[k] = (unsigned)(mx - mn + 1) >> 1;
   }
-  int alch = (a >= 0 && d.sb[a] != 0) ? 1 : 0;
-  for (int o = 16; o > 0; o >>= 1) alch |= __shfl_xor(alch, o, 32);
+  if (in && d.clusters && (s & (kClusterAtoms - 1)) == 0) {
+    d.sbc[s / kClusterAtoms] = make_uint4(cc[0], cc[1], cc[2], (unsigned)calch);
+    d.sbh[s / kClusterAtoms] = make_float4(ch[0], ch[1], ch[2], 0.f);
+  }
   if (in && (s & (kBlockAtoms - 1)) == 0) {
     const int b = s / kBlockAtoms;
     d.bbc[b] = make_uint4(c[0], c[1], c[2], 0);

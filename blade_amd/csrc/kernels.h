@@ -72,7 +72,8 @@ size_t lds_pme_spread(const Dev &d);
 bool fft_plane_path(const Dev &d);
 int grid_fft_planes(const Dev &d);
 int grid_fft_x(const Dev &d);
-int grid_nbdirect(const Dev &d);
+bool nb_clusters(long long maxchunks);   // the form of a pair-kernel launch over lists of so many chunks
+int grid_nbdirect(const Dev &d, bool clusters);
 int grid_nb_dudl(const Dev &d);
 // FP64 dU/dlambda of the nonbonded pairs, by alchemical atom
 void launch_nb_dudl(const Dev &d, bool soft, hipStream_t st);
@@ -89,7 +90,7 @@ void launch_bonded_multi(const Multi &m, bool energy, hipStream_t st);
 void launch_pme_bin_multi(const Multi &m, int order, hipStream_t st);
 void launch_pme_spread_multi(const Multi &m, int order, size_t lds, hipStream_t st);
 void launch_pme_fft_multi(const Multi &mp, const Multi &mx, int K0, int K1, bool energy, hipStream_t st);
-void launch_nbdirect_multi(const Multi &m, int elec, int vdw, bool energy, bool alch, bool soft, size_t lds,
+void launch_nbdirect_multi(const Multi &m, int elec, int vdw, bool clusters, bool alch, bool soft, size_t lds,
                            hipStream_t st);
 void launch_assemble_multi(const Multi &m, int order, unsigned mask, bool kick, hipStream_t st);
 void launch_tail_multi(const Multi &m, hipStream_t st);

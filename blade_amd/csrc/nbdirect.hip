@@ -530,6 +530,250 @@ __device__ __forceinline__ void chunk_pairs(const Dev &d, const NbConst &c, cons
 
 }
 
+// ---- the same sums by clusters of eight -----------------------------------
+// One workgroup per chunk, one wave per cluster of eight of the 32 i-atoms.
+// Eight tiles at a time are staged in LDS; each wave keeps the slots near
+// its own cluster's box (about two thirds of those near the block's) and
+// evaluates 8 i x 8 j pairs at once.  Each i-atom still sums its pairs in
+// the order of chunk_pairs: entries of even and of odd rank among a tile's
+// slots near the block in two FP32 sums, each serial in the tiles and
+// slots.  A quad of lanes holds one of the two sums of one i-atom, each lane
+// evaluates one entry, and the quad then adds its four results in turn from
+// DPP broadcasts, so the forces are the same to the bit, whichever of the
+// two forms runs.
+constexpr int kGroupTiles = 8;
+constexpr int kGroupSlots = kGroupTiles * kBlockAtoms;   // one per thread
+constexpr unsigned kNoAtom = 0xFFFFFFFFu;   // charge bits of a slot that is empty or not near the block (a NaN)
+
+struct NbStage {
+  uint4 pos[kGroupSlots];
+  int2 par[kGroupSlots];
+  unsigned em[kGroupTiles][kBlockAtoms];     // exclusion words; the diagonal tile's hold j == i too
+  unsigned long long odd[kGroupSlots / 64];  // slots of odd rank among those of their tile near the block
+  // per wave: slots near its cluster, of even and odd rank (the loop reads
+  // two rounds ahead of its entries; any byte is a staged slot)
+  unsigned char list[4][2][kGroupSlots + 16];
+  int4 seq[kTileChunk];                      // the chunk's kept tiles (J, mask index, alch flag)
+};
+
+// j-atom (fractional coordinates pj) within rcut of a cluster box (centre in
+// fractional counts, half extent in A; an empty cluster's is -1e15)
+__device__ __forceinline__ bool near_cluster(const Dev &d, uint4 ci, float4 hi, uint4 pj, float rc2) {
+  const float gx = fmaxf(fmaf(fabsf((float)(int)(pj.x - ci.x)), d.fracscale[0], -hi.x), 0.f);
+  const float gy = fmaxf(fmaf(fabsf((float)(int)(pj.y - ci.y)), d.fracscale[1], -hi.y), 0.f);
+  const float gz = fmaxf(fmaf(fabsf((float)(int)(pj.z - ci.z)), d.fracscale[2], -hi.z), 0.f);
+  return fmaf(gx, gx, fmaf(gy, gy, gz * gz)) <= rc2 * 1.0001f;
+}
+
+// lane k of each quad, to the whole quad (all lanes of the wave active)
+template <int K>
+__device__ __forceinline__ float quad_bcast(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), K * 0x55, 0xF, 0xF, true));
+}
+template <int K>
+__device__ __forceinline__ void quad_add(float fr, float dx, float dy, float dz, float &fx, float &fy, float &fz) {
+  const float f = quad_bcast<K>(fr);
+  fx += f * quad_bcast<K>(dx);
+  fy += f * quad_bcast<K>(dy);
+  fz += f * quad_bcast<K>(dz);
+}
+
+// The pairs of one cluster with the slots of its two lists (n: entries of
+// the longer one): lane l holds i-atom l / 8 (slot is of its block) and
+// entry l % 4 of every four of list l / 4 % 2.  CHK: the group has
+// exclusions or the diagonal tile.
+template <int ELEC, int VDW, bool ALCH, bool SOFT, bool CHK>
+__device__ __forceinline__ void cluster_pairs(const Dev &d, const NbConst &c, const IAtom &ia, int is, int lane,
+                                              const NbStage &st, const unsigned char *list, const float2 *svdw,
+                                              int nown, int n, float &fx, float &fy, float &fz) {
+  const float sx = d.fracscale[0], sy = d.fracscale[1], sz = d.fracscale[2];
+  const int q = lane & 3;
+  // the index two rounds ahead, the position one round ahead
+  int e = list[q], en = list[q + 4];
+  uint4 pn = st.pos[e];
+  for (int p0 = 0; p0 < n; p0 += 4) {
+    const int ic = e;
+    const uint4 pj = pn;
+    e = en;
+    pn = st.pos[e];
+    en = list[p0 + 8 + q];
+    const float dx = fdisp(ia.p.x, pj.x, sx);
+    const float dy = fdisp(ia.p.y, pj.y, sy);
+    const float dz = fdisp(ia.p.z, pj.z, sz);
+    // (spelled out as the compiler contracts tile_pairs' sum)
+    const float r2 = fmaf(dz, dz, fmaf(dx, dx, dy * dy));
+    bool ok = ia.t >= 0 && r2 < c.rc2 && p0 + q < nown;
+    if (CHK) ok = ok && !((st.em[ic >> 5][is] >> (ic & 31)) & 1u);
+    float fr = 0.f;
+    if (ok) {
+      const int2 prj = st.par[ic];
+      const float2 lj = svdw[ia.t * d.ntypes + prj.x];
+      float rinv = __frsqrt_rn(r2);
+      float r = r2 * rinv;
+      const float qq = ia.q * __uint_as_float(pj.w);
+      float s = 1.f, dredr = 1.f, lamj = 1.f;
+      const int bi = ia.b, bj = prj.y;
+      const bool alchPair = ALCH && (bi | bj);
+      if (ALCH && alchPair) {
+        if (bj & 0xFFFF) lamj = d.lambdaf[bj & 0xFFFF];
+        const bool same = (bi & 0xFFFF0000) == (bj & 0xFFFF0000);
+        s = same ? (bi == bj ? ia.lam : 0.f) : ia.lam * lamj;
+        if (SOFT) {
+          const float rSoft = kSoftCoreRadius * (1.f - s);
+          if (r < rSoft) {
+            const float q1 = r / rSoft;
+            float re = 1.f - 0.5f * q1;
+            re = re * q1 * q1 * q1 + 0.5f;
+            dredr = (3.f - 2.f * q1) * q1 * q1;
+            r = re * rSoft;
+            rinv = __builtin_amdgcn_rcpf(r);
+          }
+        }
+      }
+      float f, eq, eA, eB;
+      pair_ef<ELEC, VDW>(c, qq, lj.x, lj.y, r, rinv, f, eq, eA, eB);
+      if (ALCH) f *= s;
+      (void)eq; (void)eA; (void)eB;
+      if (SOFT && alchPair) fr = f * dredr * __frsqrt_rn(r2);
+      else fr = f * rinv;
+    }
+    // entries in turn (those that do not count add a zero)
+    quad_add<0>(fr, dx, dy, dz, fx, fy, fz);
+    quad_add<1>(fr, dx, dy, dz, fx, fy, fz);
+    quad_add<2>(fr, dx, dy, dz, fx, fy, fz);
+    quad_add<3>(fr, dx, dy, dz, fx, fy, fz);
+  }
+}
+
+template <int ELEC, int VDW, bool ALCH, bool SOFT, bool GTABLE>
+__device__ __forceinline__ void nbcluster_body(const Dev &d, int bid) {
+  __shared__ NbStage st;
+  extern __shared__ float2 s_vdw_dyn[];
+  // workgroups past this step's chunk count exit
+  const int nchunks = *d.ntiles <= d.maxtiles && *d.nchunks <= d.maxchunks ? *d.nchunks : 0;
+  if (bid >= nchunks) return;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int4 cr = d.chunk[bid];
+  const int I = cr.x, t0 = cr.y, cnt = cr.z;
+  const NbConst c = make_const(d);
+  if (!GTABLE) {
+    const int nt2 = d.ntypes * d.ntypes;
+    for (int k = threadIdx.x; k < nt2; k += blockDim.x) s_vdw_dyn[k] = d.vdw[k];
+  }
+  const float2 *s_vdw = GTABLE ? d.vdw : s_vdw_dyn;
+  // the tiles whose current block boxes come within rcut, in list order
+  // (every wave finds the same)
+  bool keep = false;
+  int tJ = 0, tE = -1;
+  if (lane < cnt) {
+    tJ = d.tile_j[t0 + lane];
+    tE = d.tile_ex[t0 + lane];
+    keep = boxes_within(d, I, tJ, c.rc2);
+  }
+  const unsigned long long below = (1ull << lane) - 1ull;
+  const unsigned long long mk = __ballot(keep);
+  const int nk = __popcll(mk), rank = __popcll(mk & below);
+  if (w == 0 && keep) st.seq[rank] = make_int4(tJ, tE, ALCH ? (int)d.bbh[tJ].w : 0, 0);
+  const uint4 bc = d.bbc[I], bh = d.bbh[I];
+  // the wave's cluster
+  const uint4 ci = d.sbc[4 * I + w];
+  const float4 hi = d.sbh[4 * I + w];
+  const int is = d.sperm[I * kBlockAtoms + w * kClusterAtoms + (lane >> 3)];
+  IAtom ia;
+  {
+    const int si = I * kBlockAtoms + is;
+    ia.p = d.spos[si];
+    const int2 pr = d.spar[si];
+    ia.t = pr.x;
+    ia.b = pr.y;
+    ia.q = __uint_as_float(ia.p.w) * kElectricF;
+    ia.qd = 0.0;
+    ia.lam = (ALCH && (ia.b & 0xFFFF)) ? d.lambdaf[ia.b & 0xFFFF] : 1.f;
+  }
+  float fx = 0.f, fy = 0.f, fz = 0.f;
+  __syncthreads();
+  // by place in seq: tiles with exclusions or the diagonal, alchemical tiles
+  const int4 sq = lane < nk ? st.seq[lane & (kTileChunk - 1)] : make_int4(-1, -1, 0, 0);
+  const unsigned mc = (unsigned)__ballot(sq.y >= 0 || sq.x == I), ma = ALCH ? (unsigned)__ballot(sq.z != 0) : 0u;
+  // the j slot of this thread in the group starting at tile g; loaded one
+  // group ahead of its use
+  const int tl = threadIdx.x / kBlockAtoms, lj = threadIdx.x % kBlockAtoms;
+  uint4 pj = make_uint4(0, 0, 0, kNoAtom);
+  int2 prj = make_int2(-1, 0);
+  unsigned em = 0u;
+  auto fetch = [&](int g) {
+    prj.x = -1;
+    if (g + tl >= nk) return;
+    const int4 t = st.seq[g + tl];
+    const int sj = t.x * kBlockAtoms + lj;
+    pj = d.spos[sj];
+    prj = d.spar[sj];
+    em = t.y >= 0 ? d.emask[t.y * kBlockAtoms + lj] : 0u;
+    if (t.x == I) em |= 1u << lj;
+  };
+  fetch(0);
+  for (int g = 0; g < nk; g += kGroupTiles) {
+    if (g) __syncthreads();   // the group before has been used
+    const bool gchk = (mc >> g) & 0xFFu;
+    const bool nearb = prj.x >= 0 && near_box(d, bc, bh, pj, c.rc2);
+    const unsigned long long nm = __ballot(nearb);
+    const unsigned long long mine = nm & (lane < 32 ? 0xFFFFFFFFull : ~0xFFFFFFFFull);
+    const unsigned long long odd = __ballot(__popcll(mine & below) & 1);
+    st.pos[threadIdx.x] = make_uint4(pj.x, pj.y, pj.z, nearb ? pj.w : kNoAtom);
+    st.par[threadIdx.x] = prj;
+    if (lane == 0) st.odd[w] = odd;
+    if (gchk) st.em[tl][lj] = em;
+    __syncthreads();
+    if (g + kGroupTiles < nk) fetch(g + kGroupTiles);
+    // the slots near the cluster, by rank parity
+    unsigned char *list = st.list[w][0];
+    const int slots = min(nk - g, kGroupTiles) * kBlockAtoms;
+    int n0 = 0, n1 = 0;
+    for (int e0 = 0; e0 < slots; e0 += 64) {
+      const int e = e0 + lane;
+      const uint4 qp = st.pos[e];
+      const bool near = qp.w != kNoAtom && near_cluster(d, ci, hi, qp, c.rc2);
+      const unsigned long long m = __ballot(near), mo = st.odd[e0 >> 6];
+      const bool o = (mo >> lane) & 1ull;
+      const unsigned long long m1 = m & mo, m0 = m & ~mo;
+      const int at = o ? kGroupSlots + 16 + n1 + __popcll(m1 & below) : n0 + __popcll(m0 & below);
+      if (near) list[at] = (unsigned char)e;
+      n0 += __popcll(m0);
+      n1 += __popcll(m1);
+    }
+    wave_lds_sync();
+    const int h = (lane >> 2) & 1;
+    const unsigned char *own = st.list[w][h];
+    const int nown = h ? n1 : n0, n = max(n0, n1);
+#define BM_TILE(AL, SO, CK) \
+  cluster_pairs<ELEC, VDW, AL, SO, CK>(d, c, ia, is, lane, st, own, s_vdw, nown, n, fx, fy, fz)
+    if (ALCH && (ci.w || ((ma >> g) & 0xFFu))) {
+      if (gchk) BM_TILE(ALCH, SOFT, true);
+      else BM_TILE(ALCH, SOFT, false);
+    } else {
+      if (gchk) BM_TILE(false, false, true);
+      else BM_TILE(false, false, false);
+    }
+#undef BM_TILE
+  }
+  // even + odd sums: the same in either quad
+  fx += __shfl_xor(fx, 4, 64);
+  fy += __shfl_xor(fy, 4, 64);
+  fz += __shfl_xor(fz, 4, 64);
+  const int comp = lane & 7;
+  if (comp < 3) d.ichunk[((long long)bid * 3 + comp) * kBlockAtoms + is] = comp == 0 ? fx : comp == 1 ? fy : fz;
+}
+
+template <int ELEC, int VDW, bool ALCH, bool SOFT, bool GTABLE>
+__global__ void __launch_bounds__(256) nbcluster_kernel(Dev d) { nbcluster_body<ELEC, VDW, ALCH, SOFT, GTABLE>(d, blockIdx.x); }
+
+template <int ELEC, int VDW, bool ALCH, bool SOFT, bool GTABLE>
+__global__ void __launch_bounds__(256) nbcluster_kernel_multi(Multi m) {
+  const MultiBlk b = multi_block(m);
+  const Dev d = m.devs[b.sys];
+  nbcluster_body<ELEC, VDW, ALCH, SOFT, GTABLE>(d, b.bid);
+}
+
 template <int ELEC, int VDW, bool ENERGY, bool ALCH, bool SOFT, bool GTABLE>
 __device__ __forceinline__ void nbdirect_kernel_body(const Dev &d, int bid, int nblk) {
   __shared__ uint4 s_pos[4][kBlockAtoms];
@@ -750,11 +994,16 @@ void launch_nb_dudl(const Dev &d, bool soft, hipStream_t st) {
 void launch_nb_dudl_multi(const Multi &m, int elec, int vdw, bool soft, hipStream_t st) {
   BM_METHODS(launch_dudl_mev, m, soft, st)
 }
-#undef BM_METHODS
 
-// one wave per chunk slot of the list capacity; waves past this step's
-// chunk count exit at once
-int grid_nbdirect(const Dev &d) { return (d.maxchunks + 3) / 4; }
+// Which form sums the chunks of a launch, the same bits either way: clusters
+// (four waves to a chunk, each a quarter as long) where one wave to a chunk
+// would leave SIMDs idle, chunks counted by the lists' capacities (about 1.6
+// times their use).
+bool nb_clusters(long long maxchunks) { return maxchunks <= 9500; }
+
+// workgroups for every chunk slot of the list capacity; those past this
+// step's chunk count exit at once
+int grid_nbdirect(const Dev &d, bool clusters) { return clusters ? d.maxchunks : (d.maxchunks + 3) / 4; }
 
 // the LJ table in LDS (0: the table is read from global memory)
 size_t lds_nbdirect(const Dev &d) {
@@ -762,22 +1011,30 @@ size_t lds_nbdirect(const Dev &d) {
   return nt2 <= kVdwLdsMax ? (size_t)nt2 * sizeof(float2) : 0;
 }
 
+// energy steps run the one-wave form, which carries the FP64 energies
 template <int ELEC, int VDW, bool ENERGY, bool ALCH, bool SOFT>
 static void launch_t(const Dev &d, hipStream_t st) {
-  const unsigned grid = (unsigned)grid_nbdirect(d);
   const size_t lds = lds_nbdirect(d);
-  if (lds)
-    nbdirect_kernel<ELEC, VDW, ENERGY, ALCH, SOFT, false><<<grid, 256, lds, st>>>(d);
-  else
-    nbdirect_kernel<ELEC, VDW, ENERGY, ALCH, SOFT, true><<<grid, 256, 0, st>>>(d);
+  if (!ENERGY && d.clusters) {
+    const unsigned grid = (unsigned)d.maxchunks;
+    if (lds) nbcluster_kernel<ELEC, VDW, ALCH, SOFT, false><<<grid, 256, lds, st>>>(d);
+    else nbcluster_kernel<ELEC, VDW, ALCH, SOFT, true><<<grid, 256, 0, st>>>(d);
+    return;
+  }
+  const unsigned grid = (unsigned)(d.maxchunks + 3) / 4;
+  if (lds) nbdirect_kernel<ELEC, VDW, ENERGY, ALCH, SOFT, false><<<grid, 256, lds, st>>>(d);
+  else nbdirect_kernel<ELEC, VDW, ENERGY, ALCH, SOFT, true><<<grid, 256, 0, st>>>(d);
 }
 
-template <int ELEC, int VDW, bool ENERGY, bool ALCH, bool SOFT>
-static void launch_mt(const Multi &m, size_t lds, hipStream_t st) {
-  if (lds)
-    nbdirect_kernel_multi<ELEC, VDW, ENERGY, ALCH, SOFT, false><<<m.nwg, 256, lds, st>>>(m);
-  else
-    nbdirect_kernel_multi<ELEC, VDW, ENERGY, ALCH, SOFT, true><<<m.nwg, 256, 0, st>>>(m);
+template <int ELEC, int VDW, bool ALCH, bool SOFT>
+static void launch_mt(const Multi &m, bool clusters, size_t lds, hipStream_t st) {
+  if (clusters) {
+    if (lds) nbcluster_kernel_multi<ELEC, VDW, ALCH, SOFT, false><<<m.nwg, 256, lds, st>>>(m);
+    else nbcluster_kernel_multi<ELEC, VDW, ALCH, SOFT, true><<<m.nwg, 256, 0, st>>>(m);
+  } else {
+    if (lds) nbdirect_kernel_multi<ELEC, VDW, false, ALCH, SOFT, false><<<m.nwg, 256, lds, st>>>(m);
+    else nbdirect_kernel_multi<ELEC, VDW, false, ALCH, SOFT, true><<<m.nwg, 256, 0, st>>>(m);
+  }
 }
 
 // systems with lambda sites run the kernel with the lambda arithmetic
@@ -797,53 +1054,24 @@ static void launch_ev(const Dev &d, bool energy, bool alch, bool soft, hipStream
 
 // one launch over several members sharing the methods and flags
 template <int ELEC, int VDW>
-static void launch_mev(const Multi &m, bool energy, bool alch, bool soft, size_t lds, hipStream_t st) {
-  if (!alch) {
-    if (energy) launch_mt<ELEC, VDW, true, false, false>(m, lds, st);
-    else launch_mt<ELEC, VDW, false, false, false>(m, lds, st);
-  } else if (!soft) {
-    if (energy) launch_mt<ELEC, VDW, true, true, false>(m, lds, st);
-    else launch_mt<ELEC, VDW, false, true, false>(m, lds, st);
-  } else {
-    if (energy) launch_mt<ELEC, VDW, true, true, true>(m, lds, st);
-    else launch_mt<ELEC, VDW, false, true, true>(m, lds, st);
-  }
+static void launch_mev(const Multi &m, bool clusters, bool alch, bool soft, size_t lds, hipStream_t st) {
+  if (!alch) launch_mt<ELEC, VDW, false, false>(m, clusters, lds, st);
+  else if (!soft) launch_mt<ELEC, VDW, true, false>(m, clusters, lds, st);
+  else launch_mt<ELEC, VDW, true, true>(m, clusters, lds, st);
 }
 
-// systems sharing the methods and flags; lds: the largest LJ table of the
-// group (0 when any of them is read from global memory)
-void launch_nbdirect_multi(const Multi &m, int elec, int vdw, bool energy, bool alch, bool soft, size_t lds,
+// systems sharing the methods, flags and form; lds: the largest LJ table of
+// the group (0 when any of them is read from global memory)
+void launch_nbdirect_multi(const Multi &m, int elec, int vdw, bool clusters, bool alch, bool soft, size_t lds,
                            hipStream_t st) {
-  if (elec == BM_PME) {
-    if (vdw == BM_VFSWITCH) launch_mev<BM_PME, BM_VFSWITCH>(m, energy, alch, soft, lds, st);
-    else if (vdw == BM_VSWITCH) launch_mev<BM_PME, BM_VSWITCH>(m, energy, alch, soft, lds, st);
-    else launch_mev<BM_PME, BM_VSHIFT>(m, energy, alch, soft, lds, st);
-  } else if (elec == BM_FSWITCH) {
-    if (vdw == BM_VFSWITCH) launch_mev<BM_FSWITCH, BM_VFSWITCH>(m, energy, alch, soft, lds, st);
-    else if (vdw == BM_VSWITCH) launch_mev<BM_FSWITCH, BM_VSWITCH>(m, energy, alch, soft, lds, st);
-    else launch_mev<BM_FSWITCH, BM_VSHIFT>(m, energy, alch, soft, lds, st);
-  } else {
-    if (vdw == BM_VFSWITCH) launch_mev<BM_FSHIFT, BM_VFSWITCH>(m, energy, alch, soft, lds, st);
-    else if (vdw == BM_VSWITCH) launch_mev<BM_FSHIFT, BM_VSWITCH>(m, energy, alch, soft, lds, st);
-    else launch_mev<BM_FSHIFT, BM_VSHIFT>(m, energy, alch, soft, lds, st);
-  }
+  BM_METHODS(launch_mev, m, clusters, alch, soft, lds, st)
 }
 
 void launch_nbdirect(const Dev &d, bool energy, bool alch, bool soft, int nwg, hipStream_t st) {
   (void)nwg;
-  if (d.elecmethod == BM_PME) {
-    if (d.vdwmethod == BM_VFSWITCH) launch_ev<BM_PME, BM_VFSWITCH>(d, energy, alch, soft, st);
-    else if (d.vdwmethod == BM_VSWITCH) launch_ev<BM_PME, BM_VSWITCH>(d, energy, alch, soft, st);
-    else launch_ev<BM_PME, BM_VSHIFT>(d, energy, alch, soft, st);
-  } else if (d.elecmethod == BM_FSWITCH) {
-    if (d.vdwmethod == BM_VFSWITCH) launch_ev<BM_FSWITCH, BM_VFSWITCH>(d, energy, alch, soft, st);
-    else if (d.vdwmethod == BM_VSWITCH) launch_ev<BM_FSWITCH, BM_VSWITCH>(d, energy, alch, soft, st);
-    else launch_ev<BM_FSWITCH, BM_VSHIFT>(d, energy, alch, soft, st);
-  } else {
-    if (d.vdwmethod == BM_VFSWITCH) launch_ev<BM_FSHIFT, BM_VFSWITCH>(d, energy, alch, soft, st);
-    else if (d.vdwmethod == BM_VSWITCH) launch_ev<BM_FSHIFT, BM_VSWITCH>(d, energy, alch, soft, st);
-    else launch_ev<BM_FSHIFT, BM_VSHIFT>(d, energy, alch, soft, st);
-  }
+  const int elec = d.elecmethod, vdw = d.vdwmethod;
+  BM_METHODS(launch_ev, d, energy, alch, soft, st)
 }
+#undef BM_METHODS
 
 }  // namespace blade

@@ -308,6 +308,7 @@ int bm_system_create(int device, const bm_topology *t, const bm_runparams *rp, c
   s->maxTiles0 = s->maxTiles;
   d.tchunk = rp->tile_chunk > 0 ? rp->tile_chunk : kTileChunk;
   d.maxchunks = (int)(s->maxTiles / d.tchunk + s->maxBlocks + 1);
+  d.clusters = nb_clusters(d.maxchunks);
   const int MB = s->maxBlocks;
   int rc = 0;
 #define ALLOC(p, c) \
@@ -419,6 +420,13 @@ int bm_system_create(int device, const bm_topology *t, const bm_runparams *rp, c
   ALLOC(d.bbhi, 3 * (size_t)MB);
   ALLOC(d.bbc, MB);
   ALLOC(d.bbh, MB);
+  {
+    std::vector<unsigned char> id((size_t)MB * kBlockAtoms);
+    for (size_t k = 0; k < id.size(); k++) id[k] = (unsigned char)(k % kBlockAtoms);
+    UPLOAD(d.sperm, id);
+  }
+  ALLOC(d.sbc, (size_t)MB * (kBlockAtoms / kClusterAtoms));
+  ALLOC(d.sbh, (size_t)MB * (kBlockAtoms / kClusterAtoms));
   ALLOC(d.spos, (size_t)MB * kBlockAtoms);
   ALLOC(d.slo, (size_t)MB * kBlockAtoms);
   ALLOC(d.spar, (size_t)MB * kBlockAtoms);
@@ -1223,7 +1231,7 @@ struct MultiPlan {
   int *wg0_d = nullptr;            // device
   // the group's template keys
   int order = 0, K0 = 0, K1 = 0, elec = 0, vdw = 0;
-  bool alch = false, soft = false;
+  bool alch = false, soft = false, clusters = false;
   size_t lds = 0;
 };
 
@@ -1295,7 +1303,7 @@ struct bm_batch {
     (void)hipEventRecord(fork2, st);
     // nbdirect first: the largest kernel takes the CUs before the second
     // stream's smaller ones fill them
-    for (MultiPlan &p : nb) blade::launch_nbdirect_multi(p.m, p.elec, p.vdw, false, p.alch, p.soft, p.lds, st);
+    for (MultiPlan &p : nb) blade::launch_nbdirect_multi(p.m, p.elec, p.vdw, p.clusters, p.alch, p.soft, p.lds, st);
     (void)hipStreamWaitEvent(st2, fork2, 0);
     (void)hipStreamWaitEvent(st3, fork2, 0);
     // the FP64 dU/dlambda of the members' alchemical atoms, the normals and
@@ -1409,7 +1417,15 @@ static int build_plans(bm_batch *b) {
   std::vector<int> alchm;
   for (int k : all)
     if (b->sys[k]->alch) alchm.push_back(k);
-  if ((rc = make_groups(b, b->nb, all, nkey, blade::grid_nbdirect))) return rc;
+  long long chunks = 0;
+  bool clusters = true;
+  for (int k : all) {
+    chunks += D(k).maxchunks;
+    clusters = clusters && D(k).clusters;
+  }
+  clusters = clusters && blade::nb_clusters(chunks);
+  if ((rc = make_groups(b, b->nb, all, nkey, [=](const Dev &d) { return blade::grid_nbdirect(d, clusters); })))
+    return rc;
   auto dkey = [&](int k) {
     const bm_system *s = b->sys[k];
     return std::make_tuple(s->d.elecmethod, s->d.vdwmethod, s->soft);
@@ -1422,6 +1438,7 @@ static int build_plans(bm_batch *b) {
       p.vdw = s->d.vdwmethod;
       p.alch = s->alch;
       p.soft = s->soft;
+      p.clusters = clusters;
       p.lds = 0;
       if (blade::lds_nbdirect(s->d))
         for (int k : p.members) p.lds = std::max(p.lds, blade::lds_nbdirect(D(k)));
