@@ -8,6 +8,8 @@
 // 1e-3 kcal/mol dU/dlambda bar.  Forces go to per-term slots, not to the
 // force array: no global atomics (the force assembly sums them per atom).
 #include "kernels.h"
+#include "normals.h"
+#include "spread.h"
 #include "erfc_coef.h"
 
 namespace blade {
@@ -789,10 +791,47 @@ __global__ void __launch_bounds__(256) bonded_kernel(Dev d, BondedLaunch L, bool
   bonded_body(d, L, blockIdx.x, energy);
 }
 
-__global__ void __launch_bounds__(256) bonded_multi(Multi m, bool energy) {
-  const MultiBlk b = multi_block(m);
-  const Dev d = m.devs[b.sys];
-  bonded_body(d, bonded_layout(d), b.bid, energy);
+// What a step computes from the packed positions beside the pair kernel, in
+// one launch: the PME spread's bricks (the longest, so they start first),
+// the bonded terms and the step's normals.  Each is a few microseconds of
+// dependent loads on a part of the chip; as launches of their own they cost
+// three starts in a row (about 2 us each in a linear graph), or, on a branch
+// beside the pair kernel, wait tens of microseconds for CU slots: the first
+// kernel of such a branch took 30-50 us at 23,558 atoms, 5 us alone.
+// N = 0: no spread.
+template <int N>
+__global__ void __launch_bounds__(256) side_kernel(Dev d, BondedLaunch L, bool energy, int nspread, int nbonded) {
+  int b = blockIdx.x;
+  if constexpr (N > 0) {
+    if (b < nspread) {
+      pme_spread_body<N>(d, b);
+      return;
+    }
+  }
+  b -= nspread;
+  if (b < nbonded) bonded_body(d, L, b, energy);
+  else upd_normals_body(d, b - nbonded);
+}
+
+// the same over several systems; the spread's plan holds the PME members of
+// spline order N
+template <int N>
+__global__ void __launch_bounds__(256) side_multi(Multi ms, Multi mb, Multi mn, bool energy) {
+  int b = blockIdx.x;
+  if constexpr (N > 0) {
+    if (b < ms.nwg) {
+      const MultiBlk k = multi_block(ms, b);
+      const Dev d = ms.devs[k.sys];
+      pme_spread_body<N>(d, k.bid);
+      return;
+    }
+    b -= ms.nwg;
+  }
+  const bool bonded = b < mb.nwg;
+  const MultiBlk k = bonded ? multi_block(mb, b) : multi_block(mn, b - mb.nwg);
+  const Dev d = bonded ? mb.devs[k.sys] : mn.devs[k.sys];
+  if (bonded) bonded_body(d, bonded_layout(d), k.bid, energy);
+  else upd_normals_body(d, k.bid);
 }
 
 int grid_bonded(const Dev &d) { return bonded_layout(d).b_bias + 1; }
@@ -801,6 +840,25 @@ void launch_bonded(const Dev &d, bool energy, unsigned fam, hipStream_t st) {
   bonded_kernel<<<grid_bonded(d), 256, 0, st>>>(d, bonded_layout(d, fam), energy);
 }
 
-void launch_bonded_multi(const Multi &m, bool energy, hipStream_t st) { bonded_multi<<<m.nwg, 256, 0, st>>>(m, energy); }
+void launch_side(const Dev &d, bool energy, bool normals, hipStream_t st) {
+  const bool pme = d.elecmethod == BM_PME;
+  const int ns = pme ? grid_pme_spread(d) : 0, nb = grid_bonded(d), nn = normals ? grid_normals(d) : 0;
+  const unsigned g = (unsigned)(ns + nb + nn);
+  const BondedLaunch L = bonded_layout(d, kFamAll);
+  if (!pme) side_kernel<0><<<g, 256, 0, st>>>(d, L, energy, ns, nb);
+  else if (d.order == 4) side_kernel<4><<<g, 256, lds_pme_spread(d), st>>>(d, L, energy, ns, nb);
+  else if (d.order == 6) side_kernel<6><<<g, 256, lds_pme_spread(d), st>>>(d, L, energy, ns, nb);
+  else side_kernel<8><<<g, 256, lds_pme_spread(d), st>>>(d, L, energy, ns, nb);
+}
+
+void launch_side_multi(const Multi *spread, const Multi &bonded, const Multi &normals, int order, size_t lds,
+                       bool energy, hipStream_t st) {
+  const Multi ms = spread ? *spread : Multi{};
+  const unsigned g = (unsigned)(ms.nwg + bonded.nwg + normals.nwg);
+  if (!spread) side_multi<0><<<g, 256, 0, st>>>(ms, bonded, normals, energy);
+  else if (order == 4) side_multi<4><<<g, 256, lds, st>>>(ms, bonded, normals, energy);
+  else if (order == 6) side_multi<6><<<g, 256, lds, st>>>(ms, bonded, normals, energy);
+  else side_multi<8><<<g, 256, lds, st>>>(ms, bonded, normals, energy);
+}
 
 }  // namespace blade

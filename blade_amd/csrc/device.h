@@ -106,13 +106,17 @@ struct Dev {
   int vdwmethod, elecmethod;
   // PME
   int K[3], order;
-  float *rgrid;                  // [K0*K1*K2] real charge grid (spread output)
-  int pnb[3];                    // spread bricks per axis (each >= order-1 points)
+  float *rgrid;                  // [K0*K1*K2] potential grid (inverse FFT output); before the FFT
+                                 // the charge grid, where pme_sum runs
+  int pnb[3];                    // spread bricks per axis (each >= order-1 points, or the whole axis)
+  int ppad[3], pvol;             // padded brick: points per axis (largest brick + order-1; z odd), in all
+  long long *pgrid;              // [nbricks*pvol] padded bricks of the charge grid, fixed point
+  longlong2 *paxis;              // [K0+K1+K2] places of a grid point in pgrid, by axis: its own brick and
+                                 // the overhang of the brick before (-1: none); the three axes add up
   int pcap;                      // atoms per brick bin
   int *pbcount;                  // [nbricks] atoms binned per brick, zeroed by the gather
-  unsigned *pbhdr;               // [nbricks*pcap] each record's first stencil point, 10 bits per axis
-  double *pbrec;                 // [nbricks*pcap] spline records by home brick
-                                 // (pme_spline_rec_words(order) doubles each)
+  uint4 *pbpos;                  // [nbricks*pcap] fractional coordinates of the atoms by brick
+  double *pblq;                  // [nbricks*pcap] their lambda*q
   float2 *cgrid;                 // [K0*K1*K2] complex work grid
   float2 *twiddle;               // [K0+K1+K2] e^{-2 pi i k/K} per axis
   float *bmod[3];                // [K] B-spline moduli per axis
@@ -199,10 +203,6 @@ struct Dev {
   unsigned long long seed;
   long long *step;               // [1] step counter (RNG counter), advanced on device
 };
-
-// One atom's PME spread record: lambda*q, the B-spline weights along each
-// axis and the first stencil point per axis (as doubles: exact small ints).
-__host__ __device__ constexpr int pme_spline_rec_words(int order) { return 1 + 3 * order + 3; }
 
 __device__ __forceinline__ long long fix_f(float v) {
   return (long long)__float2ll_rn(v * kFixScaleF);
@@ -314,6 +314,43 @@ __device__ __forceinline__ int wave_claim(int *counters, int key, bool active) {
   return active ? base + __popcll(grp & ((1ull << lane) - 1ull)) : 0;
 }
 
+// Brick of grid point u on an axis of K points cut into nb bricks; brick b
+// covers [b*K/nb, (b+1)*K/nb).
+__device__ __forceinline__ int brick_of(int u, int K, int nb) {
+  int b = (u * nb) / K;
+  if (b + 1 < nb && ((b + 1) * K) / nb <= u) b++;
+  return b;
+}
+
+// Bin atom i at fractional coordinates u (i < 0: none; every lane of the
+// wave must call it) by the brick holding its first stencil point: its
+// coordinates and lambda*q, 24 bytes.  Callers walk the list slots
+// (spatially ordered), so a wave's atoms share few bricks and one atomic
+// serves each brick.  Bin order is arbitrary; the spread sums in fixed
+// point, so the grid does not depend on it.
+__device__ __forceinline__ void pme_bin_atom(const Dev &d, int i, uint4 u) {
+  bool act = false;
+  int br = 0;
+  double lq = 0.0;
+  if (i >= 0) {
+    const int b = d.sb[i] & 0xFFFF;
+    lq = d.qd[i] * (b ? d.lambda[b] : 1.0);
+    act = lq != 0.0;
+    const int bx = brick_of((int)__umulhi(u.x, (unsigned)d.K[0]), d.K[0], d.pnb[0]);
+    const int by = brick_of((int)__umulhi(u.y, (unsigned)d.K[1]), d.K[1], d.pnb[1]);
+    const int bz = brick_of((int)__umulhi(u.z, (unsigned)d.K[2]), d.K[2], d.pnb[2]);
+    br = (bx * d.pnb[1] + by) * d.pnb[2] + bz;
+  }
+  const int slot = wave_claim(d.pbcount, br, act);
+  if (!act) return;
+  if (slot < d.pcap) {
+    d.pbpos[(long long)br * d.pcap + slot] = u;
+    d.pblq[(long long)br * d.pcap + slot] = lq;
+  } else {
+    atomicOr(d.errflag, 2);
+  }
+}
+
 // Several systems in one launch (batches): the workgroups of system k are
 // [wg0[k], wg0[k+1]) of the grid; devs holds device copies of the systems'
 // Dev.  A kernel body runs with its system's Dev and its workgroup index
@@ -328,8 +365,8 @@ struct MultiBlk {
   int sys, bid, nblk;
 };
 
-__device__ __forceinline__ MultiBlk multi_block(const Multi &m) {
-  const int b = blockIdx.x;
+// workgroup b of the launch's plan m
+__device__ __forceinline__ MultiBlk multi_block(const Multi &m, int b) {
   int lo = 0, hi = m.nsys - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
@@ -337,6 +374,23 @@ __device__ __forceinline__ MultiBlk multi_block(const Multi &m) {
     else hi = mid - 1;
   }
   return MultiBlk{lo, b - m.wg0[lo], m.wg0[lo + 1] - m.wg0[lo]};
+}
+__device__ __forceinline__ MultiBlk multi_block(const Multi &m) { return multi_block(m, blockIdx.x); }
+
+// The charge of grid point (x, y, z) from the spread's padded bricks, given
+// its entries of the three axis tables: every brick that reaches the point,
+// an exact integer sum.  All eight loads are issued (the missing ones from
+// word 0): behind branches each would wait for the one before.
+__device__ __forceinline__ float pme_charge(const long long *pgrid, longlong2 ax, longlong2 ay, longlong2 az) {
+  long long t[8];
+#pragma unroll
+  for (int q = 0; q < 8; q++) {
+    const long long x = q & 4 ? ax.y : ax.x, y = q & 2 ? ay.y : ay.x, z = q & 1 ? az.y : az.x;
+    const bool in = (x | y | z) >= 0;
+    t[q] = pgrid[in ? x + y + z : 0];
+    t[q] = in ? t[q] : 0;
+  }
+  return (float)((double)(((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]))) * kFixInvD);
 }
 
 // Block-wide fixed-point energy sum (any blockDim multiple of 64).

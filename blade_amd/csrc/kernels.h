@@ -12,7 +12,8 @@ constexpr int kRebuildKernels = 5;
 int grid_rebuild(const Dev &d, int k);
 size_t lds_rebuild(const Dev &d, int k);
 void launch_domdec_rebuild_multi(const Multi *m, const size_t *lds, hipStream_t st);
-void launch_domdec_pack(const Dev &d, int maxBlocks, hipStream_t st);
+// bin: with the PME bins of this step
+void launch_domdec_pack(const Dev &d, int maxBlocks, hipStream_t st, bool bin = false);
 // the pair kernel over the list's chunks (the FP64 dU/dlambda of the
 // alchemical atoms is launch_nb_dudl)
 void launch_nbdirect(const Dev &d, bool energy, bool alch, bool soft, int nwg, hipStream_t st);
@@ -27,6 +28,9 @@ void launch_force_assemble(const Dev &d, unsigned mask, hipStream_t st, bool kic
 bool pme_grid_supported(int K);
 // the term families in fam (kFam*); families left out zero their slots
 void launch_bonded(const Dev &d, bool energy, unsigned fam, hipStream_t st);
+// the PME spread (its bins filled), every bonded term and, with normals, the
+// standard normals of the current step, in one launch
+void launch_side(const Dev &d, bool energy, bool normals, hipStream_t st);
 // the standard normals of the current step (the O step reads them)
 void launch_normals(const Dev &d, hipStream_t st);
 // a whole update; launches its own normals
@@ -48,13 +52,18 @@ void launch_virtual_spread(const Dev &d, hipStream_t st);
 void launch_volume_move(const Dev &d, const double *scale, const double *oldbox, hipStream_t st);
 void launch_volume_restore(const Dev &d, hipStream_t st);
 void launch_set_step(const Dev &d, long long step, hipStream_t st);
-// the bins and spread of launch_pme_grid alone
+// the bins and the spread of launch_pme_grid alone
+void launch_pme_bin(const Dev &d, hipStream_t st);
 void launch_pme_spread(const Dev &d, hipStream_t st);
 // the FFT part of launch_pme_grid alone
 void launch_pme_fft(const Dev &d, bool energy, hipStream_t st);
 // the MFMA split-BF16x3 form of it (every grid edge fft_mfma_supported)
 bool fft_mfma_supported(int K);
-// the MFMA form over several members with K1 == K2 and equal grids
+// the charge grids of several members from their spread's bricks
+int grid_pme_sum(const Dev &d);
+void launch_pme_sum_multi(const Multi &m, hipStream_t st);
+// the MFMA form over several members with K1 == K2 and equal grids, their
+// charge grids summed
 int grid_fft_mfma_planes(const Dev &d);
 int grid_fft_mfma_x(const Dev &d);
 void launch_pme_fft_mfma_multi(const Multi &mp, const Multi &mx, int K0, int K1, bool energy, hipStream_t st);
@@ -66,7 +75,6 @@ void launch_pme_fft_mfma(const Dev &d, bool energy, hipStream_t st);
 int grid_pack(const Dev &d);
 int grid_normals(const Dev &d);
 int grid_bonded(const Dev &d);
-int grid_pme_bin(const Dev &d);
 int grid_pme_spread(const Dev &d);
 size_t lds_pme_spread(const Dev &d);
 bool fft_plane_path(const Dev &d);
@@ -82,12 +90,12 @@ size_t lds_nbdirect(const Dev &d);
 int grid_assemble(const Dev &d);
 int grid_tail(const Dev &d);
 // Every system of a Multi must share the template keys of its kernel: the
-// spline order (bin, spread, assembly), the grid sizes (FFT), the methods
+// spline order (spread, assembly), the grid sizes (FFT), the methods
 // and flags (nbdirect).
-void launch_pack_multi(const Multi &m, hipStream_t st);
-void launch_normals_multi(const Multi &m, hipStream_t st);
-void launch_bonded_multi(const Multi &m, bool energy, hipStream_t st);
-void launch_pme_bin_multi(const Multi &m, int order, hipStream_t st);
+void launch_pack_multi(const Multi &m, hipStream_t st);   // with the PME bins
+// launch_side over several systems (spread: null for no PME member)
+void launch_side_multi(const Multi *spread, const Multi &bonded, const Multi &normals, int order, size_t lds,
+                       bool energy, hipStream_t st);
 void launch_pme_spread_multi(const Multi &m, int order, size_t lds, hipStream_t st);
 void launch_pme_fft_multi(const Multi &mp, const Multi &mx, int K0, int K1, bool energy, hipStream_t st);
 void launch_nbdirect_multi(const Multi &m, int elec, int vdw, bool clusters, bool alch, bool soft, size_t lds,

@@ -2,14 +2,14 @@
 // (restates nbrecip/nbrecip.cu:19-485 and the grid setup of
 // system/potential.cxx:1202-1307; cuFFT is replaced by our own FFT).
 //
-//   pme_bin      atoms -> spline records (lambda*q, FP64 B-spline weights,
-//                first stencil point) in bins of the grid brick holding
-//                their first stencil point
-//   pme_spread   one workgroup per brick: lambda*q B-spline weights summed
-//                as 64-bit fixed point in LDS (order-independent sums:
-//                bit-reproducible), brick stored to the real grid
+//   pme_bin      atoms (coordinates, lambda*q) into bins of the grid brick
+//                holding their first stencil point (in a step, dd_pack)
+//   pme_spread   one workgroup per brick: lambda*q B-spline weights of its
+//                atoms summed as 64-bit fixed point in LDS (order-independent
+//                sums: bit-reproducible) over the brick and its overhang
 //   fft_lines    mixed-radix Stockham FFT of grid lines staged in LDS;
-//                pass z reads the real grid, pass x fuses forward FFT, the
+//                pass z reads the real grid (the overlapping bricks added
+//                up by pme_sum; the plane kernels add them themselves), pass x fuses forward FFT, the
 //                convolution
 //                B(m) kE/(2 pi V) exp(-pi^2 m^2/beta^2)/m^2 and the inverse
 //   force_assemble  potential gradient at each atom -> force, dU/dlambda;
@@ -17,326 +17,51 @@
 #include <algorithm>
 
 #include "kernels.h"
+#include "spread.h"
 
 namespace blade {
 
-// B-spline weights of order N: w[t] = M_N(frac+N-1-t) for grid point u0+t,
-// dw[t] its derivative (M_{N-1}(x) - M_{N-1}(x-1)).
-template <int N, class T>
-__device__ __forceinline__ void bspline_w(T frac, T *w, T *dw) {
-  T A[N];
-  A[0] = T(1);
-#pragma unroll
-  for (int k = 1; k < N; k++) A[k] = T(0);
-#pragma unroll
-  for (int m = 2; m <= N; m++) {
-    if (m == N) {
-#pragma unroll
-      for (int k = 0; k < N; k++) dw[N - 1 - k] = A[k] - (k ? A[k - 1] : T(0));
-    }
-    const T inv = T(1) / T(m - 1);
-#pragma unroll
-    for (int k = m - 1; k >= 0; k--) {
-      T a = (frac + T(k)) * A[k];
-      T b = k ? (T(m) - frac - T(k)) * A[k - 1] : T(0);
-      A[k] = (a + b) * inv;
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < N; k++) w[N - 1 - k] = A[k];
-}
-
-// grid index and fraction from the 32-bit fractional coordinate
-template <class T>
-__device__ __forceinline__ void grid_coord(unsigned u, int K, int &u0, T &frac) {
-  unsigned long long p = (unsigned long long)u * (unsigned)K;
-  u0 = (int)(p >> 32);
-  frac = (T)((unsigned)(p & 0xFFFFFFFFull)) * (T(1) / T(4294967296.0));
-}
-
-// Brick of grid point u on an axis of K points cut into nb bricks; brick b
-// covers [b*K/nb, (b+1)*K/nb).
-__device__ __forceinline__ int brick_of(int u, int K, int nb) {
-  int b = (u * nb) / K;
-  if (b + 1 < nb && ((b + 1) * K) / nb <= u) b++;
-  return b;
-}
-
-// Bin every charged atom by the brick holding its first stencil point, as
-// a spread record: lambda*q, the FP64 B-spline weights of each axis and the
-// first stencil point (computed once per atom; every brick the stencil
-// reaches reads them), and a 4-byte header holding the first stencil point
-// alone (10 bits per axis), so that a brick reads the weights only of the
-// atoms whose stencils reach it.  Threads walk the list slots (spatially ordered), so
-// a wave's atoms share few bricks and one atomic serves each brick.  Bin
-// order is arbitrary; the spread sums in fixed point, so the grid does not
-// depend on it.
-template <int N>
-__device__ __forceinline__ void pme_bin_body(const Dev &d, int bid, int nblk) {
+// the bins alone, for evaluations outside a step (a step's pack bins)
+__global__ void __launch_bounds__(256) pme_bin(Dev d) {
   // a halted step bins nothing (its bins would never be cleared)
   if (halted_wg(d)) return;
-  constexpr int W = pme_spline_rec_words(N);
-  const int s = bid * blockDim.x + threadIdx.x;
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
   const int i = s < *d.nblocks * kBlockAtoms ? d.l2g[s] : -1;
-  bool act = false;
-  int br = 0;
-  double lq = 0.0, w[3][N];
-  int u0[3] = {0, 0, 0};
-  if (i >= 0) {
-    const int b = d.sb[i] & 0xFFFF;
-    lq = d.qd[i] * (b ? d.lambda[b] : 1.0);
-    act = lq != 0.0;
-    int bb[3];
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      double fr, dw[N];
-      grid_coord(frac_u32(d.pos[k * d.n + i], d.invbox[k]), d.K[k], u0[k], fr);
-      bspline_w<N>(fr, w[k], dw);
-      bb[k] = brick_of(u0[k], d.K[k], d.pnb[k]);
-    }
-    br = (bb[0] * d.pnb[1] + bb[1]) * d.pnb[2] + bb[2];
-  }
-  const int slot = wave_claim(d.pbcount, br, act);
-  if (act) {
-    if (slot < d.pcap) {
-      double *r = d.pbrec + ((long long)br * d.pcap + slot) * W;
-      r[0] = lq;
-#pragma unroll
-      for (int k = 0; k < 3; k++)
-#pragma unroll
-        for (int t = 0; t < N; t++) r[1 + k * N + t] = w[k][t];
-#pragma unroll
-      for (int k = 0; k < 3; k++) r[1 + 3 * N + k] = (double)u0[k];
-      d.pbhdr[(long long)br * d.pcap + slot] = (unsigned)u0[0] | (unsigned)u0[1] << 10 | (unsigned)u0[2] << 20;
-    } else {
-      atomicOr(d.errflag, 2);
-    }
-  }
-}
-
-template <int N>
-__global__ void __launch_bounds__(256) pme_bin(Dev d) { pme_bin_body<N>(d, blockIdx.x, gridDim.x); }
-
-template <int N>
-__global__ void __launch_bounds__(256) pme_bin_multi(Multi m) {
-  const MultiBlk b = multi_block(m);
-  const Dev d = m.devs[b.sys];
-  pme_bin_body<N>(d, b.bid, b.nblk);
-}
-
-// candidate atoms staged per round.  The spread runs beside the pair
-// kernel, so a smaller workgroup footprint (about 30 KB of LDS for one
-// system, 15 KB in the batched launch, which has many more bricks) lets
-// more bricks share CUs with it: measured over staging sizes 32-256, these
-// gave the fastest steps (the spread alone is a little slower)
-template <int N> constexpr int spread_stage() { return N <= 6 ? 128 : 64; }
-template <int N> constexpr int spread_stage_multi() { return N <= 6 ? 64 : 32; }
-
-// v * 2^32 rounded to the nearest integer (ties to even), as
-// __double2ll_rn(v * 2^32) gives, for |v * 2^32| < 2^51: the sum with
-// 1.5 * 2^52 is rounded to an integer by the addition itself, and its low
-// mantissa bits are that integer plus a constant.
-__device__ __forceinline__ long long fix_d_small(double v) {
-  const double magic = 6755399441055744.0;   // 1.5 * 2^52
-  return __double_as_longlong(fma(v, 4294967296.0, magic)) - __double_as_longlong(magic);
-}
-
-// Exclusive prefix sum of v over a 256-thread workgroup; the sum of all
-// values goes to total.  Every thread must call it.
-__device__ __forceinline__ int block_scan256(int v, int *s_wsum, int &total) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  int x = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(x, o, 64);
-    if (lane >= o) x += y;
-  }
-  if (lane == 63) s_wsum[w] = x;
-  __syncthreads();
-  int pre = 0, tot = 0;
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int t = s_wsum[k];
-    if (k < w) pre += t;
-    tot += t;
-  }
-  total = tot;
-  return pre + x - v;
-}
-
-// The part of a stencil of N points starting at r (relative to the brick,
-// in [0, K)) that falls inside a brick of sz points: stencil points
-// t0 .. t0+n-1 at brick positions p0 .. p0+n-1 (mod K when the brick is the
-// whole axis), packed as t0 | n << 4 | p0 << 8.
-template <int N>
-__device__ __forceinline__ int stencil_clip(int r, int sz, int K) {
-  int t0 = 0, n = N, p0 = r;
-  if (sz < K) {
-    if (r < sz) {
-      n = min(N, sz - r);
-    } else {          // starts in the previous brick and wraps into this one
-      t0 = K - r;
-      if (t0 >= N) return 0;
-      n = N - t0;
-      p0 = 0;
-    }
-  }
-  return t0 | n << 4 | p0 << 8;
-}
-
-// One workgroup (256 threads) per brick.  Every brick spans >= order-1
-// points (or a whole axis), so only atoms binned in this brick or the
-// previous one along each axis can reach it.  Each round takes up to
-// spread_stage<N>() of those atoms, clips each stencil to the brick from
-// the record header alone, and stages the spline records (FP64 lambda*q,
-// B-spline weights) of the atoms whose stencils reach the brick, with the
-// part of each stencil inside it; it lists the (atom, x, y) stencil rows
-// that cross the brick and gives each thread one row at a time; its z
-// points are added as 64-bit fixed point in LDS.  The brick is
-// stored to the real grid with plain stores: no global atomics, and no
-// clearing pass.
-template <int N, int kStage>
-__device__ __forceinline__ void pme_spread_body(const Dev &d, int bid, int nblk) {
-  extern __shared__ long long acc[];
-  __shared__ double s_w[3][N][kStage];
-  __shared__ int s_clip[3][kStage];
-  __shared__ double s_lq[kStage];
-  __shared__ unsigned short s_row[kStage * N * N];   // atom | x << 8 | y << 11
-  __shared__ int s_cnt[9];
-  __shared__ int s_bin[8];
-  __shared__ int s_wsum[4];
-  int bidx[3], lo[3], sz[3];
-  {
-    int r = bid;
-    bidx[2] = r % d.pnb[2]; r /= d.pnb[2];
-    bidx[1] = r % d.pnb[1];
-    bidx[0] = r / d.pnb[1];
-  }
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    lo[k] = (bidx[k] * d.K[k]) / d.pnb[k];
-    sz[k] = ((bidx[k] + 1) * d.K[k]) / d.pnb[k] - lo[k];
-  }
-  // padded row of an odd number of 64-bit words: lanes on consecutive rows
-  // fall in different LDS banks
-  const int rowz = sz[2] + 1 + (sz[2] & 1);
-  const int npts = sz[0] * sz[1] * rowz;
-  for (int p = threadIdx.x; p < npts; p += blockDim.x) acc[p] = 0;
-  // feeding bins (this brick and the previous one along each axis, each
-  // once) and their atom counts
-  if (threadIdx.x < 8) {
-    const int f = threadIdx.x;
-    int fb[3];
-    bool dup = false;
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      const int off = (f >> k) & 1;
-      if (off && d.pnb[k] == 1) dup = true;
-      fb[k] = bidx[k] - off < 0 ? d.pnb[k] - 1 : bidx[k] - off;
-    }
-    const int br = (fb[0] * d.pnb[1] + fb[1]) * d.pnb[2] + fb[2];
-    s_bin[f] = br;
-    s_cnt[f] = dup ? 0 : min(d.pbcount[br], d.pcap);
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int run = 0;
-    for (int f = 0; f < 8; f++) {
-      const int c = s_cnt[f];
-      s_cnt[f] = run;
-      run += c;
-    }
-    s_cnt[8] = run;
-  }
-  __syncthreads();
-  const int total = s_cnt[8];
-  for (int base = 0; base < total; base += kStage) {
-    const int na = min(kStage, total - base);
-    int clip[3] = {0, 0, 0};
-    long long entry = 0;
-    bool reach = false;
-    if ((int)threadIdx.x < na) {
-      const int g = base + threadIdx.x;
-      int f = 0;
-      while (f < 7 && s_cnt[f + 1] <= g) f++;
-      entry = (long long)s_bin[f] * d.pcap + (g - s_cnt[f]);
-      const unsigned h = d.pbhdr[entry];
-#pragma unroll
-      for (int k = 0; k < 3; k++) {
-        // stencil start relative to the brick, in [0, K)
-        int r = (int)((h >> (10 * k)) & 1023u) - lo[k];
-        if (r < 0) r += d.K[k];
-        clip[k] = stencil_clip<N>(r, sz[k], d.K[k]);
-      }
-      reach = ((clip[0] >> 4) & 15) && ((clip[1] >> 4) & 15) && ((clip[2] >> 4) & 15);
-    }
-    // the atoms whose stencils reach the brick, compacted
-    int nreach;
-    const int a = block_scan256(reach ? 1 : 0, s_wsum, nreach);
-    int nrow = 0;
-    if (reach) {
-      const double *rec = d.pbrec + entry * pme_spline_rec_words(N);
-      s_lq[a] = rec[0];
-#pragma unroll
-      for (int k = 0; k < 3; k++) {
-#pragma unroll
-        for (int t = 0; t < N; t++) s_w[k][t][a] = rec[1 + k * N + t];
-        s_clip[k][a] = clip[k];
-      }
-      nrow = ((clip[0] >> 4) & 15) * ((clip[1] >> 4) & 15);
-    }
-    __syncthreads();   // s_wsum is reused by the second scan
-    int nrows;
-    const int off = block_scan256(nrow, s_wsum, nrows);
-    if (nrow) {
-      const int nx = (clip[0] >> 4) & 15, ny = (clip[1] >> 4) & 15;
-      int q = off;
-      for (int x = 0; x < nx; x++)
-        for (int y = 0; y < ny; y++) s_row[q++] = (unsigned short)(a | x << 8 | y << 11);
-    }
-    __syncthreads();
-    for (int it = threadIdx.x; it < nrows; it += blockDim.x) {
-      const unsigned e = s_row[it];
-      const int a = e & 255, x = (e >> 8) & 7, y = (e >> 11) & 7;
-      const int cx = s_clip[0][a], cy = s_clip[1][a], cz = s_clip[2][a];
-      int rx = (cx >> 8) + x;
-      if (rx >= d.K[0]) rx -= d.K[0];
-      int ry = (cy >> 8) + y;
-      if (ry >= d.K[1]) ry -= d.K[1];
-      const double wac = s_lq[a] * s_w[0][(cx & 15) + x][a] * s_w[1][(cy & 15) + y][a];
-      long long *row = acc + (rx * sz[1] + ry) * rowz;
-      const int tz = cz & 15, nz = (cz >> 4) & 15, pz0 = cz >> 8;
-#pragma unroll
-      for (int z = 0; z < N; z++) {
-        if (z < nz) {
-          int rz = pz0 + z;
-          if (rz >= d.K[2]) rz -= d.K[2];
-          // |lambda q w w w| <= |q| < 2^19: within fix_d_small's range
-          atomicAdd(reinterpret_cast<unsigned long long *>(row + rz),
-                    (unsigned long long)fix_d_small(wac * s_w[2][tz + z][a]));
-        }
-      }
-    }
-    __syncthreads();
-  }
-  for (int p = threadIdx.x; p < sz[0] * sz[1] * sz[2]; p += blockDim.x) {
-    const int pz = p % sz[2], pxy = p / sz[2];
-    const int py = pxy % sz[1], px = pxy / sz[1];
-    d.rgrid[((long long)(lo[0] + px) * d.K[1] + lo[1] + py) * d.K[2] + lo[2] + pz] =
-        (float)((double)acc[pxy * rowz + pz] * kFixInvD);
-  }
+  pme_bin_atom(d, i, i >= 0 ? d.spos[s] : make_uint4(0, 0, 0, 0));
 }
 
 template <int N>
 __global__ void __launch_bounds__(256) pme_spread(Dev d) {
-  pme_spread_body<N, spread_stage<N>()>(d, blockIdx.x, gridDim.x);
+  pme_spread_body<N>(d, blockIdx.x);
 }
 
 template <int N>
 __global__ void __launch_bounds__(256) pme_spread_multi(Multi m) {
   const MultiBlk b = multi_block(m);
   const Dev d = m.devs[b.sys];
-  pme_spread_body<N, spread_stage_multi<N>()>(d, b.bid, b.nblk);
+  pme_spread_body<N>(d, b.bid);
+}
+
+// The charge grid from the spread's bricks, a thread per point, for the
+// transforms whose first pass runs on few workgroups or holds its matrix in
+// registers (at 96^3 the MFMA plane kernel reading the bricks itself took
+// 155 us beside the pair kernel, 20 us from the grid); the compiled plane
+// kernels of small grids read the bricks directly.
+__device__ __forceinline__ void pme_sum_body(const Dev &d, int bid) {
+  const int g = bid * blockDim.x + threadIdx.x;
+  const int K1 = d.K[1], K2 = d.K[2];
+  if (g >= d.K[0] * K1 * K2) return;
+  const int z = g % K2, xy = g / K2, y = xy % K1, x = xy / K1;
+  const longlong2 *ay = d.paxis + d.K[0], *az = ay + K1;
+  d.rgrid[g] = pme_charge(d.pgrid, d.paxis[x], ay[y], az[z]);
+}
+
+__global__ void __launch_bounds__(256) pme_sum(Dev d) { pme_sum_body(d, blockIdx.x); }
+
+__global__ void __launch_bounds__(256) pme_sum_multi(Multi m) {
+  const MultiBlk b = multi_block(m);
+  const Dev d = m.devs[b.sys];
+  pme_sum_body(d, b.bid);
 }
 
 // ---------------------------------------------------------------------
@@ -646,7 +371,7 @@ __device__ __forceinline__ float2 *ct_fft(float2 *src, float2 *dst, const float2
 }
 
 // Forward transform along z then y of one x-plane (K1 x K2, in LDS): reads
-// the real charge grid, writes the complex grid.  1024 threads: there are
+// the spread's bricks, writes the complex grid.  1024 threads: there are
 // only K0 planes, so each plane's workgroup carries 16 waves.
 template <int K1, int K2>
 __device__ __forceinline__ void fft_yz_fwd_body(const Dev &d, int bid, int nblk) {
@@ -655,7 +380,10 @@ __device__ __forceinline__ void fft_yz_fwd_body(const Dev &d, int bid, int nblk)
   const long long base = (long long)bid * K1 * K2;
   for (int m = threadIdx.x; m < K1; m += blockDim.x) t1[m] = d.twiddle[d.K[0] + m];
   for (int m = threadIdx.x; m < K2; m += blockDim.x) t2[m] = d.twiddle[d.K[0] + K1 + m];
-  for (int e = threadIdx.x; e < K1 * K2; e += blockDim.x) b0[e] = make_float2(d.rgrid[base + e], 0.f);
+  const longlong2 ax = d.paxis[bid], *ay = d.paxis + d.K[0], *az = ay + K1;
+#pragma unroll 4
+  for (int e = threadIdx.x; e < K1 * K2; e += blockDim.x)
+    b0[e] = make_float2(pme_charge(d.pgrid, ax, ay[e / K2], az[e % K2]), 0.f);
   __syncthreads();
   float2 *r = ct_fft<K2, 1, K2, K1, 1, K2, false>(b0, b1, t2, -1.f);
   float2 *o = r == b0 ? b1 : b0;
@@ -937,8 +665,6 @@ static void make_plan(FftPlan &p, int K, const float2 *tw) {
   while (n % 5 == 0) { p.radix[p.nstage++] = 5; n /= 5; }
 }
 
-// (at most 1024 points per axis: the spread record header keeps 10 bits of
-// the first stencil point per axis)
 bool pme_grid_supported(int K) {
   if (K < 2 || K > kFftLds || K > 1024) return false;
   int n = K;
@@ -947,15 +673,9 @@ bool pme_grid_supported(int K) {
   return n == 1;
 }
 
-int grid_pme_bin(const Dev &d) { return (int)((32LL * d.maxblocks + 255) / 256); }
-
 int grid_pme_spread(const Dev &d) { return d.pnb[0] * d.pnb[1] * d.pnb[2]; }
 
-size_t lds_pme_spread(const Dev &d) {
-  int bmax = 1;
-  for (int k = 0; k < 3; k++) bmax *= (d.K[k] + d.pnb[k] - 1) / d.pnb[k] + (k == 2 ? 2 : 0);
-  return (size_t)bmax * sizeof(long long);
-}
+size_t lds_pme_spread(const Dev &d) { return (size_t)d.pvol * sizeof(long long); }
 
 // the three-kernel plane FFT applies (compiled size, square yz-plane in LDS)
 bool fft_plane_path(const Dev &d) {
@@ -970,7 +690,12 @@ int grid_fft_planes(const Dev &d) { return d.K[0]; }
 
 int grid_fft_x(const Dev &d) { return (d.K[1] * d.K[2] + 15) / 16; }
 
+int grid_pme_sum(const Dev &d) { return (d.K[0] * d.K[1] * d.K[2] + 255) / 256; }
+
+void launch_pme_sum_multi(const Multi &m, hipStream_t st) { pme_sum_multi<<<m.nwg, 256, 0, st>>>(m); }
+
 void launch_pme_fft(const Dev &d, bool energy, hipStream_t st) {
+  if (d.fft_mode == 1 || !fft_plane_path(d)) pme_sum<<<(unsigned)grid_pme_sum(d), 256, 0, st>>>(d);
   if (d.fft_mode == 1) {
     launch_pme_fft_mfma(d, energy, st);
     return;
@@ -1015,31 +740,22 @@ void launch_pme_fft(const Dev &d, bool energy, hipStream_t st) {
 }
 
 void launch_pme_grid(const Dev &d, bool energy, hipStream_t st) {
+  launch_pme_bin(d, st);
   launch_pme_spread(d, st);
   launch_pme_fft(d, energy, st);
+}
+
+void launch_pme_bin(const Dev &d, hipStream_t st) {
+  pme_bin<<<(unsigned)((32LL * d.maxblocks + 255) / 256), 256, 0, st>>>(d);
 }
 
 void launch_pme_spread(const Dev &d, hipStream_t st) {
   const int N = d.order;
   const unsigned nbr = (unsigned)grid_pme_spread(d);
   const size_t lds = lds_pme_spread(d);
-  const unsigned gb = (unsigned)grid_pme_bin(d);
-  if (N == 4) {
-    pme_bin<4><<<gb, 256, 0, st>>>(d);
-    pme_spread<4><<<nbr, 256, lds, st>>>(d);
-  } else if (N == 6) {
-    pme_bin<6><<<gb, 256, 0, st>>>(d);
-    pme_spread<6><<<nbr, 256, lds, st>>>(d);
-  } else {
-    pme_bin<8><<<gb, 256, 0, st>>>(d);
-    pme_spread<8><<<nbr, 256, lds, st>>>(d);
-  }
-}
-
-void launch_pme_bin_multi(const Multi &m, int order, hipStream_t st) {
-  if (order == 4) pme_bin_multi<4><<<m.nwg, 256, 0, st>>>(m);
-  else if (order == 6) pme_bin_multi<6><<<m.nwg, 256, 0, st>>>(m);
-  else pme_bin_multi<8><<<m.nwg, 256, 0, st>>>(m);
+  if (N == 4) pme_spread<4><<<nbr, 256, lds, st>>>(d);
+  else if (N == 6) pme_spread<6><<<nbr, 256, lds, st>>>(d);
+  else pme_spread<8><<<nbr, 256, lds, st>>>(d);
 }
 
 void launch_pme_spread_multi(const Multi &m, int order, size_t lds, hipStream_t st) {

@@ -94,11 +94,14 @@ double bspline_host(int n, double u) {
 
 }  // namespace
 
+// least atoms of a system whose PME transforms run on a branch of their own
+constexpr int kForkAtoms = 16000;
+
 struct bm_system {
   int device = 0;
   hipStream_t st = nullptr;
-  hipStream_t st2 = nullptr;         // PME branch of the force DAG (default priority)
-  hipStream_t st3 = nullptr;         // bonded / dU/dlambda branch (default priority)
+  hipStream_t st2 = nullptr;         // PME branch of a step (default priority)
+  hipStream_t st3 = nullptr;         // dU/dlambda branch (default priority)
   hipEvent_t evFork = nullptr, evJoin = nullptr, evJoin3 = nullptr;
   blade::Dev d{};
   int maxBlocks = 0;
@@ -155,30 +158,46 @@ struct bm_system {
     return BM_OK;
   }
 
-  // all force terms in three branches that only read positions: the pair
-  // kernel's chunk partials on the main stream, the PME chain (bins,
-  // spread, FFT and convolution) on st2, and the bonded slots with the
-  // FP64 dU/dlambda of the alchemical atoms on st3 (with the step's
-  // normals); then one per-atom assembly into the force array after all
-  // three (kick: the assembly also kicks the atoms of a non-energy step).
-  // Under stream capture the fork/join becomes three parallel graph
-  // branches.  The PME chain is a row of five dependent kernels, so the
-  // bonded work is kept off its stream.
-  void force_launches(bool energy, bool kick = false) {
-    (void)hipEventRecord(evFork, st);
-    (void)hipStreamWaitEvent(st2, evFork, 0);
-    (void)hipStreamWaitEvent(st3, evFork, 0);
-    blade::launch_nbdirect(d, energy, alch, soft, nwgNb, st);
-    if (d.elecmethod == BM_PME) blade::launch_pme_grid(d, energy, st2);
+  // The PME transforms run beside the pair kernel on a branch of their own
+  // when the pair kernel is long enough to hide them: a fork and join costs
+  // about 15 us of a step, and the launch of a graph with branches 50 us of
+  // host time against 17 us for a linear one of as many kernels, which a
+  // step of a small system cannot hide.  Measured around the line: see
+  // kForkAtoms.
+  bool forked() const { return d.elecmethod == BM_PME && d.n >= kForkAtoms; }
+
+  // all force terms: the spread, the bonded slots and the step's normals in
+  // one launch; the pair kernel's chunk partials; the PME transforms with
+  // the gather (on st2 where forked()) and the FP64 dU/dlambda of the
+  // alchemical atoms (on st3); then the per-atom assembly into the force array (kick:
+  // it also kicks the atoms of a non-energy step).  Under stream capture the
+  // fork and join become parallel graph branches.  binned: the step's pack
+  // has filled the PME bins.
+  void force_launches(bool energy, bool kick = false, bool binned = false) {
+    using namespace blade;
+    const bool pme = d.elecmethod == BM_PME, fork = forked();
+    if (pme && !binned) launch_pme_bin(d, st);
     // a non-energy step's O step runs after the assembly: its normals here
-    if (kick) blade::launch_normals(d, st3);
-    if (alch) blade::launch_nb_dudl(d, soft, st3);
-    blade::launch_bonded(d, energy, blade::kFamAll, st3);
-    (void)hipEventRecord(evJoin, st2);
-    (void)hipEventRecord(evJoin3, st3);
-    (void)hipStreamWaitEvent(st, evJoin, 0);
-    (void)hipStreamWaitEvent(st, evJoin3, 0);
-    blade::launch_force_assemble(d, blade::kAsmNb | blade::kAsmBonded | blade::kAsmPme, st, kick);
+    launch_side(d, energy, kick, st);
+    hipStream_t sp = st, sd = st;
+    if (fork) {
+      (void)hipEventRecord(evFork, st);
+      (void)hipStreamWaitEvent(sp = st2, evFork, 0);
+      if (alch) (void)hipStreamWaitEvent(sd = st3, evFork, 0);
+    }
+    launch_nbdirect(d, energy, alch, soft, nwgNb, st);
+    if (pme) launch_pme_fft(d, energy, sp);
+    if (fork) launch_force_assemble(d, kAsmPme, sp);
+    if (alch) launch_nb_dudl(d, soft, sd);
+    if (fork) {
+      (void)hipEventRecord(evJoin, st2);
+      (void)hipStreamWaitEvent(st, evJoin, 0);
+      if (alch) {
+        (void)hipEventRecord(evJoin3, st3);
+        (void)hipStreamWaitEvent(st, evJoin3, 0);
+      }
+    }
+    launch_force_assemble(d, kAsmNb | kAsmBonded | (fork ? 0u : kAsmPme), st, kick);
   }
 
   // a step: virtual sites placed (domdec/domdec.cu:215), lists, forces,
@@ -188,8 +207,8 @@ struct bm_system {
     const bool virt = d.nvirt2 + d.nvirt3 > 0;
     blade::launch_virtual_place(d, st);
     if (rebuild) blade::launch_domdec_rebuild(d, maxBlocks, st);
-    blade::launch_domdec_pack(d, maxBlocks, st);
-    force_launches(energy, !energy && !virt);
+    blade::launch_domdec_pack(d, maxBlocks, st, true);
+    force_launches(energy, !energy && !virt, true);
     blade::launch_virtual_spread(d, st);
     if (energy || virt) blade::launch_update(d, energy, st);
     else blade::launch_update_after_kick(d, st);
@@ -465,19 +484,62 @@ int bm_system_create(int device, const bm_topology *t, const bm_runparams *rp, c
     const size_t G = (size_t)d.K[0] * d.K[1] * d.K[2];
     ALLOC(d.rgrid, G);
     ALLOC(d.cgrid, G);
-    // spread bricks: floor(K/8) per axis (at least one), so each spans >= 8
-    // points (>= order-1 for orders up to 8, or the whole axis); a 64^3 grid
-    // gives 512 bricks, one workgroup each, all resident at once
-    int nbr = 1;
+    // Spread bricks, one workgroup each: about 8 points a side, which gives
+    // a 64^3 grid 512 workgroups; of small grids (fewer than 64 bricks)
+    // the least side a stencil allows, so that more CUs take part, and of
+    // large ones (over 1,024) 12 points, whose overhang is a smaller share.
+    // A brick spans >= order-1 points or its whole axis, so a grid point
+    // lies in its own brick and the overhang of the one before at most.
+    auto bricks = [&](int side) {
+      int nbr = 1;
+      for (int k = 0; k < 3; k++) {
+        int nb = std::max(1, (d.K[k] + side - 1) / side);
+        while (nb > 1 && d.K[k] / nb < d.order - 1) nb--;
+        d.pnb[k] = nb;
+        nbr *= nb;
+      }
+      return nbr;
+    };
+    int nbr = bricks(8);
+    if (nbr < 64) nbr = bricks(std::max(4, d.order - 1));
+    else if (nbr > 1024 && d.order <= 6) nbr = bricks(12);
+    d.pvol = 1;
     for (int k = 0; k < 3; k++) {
-      d.pnb[k] = std::max(1, d.K[k] / 8);
-      nbr *= d.pnb[k];
+      d.ppad[k] = (d.K[k] + d.pnb[k] - 1) / d.pnb[k] + d.order - 1;
+      if (k == 2) d.ppad[k] |= 1;   // rows of an odd number of words: neighbouring rows in different LDS banks
+      d.pvol *= d.ppad[k];
     }
     d.pcap = 64 + 4 * ((n + nbr - 1) / nbr);
     s->pcap0 = d.pcap;
     ALLOC(d.pbcount, nbr);
-    ALLOC(d.pbrec, (size_t)nbr * d.pcap * pme_spline_rec_words(d.order));
-    ALLOC(d.pbhdr, (size_t)nbr * d.pcap);
+    ALLOC(d.pbpos, (size_t)nbr * d.pcap);
+    ALLOC(d.pblq, (size_t)nbr * d.pcap);
+    ALLOC(d.pgrid, (size_t)nbr * d.pvol);
+    {
+      std::vector<longlong2> ax;
+      long long brick = d.pvol, point = 1;   // strides of a brick and of a point along the axis
+      long long bstr[3], pstr[3];
+      for (int k = 2; k >= 0; k--) {
+        bstr[k] = brick;
+        pstr[k] = point;
+        brick *= d.pnb[k];
+        point *= d.ppad[k];
+      }
+      for (int k = 0; k < 3; k++) {
+        const int K = d.K[k], nb = d.pnb[k];
+        auto lo = [&](int b) { return b * K / nb; };
+        for (int u = 0; u < K; u++) {
+          int b = u * nb / K;
+          if (b + 1 < nb && lo(b + 1) <= u) b++;
+          const int o = u - lo(b), p = b ? b - 1 : nb - 1, q = o + lo(p + 1) - lo(p);
+          longlong2 e;
+          e.x = b * bstr[k] + o * pstr[k];
+          e.y = o < d.order - 1 ? p * bstr[k] + q * pstr[k] : -1;
+          ax.push_back(e);
+        }
+      }
+      UPLOAD(d.paxis, ax);
+    }
     std::vector<float2> tw;
     for (int k = 0; k < 3; k++)
       for (int m = 0; m < d.K[k]; m++) {
@@ -1086,14 +1148,14 @@ static int set_tile_capacity(bm_system *s, long long maxTiles) {
   return BM_OK;
 }
 
-// PME brick bins of pcap spline records each (emptied)
+// PME brick bins of pcap atoms each (emptied)
 static int set_brick_capacity(bm_system *s, int pcap) {
   blade::Dev &d = s->d;
   if (d.elecmethod != BM_PME) return BM_OK;
   const size_t nbr = (size_t)d.pnb[0] * d.pnb[1] * d.pnb[2];
   d.pcap = pcap;
-  if (int rc = s->realloc_dev(d.pbrec, nbr * (size_t)pcap * blade::pme_spline_rec_words(d.order))) return rc;
-  if (int rc = s->realloc_dev(d.pbhdr, nbr * (size_t)pcap)) return rc;
+  if (int rc = s->realloc_dev(d.pbpos, nbr * (size_t)pcap)) return rc;
+  if (int rc = s->realloc_dev(d.pblq, nbr * (size_t)pcap)) return rc;
   HIPCHK(hipMemset(d.pbcount, 0, nbr * sizeof(int)));
   s->capacityGen++;
   s->drop_graphs();
@@ -1245,7 +1307,7 @@ struct bm_batch {
   hipGraph_t graphSrc[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
   // fused launches of a non-energy step
   MultiPlan pack, normals, bonded, tail;
-  std::vector<MultiPlan> bin, spread, fftp, fftx, mfp, mfx, nb, nbd, asmb;
+  std::vector<MultiPlan> spread, fftp, fftx, mfs, mfp, mfx, nb, nbd, asmb;
   MultiPlan rebuild[blade::kRebuildKernels];   // the list rebuild, one plan per kernel
   std::vector<int> fftSingle;      // PME members on neither fused FFT path (other sizes or shapes)
   std::vector<int> gens;           // members' capacity generations the launch plans were sized for
@@ -1273,7 +1335,7 @@ struct bm_batch {
   std::vector<MultiPlan *> plans() {
     std::vector<MultiPlan *> v = {&pack, &normals, &bonded, &tail};
     for (MultiPlan &p : rebuild) v.push_back(&p);
-    for (auto *g : {&bin, &spread, &fftp, &fftx, &mfp, &mfx, &nb, &nbd, &asmb})
+    for (auto *g : {&spread, &fftp, &fftx, &mfs, &mfp, &mfx, &nb, &nbd, &asmb})
       for (MultiPlan &p : *g) v.push_back(&p);
     return v;
   }
@@ -1300,34 +1362,36 @@ struct bm_batch {
       blade::launch_domdec_rebuild_multi(rm, lds, st);
     }
     blade::launch_pack_multi(pack.m, st);
+    // the spread, bonded terms and normals of every member in one launch
+    // (PME members of a second spline order: their spread in one of its own)
+    for (size_t g = 1; g < spread.size(); g++)
+      blade::launch_pme_spread_multi(spread[g].m, spread[g].order, spread[g].lds, st);
+    blade::launch_side_multi(spread.empty() ? nullptr : &spread[0].m, bonded.m, normals.m,
+                             spread.empty() ? 0 : spread[0].order, spread.empty() ? 0 : spread[0].lds, false, st);
     (void)hipEventRecord(fork2, st);
     // nbdirect first: the largest kernel takes the CUs before the second
     // stream's smaller ones fill them
     for (MultiPlan &p : nb) blade::launch_nbdirect_multi(p.m, p.elec, p.vdw, p.clusters, p.alch, p.soft, p.lds, st);
     (void)hipStreamWaitEvent(st2, fork2, 0);
-    (void)hipStreamWaitEvent(st3, fork2, 0);
-    // the FP64 dU/dlambda of the members' alchemical atoms, the normals and
-    // the bonded terms on the third stream, the PME chain on the second
-    for (MultiPlan &p : nbd) blade::launch_nb_dudl_multi(p.m, p.elec, p.vdw, p.soft, st3);
-    blade::launch_normals_multi(normals.m, st3);
-    blade::launch_bonded_multi(bonded.m, false, st3);
-    (void)hipEventRecord(join3, st3);
-    for (size_t g = 0; g < bin.size(); g++) {
-      blade::launch_pme_bin_multi(bin[g].m, bin[g].order, st2);
-      blade::launch_pme_spread_multi(spread[g].m, spread[g].order, spread[g].lds, st2);
-    }
     // FFT groups in turn on st2 (one stream per branch: the process has
-    // four hardware queues)
+    // four hardware queues) and the gather; the FP64 dU/dlambda of the
+    // members' alchemical atoms on a third
+    if (!nbd.empty()) (void)hipStreamWaitEvent(st3, fork2, 0);
+    for (MultiPlan &p : nbd) blade::launch_nb_dudl_multi(p.m, p.elec, p.vdw, p.soft, st3);
+    if (!nbd.empty()) (void)hipEventRecord(join3, st3);
     for (size_t g = 0; g < fftp.size(); g++)
       blade::launch_pme_fft_multi(fftp[g].m, fftx[g].m, fftp[g].K0, fftp[g].K1, false, st2);
+    for (MultiPlan &p : mfs) blade::launch_pme_sum_multi(p.m, st2);
     for (size_t g = 0; g < mfp.size(); g++)
       blade::launch_pme_fft_mfma_multi(mfp[g].m, mfx[g].m, mfp[g].K0, mfp[g].K1, false, st2);
     for (int k : fftSingle) blade::launch_pme_fft(sys[k]->d, false, st2);
+    for (MultiPlan &p : asmb)
+      if (p.order) blade::launch_assemble_multi(p.m, p.order, blade::kAsmPme, false, st2);
     (void)hipEventRecord(join2, st2);
     (void)hipStreamWaitEvent(st, join2, 0);
-    (void)hipStreamWaitEvent(st, join3, 0);
+    if (!nbd.empty()) (void)hipStreamWaitEvent(st, join3, 0);
     for (MultiPlan &p : asmb)
-      blade::launch_assemble_multi(p.m, p.order, blade::kAsmNb | blade::kAsmBonded | blade::kAsmPme, true, st);
+      blade::launch_assemble_multi(p.m, 0, blade::kAsmNb | blade::kAsmBonded, true, st);
     blade::launch_tail_multi(tail.m, st);
   }
 };
@@ -1389,11 +1453,10 @@ static int build_plans(bm_batch *b) {
     if ((rc = make_plan(b, b->rebuild[r], all, [r](const Dev &d) { return blade::grid_rebuild(d, r); }))) return rc;
     for (int k : all) b->rebuild[r].lds = std::max(b->rebuild[r].lds, blade::lds_rebuild(D(k), r));
   }
-  if ((rc = make_groups(b, b->bin, pme, [&](int k) { return D(k).order; }, blade::grid_pme_bin))) return rc;
   if ((rc = make_groups(b, b->spread, pme, [&](int k) { return D(k).order; }, blade::grid_pme_spread))) return rc;
-  for (size_t g = 0; g < b->bin.size(); g++) {
-    b->bin[g].order = b->spread[g].order = D(b->bin[g].members[0]).order;
-    for (int k : b->spread[g].members) b->spread[g].lds = std::max(b->spread[g].lds, blade::lds_pme_spread(D(k)));
+  for (MultiPlan &p : b->spread) {
+    p.order = D(p.members[0]).order;
+    for (int k : p.members) p.lds = std::max(p.lds, blade::lds_pme_spread(D(k)));
   }
   auto fkey = [&](int k) { return std::make_pair(D(k).K[0], D(k).K[1]); };
   if ((rc = make_groups(b, b->fftp, plane, fkey, blade::grid_fft_planes))) return rc;
@@ -1402,6 +1465,7 @@ static int build_plans(bm_batch *b) {
     b->fftp[g].K0 = D(b->fftp[g].members[0]).K[0];
     b->fftp[g].K1 = D(b->fftp[g].members[0]).K[1];
   }
+  if ((rc = make_groups(b, b->mfs, mplane, [](int) { return 0; }, blade::grid_pme_sum))) return rc;
   if ((rc = make_groups(b, b->mfp, mplane, fkey, blade::grid_fft_mfma_planes))) return rc;
   if ((rc = make_groups(b, b->mfx, mplane, fkey, blade::grid_fft_mfma_x))) return rc;
   for (size_t g = 0; g < b->mfp.size(); g++) {
@@ -1788,6 +1852,7 @@ int bm_time_pme(bm_system *s, int reps, double *out) {
   double t[3] = {0, 0, 0};
   for (int r = 0; r < reps; r++) {
     HIPCHK(hipEventRecord(s->ev[0], s->st));
+    blade::launch_pme_bin(s->d, s->st);
     blade::launch_pme_spread(s->d, s->st);
     HIPCHK(hipEventRecord(s->ev[1], s->st));
     blade::launch_pme_fft(s->d, false, s->st);

@@ -13,6 +13,7 @@
 // Energy steps split the kick: V, RATTLE velocity projection, kinetic
 // energy, V+R (update.cu:257-279).
 #include "kernels.h"
+#include "normals.h"
 
 // No contraction of separate multiplies and adds into fused ones in this
 // file: every FP64 expression rounds as written, so the constraint solves
@@ -40,36 +41,7 @@ __device__ __forceinline__ D3 minimg(const Dev &d, D3 v) {
   return d3(wrapd(v.x, d.box[0], d.invbox[0]), wrapd(v.y, d.box[1], d.invbox[1]), wrapd(v.z, d.box[2], d.invbox[2]));
 }
 
-// standard normals of DOFs 2p and 2p+1 for (seed, step): the same rule as
-// the oracle (one Philox block, Box-Muller cosine for the even DOF, sine for
-// the odd one)
-__device__ double2 normal_pair(unsigned long long seed, unsigned long long step, unsigned long long p) {
-  uint4 c = make_uint4((unsigned)p, (unsigned)step, (unsigned)(step >> 32), 0x4E524D4Cu);
-  uint4 o = philox(c, make_uint2((unsigned)seed, (unsigned)(seed >> 32)));
-  double u1 = ((double)((((unsigned long long)o.x) << 21) ^ (o.y >> 11)) + 0.5) * (1.0 / 9007199254740992.0);
-  double u2 = ((double)((((unsigned long long)o.z) << 21) ^ (o.w >> 11)) + 0.5) * (1.0 / 9007199254740992.0);
-  double rad = sqrt(-2.0 * log(u1));
-  double sn, cs;
-  sincospi(2.0 * u2, &sn, &cs);
-  return make_double2(rad * cs, rad * sn);
-}
-
-__device__ __forceinline__ void upd_normals_body(const Dev &d, int bid) {
-  const int p = bid * blockDim.x + threadIdx.x;
-  const int N = 3 * d.n + d.nl;
-  if (2 * p >= N) return;
-  const double2 z = normal_pair(d.seed, (unsigned long long)(*d.step), (unsigned long long)p);
-  d.xi[2 * p] = z.x;
-  if (2 * p + 1 < N) d.xi[2 * p + 1] = z.y;
-}
-
 __global__ void __launch_bounds__(256) upd_normals(Dev d) { upd_normals_body(d, blockIdx.x); }
-
-__global__ void __launch_bounds__(256) upd_normals_multi(Multi m) {
-  const MultiBlk b = multi_block(m);
-  const Dev d = m.devs[b.sys];
-  upd_normals_body(d, b.bid);
-}
 
 // dU/dtheta of block b: the theta biases plus the chain rule from the
 // fixed-point dU/dlambda (msld.cu:937-998).  Softmax: lambda_b fnex cos
@@ -698,8 +670,6 @@ void launch_update_after_kick(const Dev &d, hipStream_t st) { upd_tail<<<grid_ta
 void launch_normals(const Dev &d, hipStream_t st) { upd_normals<<<grid_normals(d), 256, 0, st>>>(d); }
 
 void launch_tail_multi(const Multi &m, hipStream_t st) { upd_tail_multi<<<m.nwg, 64, 0, st>>>(m); }
-
-void launch_normals_multi(const Multi &m, hipStream_t st) { upd_normals_multi<<<m.nwg, 256, 0, st>>>(m); }
 
 __global__ void upd_set_step(Dev d, long long v) { *d.step = v; }
 
