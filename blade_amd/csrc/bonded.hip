@@ -816,7 +816,7 @@ __global__ void __launch_bounds__(256) side_kernel(Dev d, BondedLaunch L, bool e
 // the same over several systems; the spread's plan holds the PME members of
 // spline order N
 template <int N>
-__global__ void __launch_bounds__(256) side_multi(Multi ms, Multi mb, Multi mn, bool energy) {
+__global__ void __launch_bounds__(256, 3) side_multi(Multi ms, Multi mb, Multi mn, bool energy) {
   int b = blockIdx.x;
   if constexpr (N > 0) {
     if (b < ms.nwg) {

@@ -319,8 +319,8 @@ static size_t lds_tile_write(const Dev &d) { return (size_t)4 * dd_row_words(d.m
 // outgrows its buffers), the row's tiles in ascending J and its chunks, then
 // the exclusions of the row's atoms: tiles holding one get 32 mask words
 // (bit j of word i: slots (I,i) and (J,j) are excluded), numbered by a claim
-// on the number of such tiles, -1 in tile_ex for the others.  Lane l makes
-// word l of every mask of its row, so no other thread writes it.
+// on the number of such tiles, -1 in tile_ex for the others.  No other wave
+// touches the masks of the row.
 __device__ __forceinline__ void dd_tile_write_body(const Dev &d, int bid) {
   if (halted_wg(d)) return;   // a halted step leaves the list as it is
   __shared__ unsigned s_lo[3 * kBoxLds], s_hi[3 * kBoxLds];
@@ -404,11 +404,25 @@ __device__ __forceinline__ void dd_tile_write_body(const Dev &d, int bid) {
     const unsigned long long m = bits[J >> 6], bit = 1ull << (J & 63);
     return m & bit ? pre[J >> 6] + __popcll(m & (bit - 1)) : -1;
   };
-  const int a = lane < kBlockAtoms ? d.l2g[I * kBlockAtoms + lane] : -1;
-  const int x0 = a >= 0 ? d.exstart[a] : 0, x1 = a >= 0 ? d.exstart[a + 1] : 0;
-  for (int x = x0; x < x1; x++) {
-    const int q = place(d.g2s[d.exadj[x]] / kBlockAtoms);
-    if (q >= 0) atomicOr(&ebits[q >> 6], 1ull << (q & 63));
+  // two lanes to a slot, on alternate exclusions, eight loads in flight each
+  // (an atom of a chain has a dozen or more, each behind two dependent loads)
+  const int l = lane & (kBlockAtoms - 1), a = d.l2g[I * kBlockAtoms + l];
+  const int x0 = a >= 0 ? d.exstart[a] + (lane >> 5) : 0, x1 = a >= 0 ? d.exstart[a + 1] : 0;
+  constexpr int kExBatch = 8;
+  auto partners = [&](int x, int (&sb)[kExBatch]) {
+#pragma unroll
+    for (int k = 0; k < kExBatch; k++) sb[k] = x + 2 * k < x1 ? d.exadj[x + 2 * k] : a;
+#pragma unroll
+    for (int k = 0; k < kExBatch; k++) sb[k] = d.g2s[sb[k]];
+  };
+  for (int x = x0; x < x1; x += 2 * kExBatch) {
+    int sb[kExBatch];
+    partners(x, sb);
+#pragma unroll
+    for (int k = 0; k < kExBatch; k++) {
+      const int q = x + 2 * k < x1 ? place(sb[k] / kBlockAtoms) : -1;
+      if (q >= 0) atomicOr(&ebits[q >> 6], 1ull << (q & 63));
+    }
   }
   dd_wave_sync();
   const int tw = (cnt + 63) / 64;   // words of ebits in use
@@ -424,15 +438,19 @@ __device__ __forceinline__ void dd_tile_write_body(const Dev &d, int bid) {
     if (t < cnt) d.tile_ex[before + t] = (m >> lane) & 1ull ? e0 + __popcll(m & below) : -1;
     e0 += __popcll(m);
   }
-  if (lane < kBlockAtoms)
-    for (int k = 0; k < flagged; k++) d.emask[(long long)(base + k) * kBlockAtoms + lane] = 0u;
-  for (int x = x0; x < x1; x++) {
-    const int sb = d.g2s[d.exadj[x]];
-    const int q = place(sb / kBlockAtoms);
-    if (q < 0) continue;
-    int e = base + __popcll(ebits[q >> 6] & ((1ull << (q & 63)) - 1));
-    for (int k = 0; k < q >> 6; k++) e += __popcll(ebits[k]);
-    atomicOr(&d.emask[(long long)e * kBlockAtoms + lane], 1u << (sb % kBlockAtoms));
+  for (int k = lane; k < flagged * kBlockAtoms; k += 64) d.emask[(long long)base * kBlockAtoms + k] = 0u;
+  __threadfence();   // the cleared words are in place before any lane sets bits in them
+  for (int x = x0; x < x1; x += 2 * kExBatch) {
+    int sb[kExBatch];
+    partners(x, sb);
+#pragma unroll
+    for (int k = 0; k < kExBatch; k++) {
+      const int q = x + 2 * k < x1 ? place(sb[k] / kBlockAtoms) : -1;
+      if (q < 0) continue;
+      int e = base + __popcll(ebits[q >> 6] & ((1ull << (q & 63)) - 1));
+      for (int i = 0; i < q >> 6; i++) e += __popcll(ebits[i]);
+      atomicOr(&d.emask[(long long)e * kBlockAtoms + l], 1u << (sb[k] % kBlockAtoms));
+    }
   }
 }
 __global__ void __launch_bounds__(256) dd_tile_write(Dev d) { dd_tile_write_body(d, blockIdx.x); }
