@@ -114,6 +114,11 @@ struct bm_system {
   int freqDomdec = 10;
   double kT = 0.0;                   // kB T of the thermostat (replica exchange)
   std::vector<void *> allocs;
+  // pinned staging of host transfers (a copy from or to pageable memory goes
+  // through a buffer of the runtime's, several times slower to start);
+  // every transfer is waited for before the call that starts it returns
+  double *stage = nullptr;
+  size_t stageBytes = 0;
   hipGraphExec_t graph[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
   hipGraph_t graphSrc[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
   hipEvent_t ev[8] = {};
@@ -335,6 +340,9 @@ int bm_system_create(int device, const bm_topology *t, const bm_runparams *rp, c
 #define UPLOAD(p, v) \
   if ((rc = s->upload(p, v))) return fail(rc)
   const size_t N = 3 * (size_t)n + nl;
+  s->stageBytes = N * sizeof(double);
+  if (hipHostMalloc(reinterpret_cast<void **>(&s->stage), s->stageBytes, hipHostMallocDefault) != hipSuccess)
+    return fail(set_err(BM_EHIP, "pinned staging"));
   // state
   {
     std::vector<double> x(N, 0.0), v(N, 0.0), ism(N, 0.0);
@@ -371,8 +379,10 @@ int bm_system_create(int device, const bm_topology *t, const bm_runparams *rp, c
     std::vector<float> lamf(nl, 1.0f);
     for (int b = 0; b < nl; b++) lamf[b] = (float)lam[b];
     UPLOAD(d.lambdaf, lamf);
-    std::vector<int> nf(1, -1);
-    UPLOAD(d.nanflag, nf);
+    // the error flag and the NaN flag side by side: one copy reads both
+    std::vector<int> fl = {0, -1};
+    UPLOAD(d.errflag, fl);
+    d.nanflag = d.errflag + 1;
     std::vector<long long> st0(1, 0);
     UPLOAD(d.step, st0);
   }
@@ -476,7 +486,6 @@ int bm_system_create(int device, const bm_topology *t, const bm_runparams *rp, c
     UPLOAD(d.exadj, adj);
   }
   ALLOC(d.workctr, 4);
-  ALLOC(d.errflag, 1);
   // PME
   if (rp->elec_method == BM_PME) {
     for (int k = 0; k < 3; k++) d.K[k] = rp->grid[k];
@@ -979,12 +988,18 @@ int bm_system_destroy(bm_system *s) {
   return BM_OK;
 }
 
-int bm_sync(bm_system *s) {
-  if (!s) return BM_EINVAL;
+// wait for the stream and read the error and NaN flags
+static int read_flags(bm_system *s, int &flag, int &nan) {
+  int *h = reinterpret_cast<int *>(s->stage);
+  HIPCHK(hipMemcpyAsync(h, s->d.errflag, 2 * sizeof(int), hipMemcpyDeviceToHost, s->st));
   HIPCHK(hipStreamSynchronize(s->st));
-  int flag = 0, nan = -1;
-  HIPCHK(hipMemcpy(&flag, s->d.errflag, sizeof(int), hipMemcpyDeviceToHost));
-  HIPCHK(hipMemcpy(&nan, s->d.nanflag, sizeof(int), hipMemcpyDeviceToHost));
+  flag = h[0];
+  nan = h[1];
+  return BM_OK;
+}
+
+// BM_OK, or the error of the flags read_flags gave
+static int flags_error(int flag, int nan) {
   if (!flag && nan < 0) return BM_OK;
   // every condition that was raised, the first non-finite value first (a
   // blow-up also scatters atoms into one column)
@@ -995,6 +1010,13 @@ int bm_sync(bm_system *s) {
   if (flag & 1) msg += "a domdec column exceeded its capacity; ";
   msg.resize(msg.size() - 2);
   return set_err(nan >= 0 ? BM_ENAN : BM_EOVERFLOW, msg.c_str());
+}
+
+int bm_sync(bm_system *s) {
+  if (!s) return BM_EINVAL;
+  int flag = 0, nan = -1;
+  if (int rc = read_flags(s, flag, nan)) return rc;
+  return flags_error(flag, nan);
 }
 
 int bm_domdec_update(bm_system *s, int rebuild) {
@@ -1264,18 +1286,15 @@ int bm_dynamics(bm_system *s, long step0, long nsteps, int freq_nrg, int use_gra
     if (int rc = dynamics_launches(s, step0, end - step0, freq_nrg, use_graph)) return rc;
     // one synchronisation per call: a capacity overflow halted the state
     // at the step that raised it; grow the buffer and run from that step
-    HIPCHK(hipStreamSynchronize(s->st));
     int flag = 0, nan = -1;
-    HIPCHK(hipMemcpy(&flag, s->d.errflag, sizeof(int), hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(&nan, s->d.nanflag, sizeof(int), hipMemcpyDeviceToHost));
-    if (!flag || nan >= 0) break;
+    if (int rc = read_flags(s, flag, nan)) return rc;
+    if (!flag || nan >= 0) return flags_error(flag, nan);
     long long at = 0;
     HIPCHK(hipMemcpy(&at, s->d.step, sizeof(long long), hipMemcpyDeviceToHost));
-    if (at < step0 || at >= end) break;
-    if (regrow(s, flag)) break;
+    if (at < step0 || at >= end) return flags_error(flag, nan);
+    if (regrow(s, flag)) return flags_error(flag, nan);
     step0 = (long)at;
   }
-  return bm_sync(s);
 }
 
 // ---------------------------------------------------------------------
@@ -1920,20 +1939,51 @@ int bm_calibration_copy(int device, size_t bytes, int reps, double *out) {
   return rc;
 }
 
+// bytes (at most stageBytes) of device memory into the staging, and wait
+static int d2stage(bm_system *s, const void *src, size_t bytes) {
+  HIPCHK(hipMemcpyAsync(s->stage, src, bytes, hipMemcpyDeviceToHost, s->st));
+  HIPCHK(hipStreamSynchronize(s->st));
+  return BM_OK;
+}
+
 static int d2h(bm_system *s, void *dst, const void *src, size_t bytes) {
+  if (bytes <= s->stageBytes) {
+    if (int rc = d2stage(s, src, bytes)) return rc;
+    std::memcpy(dst, s->stage, bytes);
+    return BM_OK;
+  }
   HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s->st));
+  HIPCHK(hipStreamSynchronize(s->st));
+  return BM_OK;
+}
+
+// a state array [x|y|z|theta] of the device to the host's two arrays
+static int get_state(bm_system *s, const double *src, double *atoms, double *theta) {
+  const size_t n3 = 3 * (size_t)s->d.n;
+  if (int rc = d2stage(s, src, (n3 + s->d.nl) * sizeof(double))) return rc;
+  if (atoms) std::memcpy(atoms, s->stage, n3 * sizeof(double));
+  if (theta) std::memcpy(theta, s->stage + n3, s->d.nl * sizeof(double));
+  return BM_OK;
+}
+
+// and back (either may be null)
+static int set_state(bm_system *s, double *dst, const double *atoms, const double *theta) {
+  const size_t n3 = 3 * (size_t)s->d.n;
+  if (atoms) {
+    std::memcpy(s->stage, atoms, n3 * sizeof(double));
+    HIPCHK(hipMemcpyAsync(dst, s->stage, n3 * sizeof(double), hipMemcpyHostToDevice, s->st));
+  }
+  if (theta) {
+    std::memcpy(s->stage + n3, theta, s->d.nl * sizeof(double));
+    HIPCHK(hipMemcpyAsync(dst + n3, s->stage + n3, s->d.nl * sizeof(double), hipMemcpyHostToDevice, s->st));
+  }
   HIPCHK(hipStreamSynchronize(s->st));
   return BM_OK;
 }
 
 int bm_get_positions(bm_system *s, double *pos, double *theta) {
   if (!s) return BM_EINVAL;
-  const int n = s->d.n;
-  std::vector<double> x(3 * (size_t)n + s->d.nl);
-  if (int rc = d2h(s, x.data(), s->d.pos, x.size() * sizeof(double))) return rc;
-  if (pos) std::memcpy(pos, x.data(), 3 * (size_t)n * sizeof(double));
-  if (theta) std::memcpy(theta, x.data() + 3 * (size_t)n, s->d.nl * sizeof(double));
-  return BM_OK;
+  return get_state(s, s->d.pos, pos, theta);
 }
 
 // the box-dependent members of the device system, as bm_system_create sets
@@ -1988,46 +2038,33 @@ int bm_get_box(bm_system *s, double *box) {
 
 int bm_set_positions(bm_system *s, const double *pos, const double *theta) {
   if (!s) return BM_EINVAL;
-  const int n = s->d.n;
-  if (pos) HIPCHK(hipMemcpyAsync(s->d.pos, pos, 3 * (size_t)n * sizeof(double), hipMemcpyHostToDevice, s->st));
-  if (theta) {
-    HIPCHK(hipMemcpyAsync(s->d.pos + 3 * (size_t)n, theta, s->d.nl * sizeof(double), hipMemcpyHostToDevice, s->st));
-    if (s->alch) blade::launch_theta_to_lambda(s->d, s->st, true);
+  if (int rc = set_state(s, s->d.pos, pos, theta)) return rc;
+  if (theta && s->alch) {
+    blade::launch_theta_to_lambda(s->d, s->st, true);
+    HIPCHK(hipStreamSynchronize(s->st));
   }
-  HIPCHK(hipStreamSynchronize(s->st));
   return BM_OK;
 }
 
 int bm_set_velocities(bm_system *s, const double *vel, const double *theta_vel) {
   if (!s) return BM_EINVAL;
-  const int n = s->d.n;
-  if (vel) HIPCHK(hipMemcpyAsync(s->d.vel, vel, 3 * (size_t)n * sizeof(double), hipMemcpyHostToDevice, s->st));
-  if (theta_vel)
-    HIPCHK(hipMemcpyAsync(s->d.vel + 3 * (size_t)n, theta_vel, s->d.nl * sizeof(double), hipMemcpyHostToDevice,
-                          s->st));
-  HIPCHK(hipStreamSynchronize(s->st));
-  return BM_OK;
+  return set_state(s, s->d.vel, vel, theta_vel);
 }
 
 int bm_get_velocities(bm_system *s, double *vel, double *theta_vel) {
   if (!s) return BM_EINVAL;
-  const int n = s->d.n;
-  std::vector<double> v(3 * (size_t)n + s->d.nl);
-  if (int rc = d2h(s, v.data(), s->d.vel, v.size() * sizeof(double))) return rc;
-  if (vel) std::memcpy(vel, v.data(), 3 * (size_t)n * sizeof(double));
-  if (theta_vel) std::memcpy(theta_vel, v.data() + 3 * (size_t)n, s->d.nl * sizeof(double));
-  return BM_OK;
+  return get_state(s, s->d.vel, vel, theta_vel);
 }
 
 int bm_get_forces(bm_system *s, double *force, double *theta_force) {
   if (!s) return BM_EINVAL;
-  const int n = s->d.n;
-  std::vector<long long> f(3 * (size_t)n + s->d.nl);
-  if (int rc = d2h(s, f.data(), s->d.force, f.size() * sizeof(long long))) return rc;
+  const size_t n3 = 3 * (size_t)s->d.n;
+  if (int rc = d2stage(s, s->d.force, (n3 + s->d.nl) * sizeof(long long))) return rc;
+  const long long *f = reinterpret_cast<const long long *>(s->stage);
   if (force)
-    for (size_t i = 0; i < 3 * (size_t)n; i++) force[i] = (double)f[i] * blade::kFixInvD;
+    for (size_t i = 0; i < n3; i++) force[i] = (double)f[i] * blade::kFixInvD;
   if (theta_force)
-    for (int b = 0; b < s->d.nl; b++) theta_force[b] = (double)f[3 * (size_t)n + b] * blade::kFixInvD;
+    for (int b = 0; b < s->d.nl; b++) theta_force[b] = (double)f[n3 + b] * blade::kFixInvD;
   return BM_OK;
 }
 
