@@ -401,14 +401,17 @@ void launch_pme_fft_mfma_multi(const Multi &mp, const Multi &mx, int K0, int K1,
   }
 }
 
-void launch_pme_fft_mfma(const Dev &d, bool energy, hipStream_t st) {
+void launch_pme_fft_mfma(const Dev &d, bool energy, hipStream_t st, int part) {
   const int K0 = d.K[0], K1 = d.K[1], K2 = d.K[2];
   const bool planes = K1 == K2;
-  if (planes) yz_t<false>(d, st);
-  else {
-    pass_t<2, 0>(d, K0 * K1, st);
-    pass_t<1, 1>(d, K0 * K2, st);
+  if (part != kFftTail) {
+    if (planes) yz_t<false>(d, st);
+    else {
+      pass_t<2, 0>(d, K0 * K1, st);
+      pass_t<1, 1>(d, K0 * K2, st);
+    }
   }
+  if (part == kFftHead) return;
   const unsigned gx = (unsigned)(K1 * K2 / 32);
   switch (K0) {
 #define BM_X(SZ) \

@@ -55,8 +55,11 @@ void launch_set_step(const Dev &d, long long step, hipStream_t st);
 // the bins and the spread of launch_pme_grid alone
 void launch_pme_bin(const Dev &d, hipStream_t st);
 void launch_pme_spread(const Dev &d, hipStream_t st);
-// the FFT part of launch_pme_grid alone
-void launch_pme_fft(const Dev &d, bool energy, hipStream_t st);
+// the FFT part of launch_pme_grid alone, or its first (kFftHead: of the MFMA
+// form the charge grid and the forward y-z transforms, of other forms what
+// precedes their first transform) or remaining kernels (kFftTail)
+constexpr int kFftAll = 0, kFftHead = 1, kFftTail = 2;
+void launch_pme_fft(const Dev &d, bool energy, hipStream_t st, int part = kFftAll);
 // the MFMA split-BF16x3 form of it (every grid edge fft_mfma_supported)
 bool fft_mfma_supported(int K);
 // the charge grids of several members from their spread's bricks
@@ -67,7 +70,7 @@ void launch_pme_sum_multi(const Multi &m, hipStream_t st);
 int grid_fft_mfma_planes(const Dev &d);
 int grid_fft_mfma_x(const Dev &d);
 void launch_pme_fft_mfma_multi(const Multi &mp, const Multi &mx, int K0, int K1, bool energy, hipStream_t st);
-void launch_pme_fft_mfma(const Dev &d, bool energy, hipStream_t st);
+void launch_pme_fft_mfma(const Dev &d, bool energy, hipStream_t st, int part);
 
 // ---- several systems per launch (Multi, device.h) ----------------------
 // Workgroups one system needs per kernel type; the single-system launches

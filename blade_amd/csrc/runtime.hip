@@ -94,6 +94,72 @@ double bspline_host(int n, double u) {
 
 }  // namespace
 
+// Step graphs: one per (rebuild, energy) variant of a step, and runs of 8, 4
+// and 2 plain steps (neither).  Between two graph launches the GPU idles 5
+// to 12 us, between two steps of one graph 1 to 2, so a run of plain steps
+// is launched in as few graphs as it divides into.
+struct StepGraphs {
+  static constexpr int kRuns = 3;
+  static constexpr int run_steps(int r) { return 8 >> r; }
+  hipGraphExec_t exec[4 + kRuns] = {};
+  hipGraph_t src[4 + kRuns] = {};
+
+  void drop() {
+    for (int k = 0; k < 4 + kRuns; k++) {
+      if (exec[k]) (void)hipGraphExecDestroy(exec[k]);
+      if (src[k]) (void)hipGraphDestroy(src[k]);
+      exec[k] = nullptr;
+      src[k] = nullptr;
+    }
+  }
+  // capture and instantiate graph k (2 rebuild + energy, or 4 + run); step(rb,
+  // en) issues the launches of a step on st
+  template <class F>
+  int capture(int k, hipStream_t st, F step) {
+    if (exec[k]) return BM_OK;
+    HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+    int rc = BM_OK;
+    for (int i = 0; !rc && i < (k < 4 ? 1 : run_steps(k - 4)); i++) rc = k < 4 ? step(k >> 1, k & 1) : step(0, 0);
+    hipGraph_t g = nullptr;
+    const hipError_t e = hipStreamEndCapture(st, &g);
+    if (rc) {
+      if (g) (void)hipGraphDestroy(g);
+      return rc;
+    }
+    HIPCHK(e);
+    src[k] = g;
+    HIPCHK(hipGraphInstantiate(&exec[k], g, nullptr, nullptr, 0));
+    return BM_OK;
+  }
+  template <class F>
+  int capture_all(hipStream_t st, F step) {
+    for (int k = 0; k < 4 + kRuns; k++)
+      if (int rc = capture(k, st, step)) return rc;
+    return BM_OK;
+  }
+  // steps [step0, step0 + nsteps), lists rebuilt at multiples of freqDomdec
+  // and energies at multiples of freqNrg
+  template <class F>
+  int play(long step0, long nsteps, long freqDomdec, long freqNrg, hipStream_t st, F step) {
+    for (long at = step0, end = step0 + nsteps; at < end;) {
+      const int rb = (at % freqDomdec) == 0, en = (at % freqNrg) == 0;
+      int k = 2 * rb + en, len = 1;
+      if (!rb && !en) {
+        const long plain = std::min({end - at, freqDomdec - at % freqDomdec, freqNrg - at % freqNrg});
+        for (int r = kRuns - 1; r >= 0; r--)
+          if (run_steps(r) <= plain) {
+            k = 4 + r;
+            len = run_steps(r);
+          }
+      }
+      if (int rc = capture(k, st, step)) return rc;
+      HIPCHK(hipGraphLaunch(exec[k], st));
+      at += len;
+    }
+    return BM_OK;
+  }
+};
+
 // least atoms of a system whose PME transforms run on a branch of their own
 constexpr int kForkAtoms = 16000;
 
@@ -119,8 +185,7 @@ struct bm_system {
   // every transfer is waited for before the call that starts it returns
   double *stage = nullptr;
   size_t stageBytes = 0;
-  hipGraphExec_t graph[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
-  hipGraph_t graphSrc[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
+  StepGraphs graphs;
   hipEvent_t ev[8] = {};
   double msNb = 0, msPme = 0, msTotal = 0;
   long nMeas = 0;
@@ -146,15 +211,7 @@ struct bm_system {
     }
     return alloc(p, count);
   }
-  void drop_graphs() {
-    for (int a = 0; a < 2; a++)
-      for (int b = 0; b < 2; b++) {
-        if (graph[a][b]) (void)hipGraphExecDestroy(graph[a][b]);
-        if (graphSrc[a][b]) (void)hipGraphDestroy(graphSrc[a][b]);
-        graph[a][b] = nullptr;
-        graphSrc[a][b] = nullptr;
-      }
-  }
+  void drop_graphs() { graphs.drop(); }
   template <class T>
   int upload(T *&p, const std::vector<T> &v) {
     int rc = alloc(p, v.size());
@@ -184,6 +241,11 @@ struct bm_system {
     if (pme && !binned) launch_pme_bin(d, st);
     // a non-energy step's O step runs after the assembly: its normals here
     launch_side(d, energy, kick, st);
+    // The MFMA transforms of a plane hold a CU's whole register file: beside
+    // the pair kernel they wait for CUs to empty (the forward planes 136 us
+    // at 96^3, alone 20), so the first half runs before it.
+    const bool head = pme && fork && d.fft_mode == 1;
+    if (head) launch_pme_fft(d, energy, st, kFftHead);
     hipStream_t sp = st, sd = st;
     if (fork) {
       (void)hipEventRecord(evFork, st);
@@ -191,7 +253,7 @@ struct bm_system {
       if (alch) (void)hipStreamWaitEvent(sd = st3, evFork, 0);
     }
     launch_nbdirect(d, energy, alch, soft, nwgNb, st);
-    if (pme) launch_pme_fft(d, energy, sp);
+    if (pme) launch_pme_fft(d, energy, sp, head ? kFftTail : kFftAll);
     if (fork) launch_force_assemble(d, kAsmPme, sp);
     if (alch) launch_nb_dudl(d, soft, sd);
     if (fork) {
@@ -223,11 +285,7 @@ struct bm_system {
     if (st3) (void)hipStreamSynchronize(st3);
     if (st2) (void)hipStreamSynchronize(st2);
     if (st) (void)hipStreamSynchronize(st);   // no graph may still run
-    for (int a = 0; a < 2; a++)
-      for (int b = 0; b < 2; b++) {
-        if (graph[a][b]) (void)hipGraphExecDestroy(graph[a][b]);
-        if (graphSrc[a][b]) (void)hipGraphDestroy(graphSrc[a][b]);
-      }
+    graphs.drop();
     for (auto &e : ev)
       if (e) (void)hipEventDestroy(e);
     if (evFork) (void)hipEventDestroy(evFork);
@@ -1227,24 +1285,9 @@ static int regrow(bm_system *s, int flag) {
   return BM_OK;
 }
 
-// capture and instantiate the step graph of one (rebuild, energy) variant
-static int capture_step_graph(bm_system *s, int rb, int en) {
-  if (s->graph[rb][en]) return BM_OK;
-  HIPCHK(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
-  s->step_launches(rb, en);
-  hipGraph_t g = nullptr;
-  HIPCHK(hipStreamEndCapture(s->st, &g));
-  s->graphSrc[rb][en] = g;
-  HIPCHK(hipGraphInstantiate(&s->graph[rb][en], g, nullptr, nullptr, 0));
-  return BM_OK;
-}
-
 int bm_capture_graphs(bm_system *s) {
   if (!s) return BM_EINVAL;
-  for (int rb = 0; rb < 2; rb++)
-    for (int en = 0; en < 2; en++)
-      if (int rc = capture_step_graph(s, rb, en)) return rc;
-  return BM_OK;
+  return s->graphs.capture_all(s->st, [&](int rb, int en) { return s->step_launches(rb, en), BM_OK; });
 }
 
 // True under rocprofv3 hardware-counter collection (it exports
@@ -1263,16 +1306,12 @@ static bool counter_collection() {
 // the launches of steps [step0, step0 + nsteps)
 static int dynamics_launches(bm_system *s, long step0, long nsteps, int freq_nrg, int use_graph) {
   blade::launch_set_step(s->d, step0, s->st);
-  for (long k = 0; k < nsteps; k++) {
-    const long step = step0 + k;
-    const int rb = (step % s->freqDomdec) == 0, en = (step % freq_nrg) == 0;
-    if (!use_graph) {
-      s->step_launches(rb, en);
-      HIPCHK(hipGetLastError());
-      continue;
-    }
-    if (int rc = capture_step_graph(s, rb, en)) return rc;
-    HIPCHK(hipGraphLaunch(s->graph[rb][en], s->st));
+  if (use_graph)
+    return s->graphs.play(step0, nsteps, s->freqDomdec, freq_nrg, s->st,
+                          [&](int rb, int en) { return s->step_launches(rb, en), BM_OK; });
+  for (long step = step0; step < step0 + nsteps; step++) {
+    s->step_launches((step % s->freqDomdec) == 0, (step % freq_nrg) == 0);
+    HIPCHK(hipGetLastError());
   }
   return BM_OK;
 }
@@ -1322,8 +1361,7 @@ struct bm_batch {
   hipStream_t st = nullptr, st2 = nullptr, st3 = nullptr;
   hipEvent_t fork = nullptr, fork2 = nullptr, join2 = nullptr, join3 = nullptr;
   std::vector<hipEvent_t> join;
-  hipGraphExec_t graph[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
-  hipGraph_t graphSrc[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
+  StepGraphs graphs;
   // fused launches of a non-energy step
   MultiPlan pack, normals, bonded, tail;
   std::vector<MultiPlan> spread, fftp, fftx, mfs, mfp, mfx, nb, nbd, asmb;
@@ -1334,11 +1372,7 @@ struct bm_batch {
     if (st) (void)hipStreamSynchronize(st);
     if (st2) (void)hipStreamSynchronize(st2);
     if (st3) (void)hipStreamSynchronize(st3);
-    for (int a = 0; a < 2; a++)
-      for (int b = 0; b < 2; b++) {
-        if (graph[a][b]) (void)hipGraphExecDestroy(graph[a][b]);
-        if (graphSrc[a][b]) (void)hipGraphDestroy(graphSrc[a][b]);
-      }
+    graphs.drop();
     for (auto e : join)
       if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : {fork, fork2, join2, join3})
@@ -1358,14 +1392,22 @@ struct bm_batch {
       for (MultiPlan &p : *g) v.push_back(&p);
     return v;
   }
-  // the members' current Dev into every plan's device copies
+  // the members' current Dev into every plan's device copies, unless they
+  // hold it already (a barostat move or grown buffers change it)
+  std::vector<blade::Dev> held;
   int upload_devs() {
+    bool same = held.size() == sys.size();
+    for (size_t k = 0; same && k < sys.size(); k++)
+      same = std::memcmp(&held[k], &sys[k]->d, sizeof(blade::Dev)) == 0;
+    if (same) return BM_OK;
+    held.clear();
     for (MultiPlan *p : plans()) {
       std::vector<blade::Dev> h;
       for (int k : p->members) h.push_back(sys[k]->d);
       if (hipMemcpy(p->devs, h.data(), h.size() * sizeof(blade::Dev), hipMemcpyHostToDevice) != hipSuccess)
         return set_err(BM_EHIP, "batch: Dev upload");
     }
+    for (bm_system *s : sys) held.push_back(s->d);
     return BM_OK;
   }
   // one non-energy step with one launch per kernel type and group
@@ -1590,27 +1632,11 @@ static int batch_step_launches(bm_batch *b, int rb, int en) {
   return BM_OK;
 }
 
-// capture and instantiate the batch step graph of one (rebuild, energy)
-// variant
-static int capture_batch_graph(bm_batch *b, int rb, int en) {
-  if (b->graph[rb][en]) return BM_OK;
-  HIPCHK(hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal));
-  if (int rc = batch_step_launches(b, rb, en)) return rc;
-  hipGraph_t g = nullptr;
-  HIPCHK(hipStreamEndCapture(b->st, &g));
-  b->graphSrc[rb][en] = g;
-  HIPCHK(hipGraphInstantiate(&b->graph[rb][en], g, nullptr, nullptr, 0));
-  return BM_OK;
-}
-
 int bm_batch_capture_graphs(bm_batch *b) {
   if (!b) return BM_EINVAL;
   HIPCHK(hipSetDevice(b->device));
   if (int rc = b->upload_devs()) return rc;
-  for (int rb = 0; rb < 2; rb++)
-    for (int en = 0; en < 2; en++)
-      if (int rc = capture_batch_graph(b, rb, en)) return rc;
-  return BM_OK;
+  return b->graphs.capture_all(b->st, [&](int rb, int en) { return batch_step_launches(b, rb, en); });
 }
 
 int bm_batch_dynamics(bm_batch *b, long step0, long nsteps, int freq_nrg) {
@@ -1631,17 +1657,14 @@ int bm_batch_dynamics(bm_batch *b, long step0, long nsteps, int freq_nrg) {
   }
   for (bm_system *s : b->sys) blade::launch_set_step(s->d, step0, b->st);
   const int freqDomdec = b->sys[0]->freqDomdec;
-  const bool eager = counter_collection();
-  for (long k = 0; k < nsteps; k++) {
-    const long step = step0 + k;
-    const int rb = (step % freqDomdec) == 0, en = (step % freq_nrg) == 0;
-    if (eager) {
-      if (int rc = batch_step_launches(b, rb, en)) return rc;
+  if (counter_collection()) {
+    for (long step = step0; step < step0 + nsteps; step++) {
+      if (int rc = batch_step_launches(b, (step % freqDomdec) == 0, (step % freq_nrg) == 0)) return rc;
       HIPCHK(hipGetLastError());
-      continue;
     }
-    if (int rc = capture_batch_graph(b, rb, en)) return rc;
-    HIPCHK(hipGraphLaunch(b->graph[rb][en], b->st));
+  } else if (int rc = b->graphs.play(step0, nsteps, freqDomdec, freq_nrg, b->st,
+                                     [&](int rb, int en) { return batch_step_launches(b, rb, en); })) {
+    return rc;
   }
   // members' later work (getters, eager steps) follows the batch
   HIPCHK(hipEventRecord(b->fork, b->st));
