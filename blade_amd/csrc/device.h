@@ -57,7 +57,7 @@ struct Dev {
   int *sb;                       // [N] siteBlock code
   double *qd;                    // [N] charge, FP64 (energy sums, spread)
   float *qlam;                   // [N] scratch: lambda*q (PME)
-  float2 *vdw;                   // [T*T] (c12, c6)
+  float2 *vdw;                   // [T*T] force factors (12 c12, 6 c6); (c12, c6) for BM_VSWITCH
   double2 *vdwd;                 // [T*T] (c12, c6) FP64 for energy sums
   double *blockq2;               // [nL] sum of q^2 over each block (Ewald self term)
   float *slo;                    // [32*maxB] slot charge low part: q - (float)q
@@ -88,6 +88,7 @@ struct Dev {
   int *nchunks;                  // [1]
   int maxchunks;
   int4 *chunk;                   // [maxchunks] (I, first tile, tiles, 0)
+  int *corder;                   // [maxchunks] the chunks, those with most tiles in reach first
   float *ichunk;                 // [maxchunks][3][32] i-force partials of a chunk (FP32, fixed
                                  // order); the force assembly converts them to fixed point
   int nalchat;                   // atoms of lambda blocks (site block != 0)
@@ -95,7 +96,7 @@ struct Dev {
   int *nexcltiles;               // [1] tiles with exclusions
   unsigned *emask;               // [32*2*n_excl]
   int *exstart, *exadj;          // [N+1],[2*n_excl] atoms excluded from each atom
-  int *workctr;                  // [4] dynamic work counters
+  int *workctr;                  // [2] long and short chunks ordered so far, zeroed by the pack
   int *errflag;                  // [1] overflow / capacity errors
   double rlist2;                 // (rcut+pad)^2, as the oracle computes it
   double ddscale[3];             // box * 2^-32, as the oracle computes it

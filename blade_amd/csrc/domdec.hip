@@ -226,8 +226,9 @@ __global__ void __launch_bounds__(256) dd_sort_columns_multi(Multi m) {
 // The gap to either side is a difference modulo 2^32.  Pairs clearly inside
 // or outside in FP32 (whose error is below 1e-6 relative) are settled
 // there; the rest in the oracle's FP64 arithmetic.
+// core: the boxes are within rcut as they stand.
 __device__ __forceinline__ bool dd_close(const Dev &d, const unsigned (&aLo)[3], const unsigned (&aHi)[3],
-                                         const unsigned (&bLo)[3], const unsigned (&bHi)[3]) {
+                                         const unsigned (&bLo)[3], const unsigned (&bHi)[3], bool &core) {
   unsigned gap[3];
   float sf = 0.f;
 #pragma unroll
@@ -238,6 +239,7 @@ __device__ __forceinline__ bool dd_close(const Dev &d, const unsigned (&aLo)[3],
     sf += g * g;
   }
   const float r2 = (float)d.rlist2;
+  core = sf <= d.rc2;
   if (sf < r2 * 0.99999f) return true;
   if (sf > r2 * 1.00001f) return false;
   double g[3];
@@ -268,7 +270,8 @@ __device__ __forceinline__ void dd_stage_boxes(const Dev &d, int nb, unsigned *l
 }
 
 __device__ __forceinline__ bool dd_tile_keep(const Dev &d, const unsigned *lo, const unsigned *hi, int I,
-                                             const unsigned (&aLo)[3], const unsigned (&aHi)[3], int J) {
+                                             const unsigned (&aLo)[3], const unsigned (&aHi)[3], int J, bool &core) {
+  core = true;
   if (J == I) return true;
   unsigned bLo[3], bHi[3];
 #pragma unroll
@@ -276,7 +279,7 @@ __device__ __forceinline__ bool dd_tile_keep(const Dev &d, const unsigned *lo, c
     bLo[k] = J < kBoxLds ? lo[3 * J + k] : d.bblo[3 * J + k];
     bHi[k] = J < kBoxLds ? hi[3 * J + k] : d.bbhi[3 * J + k];
   }
-  return dd_close(d, aLo, aHi, bLo, bHi);
+  return dd_close(d, aLo, aHi, bLo, bHi, core);
 }
 
 // one wave per i-block: number of blocks J within the list radius (all J)
@@ -297,7 +300,8 @@ __device__ __forceinline__ void dd_tile_count_body(const Dev &d, int bid, int nb
   int cnt = 0;
   for (int J0 = 0; J0 < nb; J0 += 64) {
     const int J = J0 + lane;
-    const bool keep = J < nb && dd_tile_keep(d, s_lo, s_hi, I, aLo, aHi, J);
+    bool core;
+    const bool keep = J < nb && dd_tile_keep(d, s_lo, s_hi, I, aLo, aHi, J, core);
     cnt += __popcll(__ballot(keep));
   }
   if (lane == 0) d.tcount[I] = cnt;
@@ -325,6 +329,8 @@ __device__ __forceinline__ void dd_tile_write_body(const Dev &d, int bid) {
   if (halted_wg(d)) return;   // a halted step leaves the list as it is
   __shared__ unsigned s_lo[3 * kBoxLds], s_hi[3 * kBoxLds];
   __shared__ int s_sum[4];
+  constexpr int kRowChunks = 64;   // chunks of a row counted one by one (later ones share the last count)
+  __shared__ int s_core[4][kRowChunks];
   extern __shared__ unsigned long long s_row[];
   const int nb = *d.nblocks, rows = 4;
   const int tc = d.tchunk, I0 = bid * rows;
@@ -350,6 +356,7 @@ __device__ __forceinline__ void dd_tile_write_body(const Dev &d, int bid) {
   if (all > d.maxtiles || call > d.maxchunks) return;
   before = wg_sum256(before, s_sum);
   cbefore = wg_sum256(cbefore, s_sum);
+  s_core[threadIdx.x >> 6][threadIdx.x & 63] = 0;
   dd_stage_boxes(d, nb, s_lo, s_hi);
   const int w = threadIdx.x >> 6, I = I0 + w;
   const int lane = threadIdx.x & 63;
@@ -382,10 +389,12 @@ __device__ __forceinline__ void dd_tile_write_body(const Dev &d, int bid) {
   int run = 0;
   for (int J0 = 0; J0 < nb; J0 += 64) {
     const int J = J0 + lane;
-    const bool keep = J < nb && dd_tile_keep(d, s_lo, s_hi, I, aLo, aHi, J);
+    bool core = false;
+    const bool keep = J < nb && dd_tile_keep(d, s_lo, s_hi, I, aLo, aHi, J, core);
     const unsigned long long m = __ballot(keep);
     if (keep) {
-      const int t = before + run + __popcll(m & below);
+      const int q = run + __popcll(m & below), t = before + q;
+      if (core) atomicAdd(&s_core[w][min(q / tc, kRowChunks - 1)], 1);
       d.tile_i[t] = I;
       d.tile_j[t] = J;
     }
@@ -396,9 +405,28 @@ __device__ __forceinline__ void dd_tile_write_body(const Dev &d, int bid) {
     }
     run += __popcll(m);
   }
-  for (int k = lane; k < nchunk; k += 64)
-    d.chunk[cbefore + k] = make_int4(I, before + k * tc, min(tc, cnt - k * tc), 0);
   dd_wave_sync();
+  // The chunks, and the order of the pair kernel's waves: those with more
+  // than half their tiles within rcut from the front, the others from the
+  // back.  A SIMD serves about eight waves of 2 to 16 near tiles at this
+  // list's usual sizes, so the last ones to start should be short.
+  for (int k0 = 0; k0 < nchunk; k0 += 64) {
+    const int k = k0 + lane;
+    const bool in = k < nchunk;
+    const bool lng = in && 2 * s_core[w][min(k, kRowChunks - 1)] > tc;
+    const unsigned long long ml = __ballot(lng), ms = __ballot(in && !lng);
+    int bl = 0, bs = 0;
+    if (lane == 0) {
+      if (ml) bl = atomicAdd(&d.workctr[0], __popcll(ml));
+      if (ms) bs = atomicAdd(&d.workctr[1], __popcll(ms));
+    }
+    bl = __shfl(bl, 0, 64);
+    bs = __shfl(bs, 0, 64);
+    if (in) {
+      d.chunk[cbefore + k] = make_int4(I, before + k * tc, min(tc, cnt - k * tc), 0);
+      d.corder[lng ? bl + __popcll(ml & below) : call - 1 - (bs + __popcll(ms & below))] = cbefore + k;
+    }
+  }
   // place in the row of the tile to block J, -1 if the row has none
   auto place = [&](int J) {
     const unsigned long long m = bits[J >> 6], bit = 1ull << (J & 63);

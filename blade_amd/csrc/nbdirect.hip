@@ -73,7 +73,9 @@ __device__ __forceinline__ NbConst make_const(const Dev &d) {
   return c;
 }
 
-// One pair at distance r (1/r = rinv); qq already x kE.  f = dE/dr.  The
+// One pair at distance r (1/r = rinv); qq already x kE, and, except for the
+// switched potential, c12 and c6 already x 12 and x 6 (as the table of force
+// factors holds them).  f = dE/dr.  The
 // energy is returned factored, E = qq*eq + c12*eA - c6*eB, so an energy
 // sum can apply the parameters in FP64 (the factors carry only the
 // distance-dependent FP32 rounding, which does not bias the sum).
@@ -84,7 +86,8 @@ __device__ __forceinline__ void pair_ef(const NbConst &c, float qq, float c12, f
     float br = c.beta * r;
     // argument >= -(beta rcut)^2 log2(e), far above the denormal range
     float ex = __builtin_amdgcn_exp2f(-c.beta2log2e * r * r);
-    float erfcrinv = erfc_fit(fminf(br, BM_ERFC_XMAX), ex) * rinv;
+    // (past the fit's range, beta r > 4, its error is below 1e-4 of 1.5e-8)
+    float erfcrinv = erfc_fit(br, ex) * rinv;
     f = -qq * (erfcrinv + kTwoOverSqrtPi * c.beta * ex) * rinv;
     eq = erfcrinv;
   } else if (ELEC == BM_FSWITCH) {
@@ -118,7 +121,7 @@ __device__ __forceinline__ void pair_ef(const NbConst &c, float qq, float c12, f
     const float a3 = rinv3 - c.rcinv3, a6 = rinv6 - c.rcinv6;
     const float A = in ? rinv6 : c.k6 * a3 * rinv3;
     const float B = in ? rinv6 * rinv6 : c.k12 * a6 * rinv6;
-    f += (6 * c6 * A - 12 * c12 * B) * rinv;
+    f += (c6 * A - c12 * B) * rinv;
     eA = in ? rinv6 * rinv6 - c.dv6 * c.dv6 : c.k12 * a6 * a6;
     eB = in ? rinv6 - c.dv6 : c.k6 * a3 * a3;
   } else if (VDW == BM_VSWITCH) {
@@ -136,7 +139,7 @@ __device__ __forceinline__ void pair_ef(const NbConst &c, float qq, float c12, f
   } else {
     float r2 = r * r, r5 = r2 * r2 * r;
     float rinv7 = rinv6 * rinv, rinv12 = rinv6 * rinv6, rinv13 = rinv12 * rinv;
-    f += 6 * c6 * (rinv7 - r5 * c.rcinv12) - 12 * c12 * (rinv13 + r5 * c.rcinv18);
+    f += c6 * (rinv7 - r5 * c.rcinv12) - c12 * (rinv13 + r5 * c.rcinv18);
     // shifted energies vanish as (rc-r)^2: FP64 (alchemical pairs only)
     const double ri = 1.0 / (double)r, ri6 = ri * ri * ri * ri * ri * ri, rd = r;
     const double r6d = rd * rd * rd * rd * rd * rd;
@@ -277,24 +280,15 @@ __device__ __forceinline__ bool boxes_within(const Dev &d, int I, int J, float r
 
 // j-atom (fractional coordinates pj) within rcut of the current box of
 // block I (centre/half extent in fractional counts)
+__device__ __forceinline__ float box_gap(unsigned d, unsigned h, float scale) {
+  const unsigned a = (unsigned)abs((int)d);   // 2^31 stays 2^31
+  return a > h ? (float)(a - h) * scale : 0.f;
+}
 __device__ __forceinline__ bool near_box(const Dev &d, uint4 ci, uint4 hi, uint4 pj, float rc2) {
-  float g2 = 0;
-  {
-    long long g = llabs((long long)(int)(pj.x - ci.x)) - (long long)hi.x;
-    float gf = g > 0 ? (float)g * d.fracscale[0] : 0.f;
-    g2 += gf * gf;
-  }
-  {
-    long long g = llabs((long long)(int)(pj.y - ci.y)) - (long long)hi.y;
-    float gf = g > 0 ? (float)g * d.fracscale[1] : 0.f;
-    g2 += gf * gf;
-  }
-  {
-    long long g = llabs((long long)(int)(pj.z - ci.z)) - (long long)hi.z;
-    float gf = g > 0 ? (float)g * d.fracscale[2] : 0.f;
-    g2 += gf * gf;
-  }
-  return g2 <= rc2 * 1.0001f;
+  const float gx = box_gap(pj.x - ci.x, hi.x, d.fracscale[0]);
+  const float gy = box_gap(pj.y - ci.y, hi.y, d.fracscale[1]);
+  const float gz = box_gap(pj.z - ci.z, hi.z, d.fracscale[2]);
+  return fmaf(gz, gz, fmaf(gx, gx, gy * gy)) <= rc2 * 1.0001f;
 }
 
 // an atom within rcut of the current box of block J
@@ -801,10 +795,11 @@ __device__ __forceinline__ void nbdirect_kernel_body(const Dev &d, int bid, int 
   unsigned char *sjx = s_jx[w];
 
   (void)nblk;
-  // one chunk per wave; waves past this step's chunk count exit
+  // one chunk per wave, the long ones first; waves past this step's chunk
+  // count exit
   const int k = bid * 4 + w;
   if (k >= nchunks) return;
-  chunk_pairs<ELEC, VDW, ENERGY, ALCH, SOFT>(d, c, ec, s_vdw, k, lane, half, li, sp, spr, slo, sjx, eacc);
+  chunk_pairs<ELEC, VDW, ENERGY, ALCH, SOFT>(d, c, ec, s_vdw, d.corder[k], lane, half, li, sp, spr, slo, sjx, eacc);
   if (ENERGY) {
     long long v = (long long)__double2ll_rn(eacc * kFixScaleD);
     wave_atomic_fix(&d.energy[BM_ENBDIRECT], v);
@@ -934,7 +929,8 @@ __device__ __forceinline__ void nb_dudl_body(const Dev &d, int bid) {
     if (SOFT && dredll != 0.0) {
       float f, eq, eA, eB;
       const float rf = (float)reff;
-      pair_ef<ELEC, VDW>(c, (float)qq, (float)ljd.x, (float)ljd.y, rf, 1.f / rf, f, eq, eA, eB);
+      const float m12 = VDW == BM_VSWITCH ? 1.f : 12.f, m6 = VDW == BM_VSWITCH ? 1.f : 6.f;
+      pair_ef<ELEC, VDW>(c, (float)qq, m12 * (float)ljd.x, m6 * (float)ljd.y, rf, 1.f / rf, f, eq, eA, eB);
       fl += sd * (double)f * dredll;
     }
     acc += same ? 0.5 * fl : lo * fl;

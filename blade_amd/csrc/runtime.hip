@@ -471,7 +471,9 @@ int bm_system_create(int device, const bm_topology *t, const bm_runparams *rp, c
     UPLOAD(d.mass, ms);
     ALLOC(d.qlam, n);
     std::vector<float2> vdw((size_t)t->n_types * t->n_types);
-    for (size_t k = 0; k < vdw.size(); k++) vdw[k] = make_float2((float)t->vdw_c12[k], (float)t->vdw_c6[k]);
+    const float m12 = rp->vdw_method == BM_VSWITCH ? 1.f : 12.f, m6 = rp->vdw_method == BM_VSWITCH ? 1.f : 6.f;
+    for (size_t k = 0; k < vdw.size(); k++)
+      vdw[k] = make_float2(m12 * (float)t->vdw_c12[k], m6 * (float)t->vdw_c6[k]);
     UPLOAD(d.vdw, vdw);
     std::vector<double2> vdwd(vdw.size());
     for (size_t k = 0; k < vdw.size(); k++) vdwd[k] = make_double2(t->vdw_c12[k], t->vdw_c6[k]);
@@ -526,6 +528,7 @@ int bm_system_create(int device, const bm_topology *t, const bm_runparams *rp, c
   ALLOC(d.cstart, MB + 1);
   ALLOC(d.nchunks, 1);
   ALLOC(d.chunk, d.maxchunks);
+  ALLOC(d.corder, d.maxchunks);
   ALLOC(d.ichunk, (size_t)d.maxchunks * 3 * kBlockAtoms);
   ALLOC(d.nexcltiles, 1);
   ALLOC(d.emask, 2 * (size_t)std::max(1, t->n_excl) * kBlockAtoms);
@@ -543,7 +546,7 @@ int bm_system_create(int device, const bm_topology *t, const bm_runparams *rp, c
     UPLOAD(d.exstart, start);
     UPLOAD(d.exadj, adj);
   }
-  ALLOC(d.workctr, 4);
+  ALLOC(d.workctr, 2);
   // PME
   if (rp->elec_method == BM_PME) {
     for (int k = 0; k < 3; k++) d.K[k] = rp->grid[k];
@@ -1220,7 +1223,7 @@ static int set_tile_capacity(bm_system *s, long long maxTiles) {
   const size_t T = (size_t)maxTiles + 1;
   if ((rc = s->realloc_dev(d.tile_i, T)) || (rc = s->realloc_dev(d.tile_j, T)) ||
       (rc = s->realloc_dev(d.tile_ex, T)) ||
-      (rc = s->realloc_dev(d.chunk, (size_t)d.maxchunks)) ||
+      (rc = s->realloc_dev(d.chunk, (size_t)d.maxchunks)) || (rc = s->realloc_dev(d.corder, (size_t)d.maxchunks)) ||
       (rc = s->realloc_dev(d.ichunk, (size_t)d.maxchunks * 3 * blade::kBlockAtoms)))
     return rc;
   s->capacityGen++;

@@ -374,7 +374,7 @@ int bm_dynamics(bm_system *sys, long step0, long nsteps, int freq_nrg, int use_g
    that no later bm_dynamics call captures one (a timed run starts with
    every graph instantiated).  No counterpart in the reference. */
 int bm_capture_graphs(bm_system *sys);
-/* Set the list capacities (directed tiles; spline records per PME brick;
+/* Set the list capacities (directed tiles; atoms per PME brick;
    a value <= 0 keeps that one).  The list is emptied: the next step must
    rebuild it (a step s with s % freq_domdec == 0).  Tests use it to start
    from capacities too small for the system.  No counterpart in the
