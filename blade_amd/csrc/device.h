@@ -81,7 +81,8 @@ struct Dev {
   float4 *sbh;                   // [4*maxB] per-step cluster half extent (A; hugely negative: empty)
   uint4 *spos;                   // [32*maxB] slot (ux,uy,uz,q bits)
   int2 *spar;                    // [32*maxB] slot (type or -1, siteBlock)
-  int *tcount, *tstart;          // [maxB],[maxB+1] directed tiles per row
+  int4 *rowcount;                // [maxB] tiles, chunks, tiles with exclusions, long chunks of each row
+  int *tstart;                   // [maxB+1] directed tiles before each row
   int *ntiles;                   // [1]
   int *tile_i, *tile_j, *tile_ex;// [maxtiles]
   int *cstart;                   // [maxB+1] chunks before each row
@@ -96,7 +97,6 @@ struct Dev {
   int *nexcltiles;               // [1] tiles with exclusions
   unsigned *emask;               // [32*2*n_excl]
   int *exstart, *exadj;          // [N+1],[2*n_excl] atoms excluded from each atom
-  int *workctr;                  // [2] long and short chunks ordered so far, zeroed by the pack
   int *errflag;                  // [1] overflow / capacity errors
   double rlist2;                 // (rcut+pad)^2, as the oracle computes it
   double ddscale[3];             // box * 2^-32, as the oracle computes it

@@ -30,15 +30,19 @@
 
 namespace blade {
 
-// Sum of v over the 256 threads of a workgroup, for all of them (every
-// thread must call it; s_sum: four ints of LDS, free again on return).
-__device__ __forceinline__ int wg_sum256(int v, int *s_sum) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = v;
+// Sums of N values over the 256 threads of a workgroup, for all of them
+// (every thread must call it; s_sum: 4 N ints of LDS, free again on return).
+template <int N>
+__device__ __forceinline__ void wg_sum256(int (&v)[N], int *s_sum) {
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o, 64);
+    if ((threadIdx.x & 63) == 0) s_sum[(threadIdx.x >> 6) * N + k] = v[k];
+  }
   __syncthreads();
-  const int t = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
+#pragma unroll
+  for (int k = 0; k < N; k++) v[k] = s_sum[k] + s_sum[N + k] + s_sum[2 * N + k] + s_sum[3 * N + k];
   __syncthreads();
-  return t;
 }
 
 // Exclusive prefix sum of f(0..n) into out[0..n], out[n] the total, by the
@@ -121,10 +125,7 @@ __device__ __forceinline__ void dd_scatter_body(const Dev &d, int bid) {
   if (bid == 0) {
     for (int c = threadIdx.x; c <= d.ncol; c += blockDim.x) d.colstart[c] = s_start[c];
     wg_scan256(d.ncol, [&](int c) { return (d.colcount[c] + kBlockAtoms - 1) / kBlockAtoms; }, d.blkstart, s_sum);
-    if (threadIdx.x == 0) {
-      *d.nblocks = d.blkstart[d.ncol];   // this thread's own store
-      *d.nexcltiles = 0;
-    }
+    if (threadIdx.x == 0) *d.nblocks = d.blkstart[d.ncol];   // this thread's own store
   }
 }
 __global__ void __launch_bounds__(256) dd_scatter(Dev d) { dd_scatter_body(d, blockIdx.x); }
@@ -256,15 +257,22 @@ __device__ __forceinline__ void dd_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-constexpr int kBoxLds = 2048;   // block boxes staged in LDS by the tile kernels
+constexpr int kBoxLds = 3072;   // block boxes staged in LDS by the tile kernels (72 KB: two workgroups to a CU)
 
 // stage the first kBoxLds block boxes in LDS (every thread of the block
-// must call it)
+// must call it); 16 bytes a load, four in flight: word by word this was most
+// of the tile kernels' time at 2,900 blocks
 __device__ __forceinline__ void dd_stage_boxes(const Dev &d, int nb, unsigned *lo, unsigned *hi) {
-  const int m = 3 * min(nb, kBoxLds);
-  for (int k = threadIdx.x; k < m; k += blockDim.x) {
-    lo[k] = d.bblo[k];
-    hi[k] = d.bbhi[k];
+  const int m = 3 * min(nb, kBoxLds), m4 = m / 4;
+  const uint4 *glo = reinterpret_cast<const uint4 *>(d.bblo), *ghi = reinterpret_cast<const uint4 *>(d.bbhi);
+#pragma unroll 4
+  for (int k = threadIdx.x; k < m4; k += 256) {
+    reinterpret_cast<uint4 *>(lo)[k] = glo[k];
+    reinterpret_cast<uint4 *>(hi)[k] = ghi[k];
+  }
+  if ((int)threadIdx.x < m - 4 * m4) {
+    lo[4 * m4 + threadIdx.x] = d.bblo[4 * m4 + threadIdx.x];
+    hi[4 * m4 + threadIdx.x] = d.bbhi[4 * m4 + threadIdx.x];
   }
   __syncthreads();
 }
@@ -282,203 +290,236 @@ __device__ __forceinline__ bool dd_tile_keep(const Dev &d, const unsigned *lo, c
   return dd_close(d, aLo, aHi, bLo, bHi, core);
 }
 
-// one wave per i-block: number of blocks J within the list radius (all J)
-__device__ __forceinline__ void dd_tile_count_body(const Dev &d, int bid, int nblk) {
-  if (halted_wg(d)) return;   // a halted step leaves the list as it is
-  __shared__ unsigned s_lo[3 * kBoxLds], s_hi[3 * kBoxLds];
-  const int nb = *d.nblocks;
-  dd_stage_boxes(d, nb, s_lo, s_hi);
-  const int I = (bid * blockDim.x + threadIdx.x) >> 6;
-  const int lane = threadIdx.x & 63;
-  if (I >= nb) return;
-  unsigned aLo[3], aHi[3];
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    aLo[k] = d.bblo[3 * I + k];
-    aHi[k] = d.bbhi[3 * I + k];
-  }
-  int cnt = 0;
-  for (int J0 = 0; J0 < nb; J0 += 64) {
-    const int J = J0 + lane;
-    bool core;
-    const bool keep = J < nb && dd_tile_keep(d, s_lo, s_hi, I, aLo, aHi, J, core);
-    cnt += __popcll(__ballot(keep));
-  }
-  if (lane == 0) d.tcount[I] = cnt;
-}
-__global__ void __launch_bounds__(256) dd_tile_count(Dev d) { dd_tile_count_body(d, blockIdx.x, gridDim.x); }
-__global__ void __launch_bounds__(256) dd_tile_count_multi(Multi m) {
-  const MultiBlk b = multi_block(m);
-  const Dev d = m.devs[b.sys];
-  dd_tile_count_body(d, b.bid, b.nblk);
-}
-
-// LDS of one row in dd_tile_write: the bitmap of its blocks J (64-bit
-// words), the tiles before each word, and a bit per tile for exclusions
+// LDS of one row: the bitmap of its blocks J (64-bit words), a bit per tile
+// for exclusions, the tiles before each word of the bitmap, and the tiles
+// within rcut of each chunk
 __host__ __device__ inline int dd_row_words(int maxblocks) { return (maxblocks + 63) / 64; }
-static size_t lds_tile_write(const Dev &d) { return (size_t)4 * dd_row_words(d.maxblocks) * (8 + 8 + 4); }
+constexpr int kRowChunks = 64;   // chunks of a row counted one by one (later ones share the last count)
+constexpr int kRows = 4;         // rows (waves) of a workgroup
+static size_t lds_rows(const Dev &d) {
+  return (size_t)kRows * (dd_row_words(d.maxblocks) * (8 + 8 + 4) + kRowChunks * 4);
+}
 
-// One wave per row I (four to a workgroup): row starts of
-// tiles and chunks (sums of the counts of the rows before; flags a list that
-// outgrows its buffers), the row's tiles in ascending J and its chunks, then
-// the exclusions of the row's atoms: tiles holding one get 32 mask words
-// (bit j of word i: slots (I,i) and (J,j) are excluded), numbered by a claim
-// on the number of such tiles, -1 in tile_ex for the others.  No other wave
-// touches the masks of the row.
-__device__ __forceinline__ void dd_tile_write_body(const Dev &d, int bid) {
-  if (halted_wg(d)) return;   // a halted step leaves the list as it is
-  __shared__ unsigned s_lo[3 * kBoxLds], s_hi[3 * kBoxLds];
-  __shared__ int s_sum[4];
-  constexpr int kRowChunks = 64;   // chunks of a row counted one by one (later ones share the last count)
-  __shared__ int s_core[4][kRowChunks];
-  extern __shared__ unsigned long long s_row[];
-  const int nb = *d.nblocks, rows = 4;
-  const int tc = d.tchunk, I0 = bid * rows;
-  if (I0 >= nb) return;
-  // (32-bit sums: a list of 2^31 tiles is beyond any capacity of its arrays)
-  int before = 0, cbefore = 0, all = 0, call = 0;
-  for (int k = threadIdx.x; k < nb; k += blockDim.x) {
-    const int t = d.tcount[k], c = (t + tc - 1) / tc;
-    all += t;
-    call += c;
-    if (k < I0) {
-      before += t;
-      cbefore += c;
-    }
+struct DdRow {
+  unsigned long long *bits, *ebits;   // kept blocks; tiles with exclusions
+  int *pre, *core;                    // tiles before a word of bits; tiles of a chunk within rcut
+  int cnt;                            // tiles of the row
+
+  __device__ __forceinline__ void place_lds(const Dev &d, unsigned long long *lds, int w) {
+    const int nw = dd_row_words(d.maxblocks);
+    bits = lds + w * nw;
+    ebits = lds + (kRows + w) * nw;
+    pre = reinterpret_cast<int *>(lds + 2 * kRows * nw) + w * nw;
+    core = reinterpret_cast<int *>(lds + 2 * kRows * nw) + kRows * nw + w * kRowChunks;
   }
-  all = wg_sum256(all, s_sum);
-  call = wg_sum256(call, s_sum);
-  if (bid == 0 && threadIdx.x == 0) {
-    *d.ntiles = all;
-    *d.nchunks = call;
-    if (all > d.maxtiles || call > d.maxchunks) atomicOr(d.errflag, 4);
+  // place in the row of the tile to block J, -1 if the row has none
+  __device__ __forceinline__ int place(int J) const {
+    const unsigned long long m = bits[J >> 6], bit = 1ull << (J & 63);
+    return m & bit ? pre[J >> 6] + __popcll(m & (bit - 1)) : -1;
   }
-  if (all > d.maxtiles || call > d.maxchunks) return;
-  before = wg_sum256(before, s_sum);
-  cbefore = wg_sum256(cbefore, s_sum);
-  s_core[threadIdx.x >> 6][threadIdx.x & 63] = 0;
-  dd_stage_boxes(d, nb, s_lo, s_hi);
-  const int w = threadIdx.x >> 6, I = I0 + w;
+  // chunk k has more than half its tiles within rcut
+  __device__ __forceinline__ bool is_long(const Dev &d, int k) const {
+    return 2 * core[min(k, kRowChunks - 1)] > d.tchunk;
+  }
+};
+
+// Exclusions of slot lane % 32 of a block, two lanes to a slot on alternate
+// ones, eight loads in flight each (an atom of a chain has a dozen or more,
+// each behind two dependent loads): f(partner's slot).
+template <class F>
+__device__ __forceinline__ void dd_exclusions(const Dev &d, int I, F f) {
+  constexpr int kBatch = 8;
+  const int lane = threadIdx.x & 63, a = d.l2g[I * kBlockAtoms + (lane & (kBlockAtoms - 1))];
+  const int x0 = a >= 0 ? d.exstart[a] + (lane >> 5) : 0, x1 = a >= 0 ? d.exstart[a + 1] : 0;
+  for (int x = x0; x < x1; x += 2 * kBatch) {
+    int sb[kBatch];
+#pragma unroll
+    for (int k = 0; k < kBatch; k++) sb[k] = x + 2 * k < x1 ? d.exadj[x + 2 * k] : a;
+#pragma unroll
+    for (int k = 0; k < kBatch; k++) sb[k] = d.g2s[sb[k]];
+#pragma unroll
+    for (int k = 0; k < kBatch; k++)
+      if (x + 2 * k < x1) f(sb[k]);
+  }
+}
+
+// One wave, row I: its blocks J within the list radius in ascending order
+// (tile(place, J) for each), its chunks' tiles within rcut, and the tiles
+// holding an excluded pair.
+template <class F>
+__device__ __forceinline__ void dd_scan_row(const Dev &d, const unsigned *lo, const unsigned *hi, int nb, int I,
+                                            DdRow &r, F tile) {
   const int lane = threadIdx.x & 63;
-  if (I >= nb) return;
-  for (int k = I0; k < I; k++) {
-    const int t = d.tcount[k];
-    before += t;
-    cbefore += (t + tc - 1) / tc;
-  }
-  const int cnt = d.tcount[I], nchunk = (cnt + tc - 1) / tc;
-  if (lane == 0) {
-    d.tstart[I] = before;
-    d.cstart[I] = cbefore;
-    if (I == nb - 1) {
-      d.tstart[nb] = before + cnt;
-      d.cstart[nb] = cbefore + nchunk;
-    }
-  }
   unsigned aLo[3], aHi[3];
 #pragma unroll
   for (int k = 0; k < 3; k++) {
     aLo[k] = d.bblo[3 * I + k];
     aHi[k] = d.bbhi[3 * I + k];
   }
-  const int nw = dd_row_words(d.maxblocks);
-  unsigned long long *bits = s_row + w * nw;                                     // kept blocks
-  unsigned long long *ebits = s_row + (rows + w) * nw;                           // tiles with exclusions
-  int *pre = reinterpret_cast<int *>(s_row + 2 * rows * nw) + w * nw;            // tiles before a word
+  r.core[lane] = 0;
+  dd_wave_sync();
   const unsigned long long below = (1ull << lane) - 1;
   int run = 0;
   for (int J0 = 0; J0 < nb; J0 += 64) {
     const int J = J0 + lane;
     bool core = false;
-    const bool keep = J < nb && dd_tile_keep(d, s_lo, s_hi, I, aLo, aHi, J, core);
+    const bool keep = J < nb && dd_tile_keep(d, lo, hi, I, aLo, aHi, J, core);
     const unsigned long long m = __ballot(keep);
     if (keep) {
-      const int q = run + __popcll(m & below), t = before + q;
-      if (core) atomicAdd(&s_core[w][min(q / tc, kRowChunks - 1)], 1);
-      d.tile_i[t] = I;
-      d.tile_j[t] = J;
+      const int q = run + __popcll(m & below);
+      if (core) atomicAdd(&r.core[min(q / d.tchunk, kRowChunks - 1)], 1);
+      tile(q, J);
     }
     if (lane == 0) {
-      bits[J0 >> 6] = m;
-      pre[J0 >> 6] = run;
-      ebits[J0 >> 6] = 0;
+      r.bits[J0 >> 6] = m;
+      r.pre[J0 >> 6] = run;
+      r.ebits[J0 >> 6] = 0;
     }
     run += __popcll(m);
   }
+  r.cnt = run;
   dd_wave_sync();
-  // The chunks, and the order of the pair kernel's waves: those with more
-  // than half their tiles within rcut from the front, the others from the
-  // back.  A SIMD serves about eight waves of 2 to 16 near tiles at this
+  dd_exclusions(d, I, [&](int sb) {
+    const int q = r.place(sb / kBlockAtoms);
+    if (q >= 0) atomicOr(&r.ebits[q >> 6], 1ull << (q & 63));
+  });
+  dd_wave_sync();
+}
+
+// one wave per i-block: its tiles, those with exclusions and its long chunks
+__device__ __forceinline__ void dd_tile_count_body(const Dev &d, int bid) {
+  if (halted_wg(d)) return;   // a halted step leaves the list as it is
+  __shared__ __attribute__((aligned(16))) unsigned s_lo[3 * kBoxLds], s_hi[3 * kBoxLds];
+  extern __shared__ unsigned long long s_row[];
+  const int nb = *d.nblocks;
+  dd_stage_boxes(d, nb, s_lo, s_hi);
+  const int w = threadIdx.x >> 6, I = bid * kRows + w, lane = threadIdx.x & 63;
+  if (I >= nb) return;
+  DdRow r;
+  r.place_lds(d, s_row, w);
+  dd_scan_row(d, s_lo, s_hi, nb, I, r, [](int, int) {});
+  const int nchunk = (r.cnt + d.tchunk - 1) / d.tchunk;
+  int flagged = 0, lng = 0;
+  for (int k = 0; 64 * k < r.cnt; k++) flagged += __popcll(r.ebits[k]);
+  for (int k0 = 0; k0 < nchunk; k0 += 64) lng += __popcll(__ballot(k0 + lane < nchunk && r.is_long(d, k0 + lane)));
+  if (lane == 0) d.rowcount[I] = make_int4(r.cnt, nchunk, flagged, lng);
+}
+__global__ void __launch_bounds__(256) dd_tile_count(Dev d) { dd_tile_count_body(d, blockIdx.x); }
+__global__ void __launch_bounds__(256) dd_tile_count_multi(Multi m) {
+  const MultiBlk b = multi_block(m);
+  const Dev d = m.devs[b.sys];
+  dd_tile_count_body(d, b.bid);
+}
+
+// One wave per row I: row starts of tiles, chunks, masks and long chunks
+// (sums of the counts of the rows before: claims on shared counters instead
+// serialise, 58 us at 740 rows and 200 at 2,900; flags a list that outgrows
+// its buffers), then the row's tiles and chunks, and the 32 mask words of
+// its tiles with exclusions (bit j of word i: slots (I,i) and (J,j) are
+// excluded; tile_ex: their index, -1 for the other tiles).  No other wave
+// touches the masks of the row.
+__device__ __forceinline__ void dd_tile_write_body(const Dev &d, int bid) {
+  if (halted_wg(d)) return;   // a halted step leaves the list as it is
+  __shared__ __attribute__((aligned(16))) unsigned s_lo[3 * kBoxLds], s_hi[3 * kBoxLds];
+  __shared__ int s_sum[4 * 8];
+  constexpr int kMaskTiles = 16;
+  __shared__ unsigned s_mask[kRows][kMaskTiles * kBlockAtoms];
+  extern __shared__ unsigned long long s_row[];
+  const int nb = *d.nblocks, I0 = bid * kRows;
+  if (I0 >= nb) return;
+  // tiles, chunks, masks, long chunks of all rows and of the rows before
+  // (32-bit sums: a list of 2^31 tiles is beyond any capacity of its arrays)
+  int v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  for (int k = threadIdx.x; k < nb; k += blockDim.x) {
+    const int4 c = d.rowcount[k];
+    v[0] += c.x;
+    v[1] += c.y;
+    v[2] += c.z;
+    v[3] += c.w;
+    if (k < I0) {
+      v[4] += c.x;
+      v[5] += c.y;
+      v[6] += c.z;
+      v[7] += c.w;
+    }
+  }
+  wg_sum256(v, s_sum);
+  const bool over = v[0] > d.maxtiles || v[1] > d.maxchunks;
+  if (bid == 0 && threadIdx.x == 0) {
+    *d.ntiles = v[0];
+    *d.nchunks = v[1];
+    *d.nexcltiles = v[2];
+    if (over) atomicOr(d.errflag, 4);
+  }
+  if (over) return;
+  dd_stage_boxes(d, nb, s_lo, s_hi);
+  const int w = threadIdx.x >> 6, I = I0 + w, lane = threadIdx.x & 63;
+  if (I >= nb) return;
+  int t0 = v[4], c0 = v[5], e0 = v[6], l0 = v[7];
+  for (int k = I0; k < I; k++) {
+    const int4 c = d.rowcount[k];
+    t0 += c.x;
+    c0 += c.y;
+    e0 += c.z;
+    l0 += c.w;
+  }
+  DdRow r;
+  r.place_lds(d, s_row, w);
+  dd_scan_row(d, s_lo, s_hi, nb, I, r, [&](int q, int J) {
+    d.tile_i[t0 + q] = I;
+    d.tile_j[t0 + q] = J;
+  });
+  const int tc = d.tchunk, nchunk = (r.cnt + tc - 1) / tc;
+  if (lane == 0) {
+    d.tstart[I] = t0;
+    d.cstart[I] = c0;
+    if (I == nb - 1) {
+      d.tstart[nb] = t0 + r.cnt;
+      d.cstart[nb] = c0 + nchunk;
+    }
+  }
+  const unsigned long long below = (1ull << lane) - 1;
+  // The chunks, and the order of the pair kernel's waves: first the long
+  // chunks.  A SIMD serves about eight waves of 2 to 16 near tiles at this
   // list's usual sizes, so the last ones to start should be short.
+  int nl = l0, ns = v[3] + c0 - l0;
   for (int k0 = 0; k0 < nchunk; k0 += 64) {
     const int k = k0 + lane;
-    const bool in = k < nchunk;
-    const bool lng = in && 2 * s_core[w][min(k, kRowChunks - 1)] > tc;
+    const bool in = k < nchunk, lng = in && r.is_long(d, k);
     const unsigned long long ml = __ballot(lng), ms = __ballot(in && !lng);
-    int bl = 0, bs = 0;
-    if (lane == 0) {
-      if (ml) bl = atomicAdd(&d.workctr[0], __popcll(ml));
-      if (ms) bs = atomicAdd(&d.workctr[1], __popcll(ms));
-    }
-    bl = __shfl(bl, 0, 64);
-    bs = __shfl(bs, 0, 64);
     if (in) {
-      d.chunk[cbefore + k] = make_int4(I, before + k * tc, min(tc, cnt - k * tc), 0);
-      d.corder[lng ? bl + __popcll(ml & below) : call - 1 - (bs + __popcll(ms & below))] = cbefore + k;
+      d.chunk[c0 + k] = make_int4(I, t0 + k * tc, min(tc, r.cnt - k * tc), 0);
+      d.corder[lng ? nl + __popcll(ml & below) : ns + __popcll(ms & below)] = c0 + k;
     }
+    nl += __popcll(ml);
+    ns += __popcll(ms);
   }
-  // place in the row of the tile to block J, -1 if the row has none
-  auto place = [&](int J) {
-    const unsigned long long m = bits[J >> 6], bit = 1ull << (J & 63);
-    return m & bit ? pre[J >> 6] + __popcll(m & (bit - 1)) : -1;
-  };
-  // two lanes to a slot, on alternate exclusions, eight loads in flight each
-  // (an atom of a chain has a dozen or more, each behind two dependent loads)
-  const int l = lane & (kBlockAtoms - 1), a = d.l2g[I * kBlockAtoms + l];
-  const int x0 = a >= 0 ? d.exstart[a] + (lane >> 5) : 0, x1 = a >= 0 ? d.exstart[a + 1] : 0;
-  constexpr int kExBatch = 8;
-  auto partners = [&](int x, int (&sb)[kExBatch]) {
-#pragma unroll
-    for (int k = 0; k < kExBatch; k++) sb[k] = x + 2 * k < x1 ? d.exadj[x + 2 * k] : a;
-#pragma unroll
-    for (int k = 0; k < kExBatch; k++) sb[k] = d.g2s[sb[k]];
-  };
-  for (int x = x0; x < x1; x += 2 * kExBatch) {
-    int sb[kExBatch];
-    partners(x, sb);
-#pragma unroll
-    for (int k = 0; k < kExBatch; k++) {
-      const int q = x + 2 * k < x1 ? place(sb[k] / kBlockAtoms) : -1;
-      if (q >= 0) atomicOr(&ebits[q >> 6], 1ull << (q & 63));
-    }
+  int e = e0;
+  for (int k = 0; 64 * k < r.cnt; k++) {
+    const unsigned long long m = r.ebits[k];
+    const int q = k * 64 + lane;
+    if (q < r.cnt) d.tile_ex[t0 + q] = (m >> lane) & 1ull ? e + __popcll(m & below) : -1;
+    e += __popcll(m);
   }
-  dd_wave_sync();
-  const int tw = (cnt + 63) / 64;   // words of ebits in use
-  int flagged = 0;
-  for (int k = 0; k < tw; k++) flagged += __popcll(ebits[k]);
-  int base = 0;
-  if (lane == 0 && flagged) base = atomicAdd(d.nexcltiles, flagged);
-  base = __shfl(base, 0, 64);
-  int e0 = base;
-  for (int k = 0; k < tw; k++) {
-    const unsigned long long m = ebits[k];
-    const int t = k * 64 + lane;
-    if (t < cnt) d.tile_ex[before + t] = (m >> lane) & 1ull ? e0 + __popcll(m & below) : -1;
-    e0 += __popcll(m);
-  }
-  for (int k = lane; k < flagged * kBlockAtoms; k += 64) d.emask[(long long)base * kBlockAtoms + k] = 0u;
-  __threadfence();   // the cleared words are in place before any lane sets bits in them
-  for (int x = x0; x < x1; x += 2 * kExBatch) {
-    int sb[kExBatch];
-    partners(x, sb);
-#pragma unroll
-    for (int k = 0; k < kExBatch; k++) {
-      const int q = x + 2 * k < x1 ? place(sb[k] / kBlockAtoms) : -1;
-      if (q < 0) continue;
-      int e = base + __popcll(ebits[q >> 6] & ((1ull << (q & 63)) - 1));
-      for (int i = 0; i < q >> 6; i++) e += __popcll(ebits[i]);
-      atomicOr(&d.emask[(long long)e * kBlockAtoms + l], 1u << (sb[k] % kBlockAtoms));
-    }
+  // the masks, built in LDS some tiles at a time and stored whole (clearing
+  // them in memory and setting bits there takes a device-wide fence between,
+  // 25 us here)
+  unsigned *mask = s_mask[w];
+  for (int m0 = e0; m0 < e; m0 += kMaskTiles) {
+    const int words = min(kMaskTiles, e - m0) * kBlockAtoms;
+    for (int k = lane; k < words; k += 64) mask[k] = 0u;
+    dd_wave_sync();
+    dd_exclusions(d, I, [&](int sb) {
+      const int q = r.place(sb / kBlockAtoms);
+      if (q < 0) return;
+      int at = e0 - m0 + __popcll(r.ebits[q >> 6] & ((1ull << (q & 63)) - 1));
+      for (int i = 0; i < q >> 6; i++) at += __popcll(r.ebits[i]);
+      if (at >= 0 && at < kMaskTiles)
+        atomicOr(&mask[at * kBlockAtoms + (lane & (kBlockAtoms - 1))], 1u << (sb % kBlockAtoms));
+    });
+    dd_wave_sync();
+    for (int k = lane; k < words; k += 64) d.emask[(long long)m0 * kBlockAtoms + k] = mask[k];
+    dd_wave_sync();
   }
 }
 __global__ void __launch_bounds__(256) dd_tile_write(Dev d) { dd_tile_write_body(d, blockIdx.x); }
@@ -506,10 +547,6 @@ __device__ __forceinline__ void dd_pack_body(const Dev &d, int bid, bool bin) {
   }
   if (s < BM_NTERMS) d.energy[s] = 0;
   if (s < d.ncol) d.colcount[s] = 0;   // for the next rebuild
-  if (s == 0) {
-    d.workctr[0] = 0;
-    d.workctr[1] = 0;
-  }
   if (bid * (int)blockDim.x >= nb * kBlockAtoms) return;  // whole wave idle
   const bool in = s < nb * kBlockAtoms;
   const int a = in ? d.l2g[s] : -1;
@@ -589,7 +626,7 @@ void launch_domdec_rebuild(const Dev &d, int maxBlocks, hipStream_t st) {
   dd_wrap_count<<<grid_rebuild(d, 0), 256, 0, st>>>(d);
   dd_scatter<<<grid_rebuild(d, 1), 256, lds_rebuild(d, 1), st>>>(d);
   dd_sort_columns<<<grid_rebuild(d, 2), 256, 0, st>>>(d);
-  dd_tile_count<<<grid_rebuild(d, 3), 256, 0, st>>>(d);
+  dd_tile_count<<<grid_rebuild(d, 3), 256, lds_rebuild(d, 3), st>>>(d);
   dd_tile_write<<<grid_rebuild(d, 4), 256, lds_rebuild(d, 4), st>>>(d);
 }
 
@@ -598,7 +635,7 @@ void launch_domdec_rebuild(const Dev &d, int maxBlocks, hipStream_t st) {
 // launches over the per-kernel plans m[kRebuildKernels] (lds: the largest
 // of their systems).
 int grid_rebuild(const Dev &d, int k) {
-  const int slots = (int)((32LL * d.maxblocks + 255) / 256), rows = (d.maxblocks + 3) / 4;
+  const int slots = (int)((32LL * d.maxblocks + 255) / 256), rows = (d.maxblocks + kRows - 1) / kRows;
   switch (k) {
     case 0: return slots;   // dd_wrap_count
     case 1: return slots;   // dd_scatter
@@ -609,14 +646,14 @@ int grid_rebuild(const Dev &d, int k) {
 
 size_t lds_rebuild(const Dev &d, int k) {
   if (k == 1) return ((size_t)d.ncol + 1) * sizeof(int);
-  return k == 4 ? lds_tile_write(d) : 0;
+  return k >= 3 ? lds_rows(d) : 0;
 }
 
 void launch_domdec_rebuild_multi(const Multi *m, const size_t *lds, hipStream_t st) {
   dd_wrap_count_multi<<<m[0].nwg, 256, 0, st>>>(m[0]);
   dd_scatter_multi<<<m[1].nwg, 256, lds[1], st>>>(m[1]);
   dd_sort_columns_multi<<<m[2].nwg, 256, 0, st>>>(m[2]);
-  dd_tile_count_multi<<<m[3].nwg, 256, 0, st>>>(m[3]);
+  dd_tile_count_multi<<<m[3].nwg, 256, lds[3], st>>>(m[3]);
   dd_tile_write_multi<<<m[4].nwg, 256, lds[4], st>>>(m[4]);
 }
 

@@ -97,14 +97,19 @@ double bspline_host(int n, double u) {
 // Step graphs: one per (rebuild, energy) variant of a step, and runs of 8, 4
 // and 2 plain steps (neither).  Between two graph launches the GPU idles 5
 // to 12 us, between two steps of one graph 1 to 2, so a run of plain steps
-// is launched in as few graphs as it divides into.
+// is launched in as few graphs as it divides into.  Capturing the runs takes
+// as long as they save in a thousand steps: they are captured up front with
+// capture_all, or after runAfter plain steps (a barostat drops the graphs at
+// every volume move, and its intervals should not pay for runs).
 struct StepGraphs {
   static constexpr int kRuns = 3;
   static constexpr int run_steps(int r) { return 8 >> r; }
   hipGraphExec_t exec[4 + kRuns] = {};
   hipGraph_t src[4 + kRuns] = {};
+  long runAfter = 1000, plainSteps = 0;   // plain steps played since the last drop
 
   void drop() {
+    plainSteps = 0;
     for (int k = 0; k < 4 + kRuns; k++) {
       if (exec[k]) (void)hipGraphExecDestroy(exec[k]);
       if (src[k]) (void)hipGraphDestroy(src[k]);
@@ -147,10 +152,11 @@ struct StepGraphs {
       if (!rb && !en) {
         const long plain = std::min({end - at, freqDomdec - at % freqDomdec, freqNrg - at % freqNrg});
         for (int r = kRuns - 1; r >= 0; r--)
-          if (run_steps(r) <= plain) {
+          if (run_steps(r) <= plain && (exec[4 + r] || plainSteps >= runAfter)) {
             k = 4 + r;
             len = run_steps(r);
           }
+        plainSteps += len;
       }
       if (int rc = capture(k, st, step)) return rc;
       HIPCHK(hipGraphLaunch(exec[k], st));
@@ -519,7 +525,7 @@ int bm_system_create(int device, const bm_topology *t, const bm_runparams *rp, c
   ALLOC(d.spos, (size_t)MB * kBlockAtoms);
   ALLOC(d.slo, (size_t)MB * kBlockAtoms);
   ALLOC(d.spar, (size_t)MB * kBlockAtoms);
-  ALLOC(d.tcount, MB);
+  ALLOC(d.rowcount, MB);
   ALLOC(d.tstart, MB + 1);
   ALLOC(d.ntiles, 1);
   ALLOC(d.tile_i, s->maxTiles + 1);
@@ -546,7 +552,6 @@ int bm_system_create(int device, const bm_topology *t, const bm_runparams *rp, c
     UPLOAD(d.exstart, start);
     UPLOAD(d.exadj, adj);
   }
-  ALLOC(d.workctr, 2);
   // PME
   if (rp->elec_method == BM_PME) {
     for (int k = 0; k < 3; k++) d.K[k] = rp->grid[k];
@@ -1593,6 +1598,7 @@ int bm_batch_create(int n, bm_system *const *systems, bm_batch **out) {
   HIPCHK(hipSetDevice(systems[0]->device));
   bm_batch *b = new bm_batch();
   b->device = systems[0]->device;
+  b->graphs.runAfter = 0;   // a batch keeps its graphs
   b->sys.assign(systems, systems + n);
   for (int k = 0; k < n; k++) b->gens.push_back(systems[k]->capacityGen);
   b->join.assign(n, nullptr);
