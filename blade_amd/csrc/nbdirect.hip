@@ -5,7 +5,10 @@
 // I of the rebuild list.  One wave64 owns a chunk: both 32-lane halves hold
 // the 32 i-atoms of block I in registers, so i-forces accumulate without
 // any cross-lane or memory traffic, and no j-side force is ever written
-// (every pair is visited from both sides; energies are taken on one).
+// (every pair is visited from both sides; energies are taken on one).  Lists
+// with too few chunks for the chip give a chunk to four waves instead, each
+// with the i-atoms in clusters of eight (nbcluster_kernel), with the same
+// bits.  Both are bound by VALU issue, not by memory or LDS.
 //
 // Per tile and step: the tile is skipped when the current block boxes are
 // farther apart than rcut; otherwise the j-atoms within rcut of the current
@@ -994,7 +997,10 @@ void launch_nb_dudl_multi(const Multi &m, int elec, int vdw, bool soft, hipStrea
 // Which form sums the chunks of a launch, the same bits either way: clusters
 // (four waves to a chunk, each a quarter as long) where one wave to a chunk
 // would leave SIMDs idle, chunks counted by the lists' capacities (about 1.6
-// times their use).
+// times their use).  One launch, one wave to a chunk against clusters: 53
+// and 21 us at 648 atoms, 88 and 117 us at 23,558 (the ordered adds of the
+// partial sums cost more than the pairs that clusters leave out once every
+// SIMD has work); the 11,121-atom cutoff box lies just below the line.
 bool nb_clusters(long long maxchunks) { return maxchunks <= 9500; }
 
 // workgroups for every chunk slot of the list capacity; those past this

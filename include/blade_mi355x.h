@@ -278,8 +278,8 @@ typedef struct bm_runparams {
   int32_t fft_mode;                /* PME FFT: 0 FP32 Stockham; 1 DFT contractions on
                                       MFMA in split-BF16x3 (every grid edge a multiple
                                       of 16 from 16 to 128, else BM_ENOTSUP) */
-  int32_t tile_chunk;              /* directed tiles per nonbonded work unit (one
-                                      wave), 1..16; 0 => 16 */
+  int32_t tile_chunk;              /* directed tiles per nonbonded work unit, 1..16;
+                                      0 => 16 */
   double soft_bond_alpha;          /* 1/softBondRadius^2, A^-2 */
   double soft_bond_power;          /* softBondExponent p of soft bonds */
 } bm_runparams;
