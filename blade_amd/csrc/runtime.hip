@@ -4,11 +4,12 @@
 // the reference's State, Potential, Domdec and the device half of Msld) and
 // drives the per-step launch sequence:
 //   [rebuild]  domdec kernels               (every freq_domdec steps)
-//   pack       slot coordinates, block boxes, zero accumulators
-//   nbdirect   tile kernel
-//   pme        spread, 5 FFT passes (convolution fused), gather + self
-//   bonded     bonds..nbex, lambda biases
-//   update     kick/drift, constraints, O/drift, constraints, theta->lambda
+//   pack       slot coordinates, block boxes, PME bins, zero accumulators
+//   side       PME spread, bonded terms and biases, the step's normals
+//   nbdirect   tile kernel (and the FP64 dU/dlambda of alchemical atoms)
+//   pme        three FFT passes (convolution fused) and the gather
+//   assembly   chunk partials into the force array, with the first kick
+//   update     drift, constraints, O/drift, constraints, theta->lambda
 // Each (rebuild, energy) step variant can be captured once into a hipGraph
 // and replayed; all counts the kernels need live in device memory, so the
 // captured graphs need no host input between replays.
@@ -166,13 +167,21 @@ struct StepGraphs {
   }
 };
 
-// least atoms of a system whose PME transforms run on a branch of their own
-constexpr int kForkAtoms = 16000;
+// least atoms of a system whose PME transforms run on a branch of their own.
+// us a step of a water box, linear and forked: 3,500 atoms 75 and 79, 4,500
+// 79 and 80, 6,000 86 and 83, 9,000 100 and 97, 12,000 122 and 105, 16,000
+// 139 and 110.  MFMA transforms, which start half of theirs before the
+// fork, cross later: 6,500 atoms 92 and 96, 9,000 (one site) 127 and 124,
+// 14,000 120 and 111.
+constexpr int kForkAtoms = 6000, kForkAtomsMfma = 9000;
+// most atoms of one whose line-form transforms take the step's own stream
+// and leave the branch to the pair kernel (see force_launches)
+constexpr int kLeadAtoms = 64000;
 
 struct bm_system {
   int device = 0;
   hipStream_t st = nullptr;
-  hipStream_t st2 = nullptr;         // PME branch of a step (default priority)
+  hipStream_t st2 = nullptr;         // PME or pair branch of a step (default priority)
   hipStream_t st3 = nullptr;         // dU/dlambda branch (default priority)
   hipEvent_t evFork = nullptr, evJoin = nullptr, evJoin3 = nullptr;
   blade::Dev d{};
@@ -230,13 +239,12 @@ struct bm_system {
   // when the pair kernel is long enough to hide them: a fork and join costs
   // about 15 us of a step, and the launch of a graph with branches 50 us of
   // host time against 17 us for a linear one of as many kernels, which a
-  // step of a small system cannot hide.  Measured around the line: see
-  // kForkAtoms.
-  bool forked() const { return d.elecmethod == BM_PME && d.n >= kForkAtoms; }
+  // step of a small system cannot hide.
+  bool forked() const { return d.elecmethod == BM_PME && d.n >= (d.fft_mode == 1 ? kForkAtomsMfma : kForkAtoms); }
 
   // all force terms: the spread, the bonded slots and the step's normals in
   // one launch; the pair kernel's chunk partials; the PME transforms with
-  // the gather (on st2 where forked()) and the FP64 dU/dlambda of the
+  // the gather (one of the two on st2 where forked()) and the FP64 dU/dlambda of the
   // alchemical atoms (on st3); then the per-atom assembly into the force array (kick:
   // it also kicks the atoms of a non-energy step).  Under stream capture the
   // fork and join become parallel graph branches.  binned: the step's pack
@@ -252,14 +260,23 @@ struct bm_system {
     // at 96^3, alone 20), so the first half runs before it.
     const bool head = pme && fork && d.fft_mode == 1;
     if (head) launch_pme_fft(d, energy, st, kFftHead);
-    hipStream_t sp = st, sd = st;
+    // On the line form (six launches) the transforms outlast the pair
+    // kernel, as the first kernel of a branch waits for free slots: they keep
+    // this stream and the pair kernel takes the branch.  A step of 18,000
+    // atoms 182 -> 169 us, 24,000 215 -> 205, 40,000 259 -> 249, 50,000
+    // 294 -> 287; at 92,000 the pair kernel is the longer one and it gives
+    // 436 -> 427 at order 6 but 484 -> 494 at order 8 with two sites.  The
+    // plane form (three launches) loses by it: 157 -> 163 at 23,558 atoms.
+    const bool lead = fork && d.fft_mode == 0 && !fft_plane_path(d) && d.n < kLeadAtoms;
+    hipStream_t sp = st, sn = st, sd = st;
     if (fork) {
       (void)hipEventRecord(evFork, st);
-      (void)hipStreamWaitEvent(sp = st2, evFork, 0);
+      (void)hipStreamWaitEvent((lead ? sn : sp) = st2, evFork, 0);
       if (alch) (void)hipStreamWaitEvent(sd = st3, evFork, 0);
     }
-    launch_nbdirect(d, energy, alch, soft, nwgNb, st);
-    if (pme) launch_pme_fft(d, energy, sp, head ? kFftTail : kFftAll);
+    if (lead) launch_pme_fft(d, energy, sp);
+    launch_nbdirect(d, energy, alch, soft, nwgNb, sn);
+    if (pme && !lead) launch_pme_fft(d, energy, sp, head ? kFftTail : kFftAll);
     if (fork) launch_force_assemble(d, kAsmPme, sp);
     if (alch) launch_nb_dudl(d, soft, sd);
     if (fork) {
