@@ -142,7 +142,10 @@ __device__ __forceinline__ void pair_ef(const NbConst &c, float qq, float c12, f
   } else {
     float r2 = r * r, r5 = r2 * r2 * r;
     float rinv7 = rinv6 * rinv, rinv12 = rinv6 * rinv6, rinv13 = rinv12 * rinv;
-    f += c6 * (rinv7 - r5 * c.rcinv12) - c12 * (rinv13 + r5 * c.rcinv18);
+    // (spelled out: left to the compiler, the contraction differs between the
+    // two forms of the pair kernel with soft core)
+    const float att = fmaf(-r5, c.rcinv12, rinv7), rep = fmaf(r5, c.rcinv18, rinv13);
+    f += fmaf(c6, att, -(c12 * rep));
     // shifted energies vanish as (rc-r)^2: FP64 (alchemical pairs only)
     const double ri = 1.0 / (double)r, ri6 = ri * ri * ri * ri * ri * ri, rd = r;
     const double r6d = rd * rd * rd * rd * rd * rd;

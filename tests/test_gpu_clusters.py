@@ -23,7 +23,7 @@ pytestmark = pytest.mark.gpu
     ("config2_small", {}),
     ("config2_small", {"tile_chunk": 5}),                   # groups of eight tiles cut short
     ("two_site_small", {"soft_core": True, "tile_chunk": 16}),
-])
+] + [("msld_small", {"soft_core": True, "vdw_method": v, "elec_method": e}) for v in range(3) for e in range(3)])
 def test_cluster_and_wave_forms_are_bit_identical(base, kw):
     sp = copy.copy(spec(base))
     for k, v in kw.items():
