@@ -556,9 +556,9 @@ __device__ __forceinline__ void bonded_body(const Dev &d, const BondedLaunch &L,
         atomic_fix(&d.dudl[s.b0], fix_d((s.b1 ? d.lambda[s.b1] : 1.0) * g));
         if (s.b1) atomic_fix(&d.dudl[s.b1], fix_d(d.lambda[s.b0] * g));
       }
-      f *= dredr;
-      put_d(d, d.sl_nb14 + 2 * t, (f / r), dr);
-      put_d(d, d.sl_nb14 + 2 * t + 1, (-f / r), dr);
+      const double fr = dredr != 0.0 ? f * dredr / r : 0.0;   // 0: a soft pair at r = 0
+      put_d(d, d.sl_nb14 + 2 * t, fr, dr);
+      put_d(d, d.sl_nb14 + 2 * t + 1, -fr, dr);
       e = et * ll;
     }
   } else if (bid < L.b_cats) {

@@ -319,6 +319,14 @@ struct IAtom {
 // kVdwLdsMax entries are read from global memory by a separate variant
 constexpr int kVdwLdsMax = 6144;
 
+// An alchemical pair without a force: one scaled to nothing, at whatever
+// distance, and a soft-core pair at r = 0, where dE/dr is zero.  Computed like
+// the others, 0 * inf would take the atom's whole sum with it.
+template <bool SOFT>
+__device__ __forceinline__ bool no_force(float s, float r2) {
+  return s == 0.f || (SOFT && !(r2 > 0.f));
+}
+
 // The pairs of one tile for the lane's i-atom: the nj j-atoms near the
 // i-box, compacted into sp/spr/slo (sjx: their slot index in block J),
 // shared out between the halves (half 0 takes entries 0, 2, ..., half 1
@@ -358,6 +366,7 @@ __device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const
       s = same ? (bi == bj ? ia.lam : 0.f) : ia.lam * lamj;
       if (SOFT) {
         const float rSoft = kSoftCoreRadius * (1.f - s);
+        if (!(r2 > 0.f)) r = 0.f;   // (0 * inf above)
         if (r < rSoft) {
           const float q = r / rSoft;
           float re = 1.f - 0.5f * q;
@@ -371,7 +380,8 @@ __device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const
     float f, eq, eA, eB;
     pair_ef<ELEC, VDW>(c, qq, lj.x, lj.y, r, rinv, f, eq, eA, eB);
     if (ALCH) f *= s;
-    if (ENERGY) {
+    const bool none = ALCH && alchPair && s == 0.f;
+    if (ENERGY && !none) {
       // FP64 pair energy from the exact integer displacement and FP64
       // charges / LJ parameters
       const double2 ljd = d.vdwd[vi];
@@ -381,6 +391,10 @@ __device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const
       const double ddz = (double)(int)(ia.p.z - pj.z) * d.ddscale[2];
       const double dd2 = ddx * ddx + ddy * ddy + ddz * ddz;
       double rid = rsqrt_d(dd2), rd = dd2 * rid;
+      if (!(dd2 > 0.0)) {   // (0 * inf in the Newton steps)
+        rid = HUGE_VAL;
+        rd = 0.0;
+      }
       double sd = 1.0;
       if (ALCH && alchPair) {
         const double li_d = (bi & 0xFFFF) ? d.lambda[bi & 0xFFFF] : 1.0;
@@ -402,6 +416,7 @@ __device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const
     float fr;
     if (SOFT && alchPair) fr = f * dredr * __frsqrt_rn(r2);
     else fr = f * rinv;
+    if (ALCH && alchPair && no_force<SOFT>(s, r2)) fr = 0.f;
     fx += fr * dx;
     fy += fr * dy;
     fz += fr * dz;
@@ -620,6 +635,7 @@ __device__ __forceinline__ void cluster_pairs(const Dev &d, const NbConst &c, co
         s = same ? (bi == bj ? ia.lam : 0.f) : ia.lam * lamj;
         if (SOFT) {
           const float rSoft = kSoftCoreRadius * (1.f - s);
+          if (!(r2 > 0.f)) r = 0.f;
           if (r < rSoft) {
             const float q1 = r / rSoft;
             float re = 1.f - 0.5f * q1;
@@ -636,6 +652,7 @@ __device__ __forceinline__ void cluster_pairs(const Dev &d, const NbConst &c, co
       (void)eq; (void)eA; (void)eB;
       if (SOFT && alchPair) fr = f * dredr * __frsqrt_rn(r2);
       else fr = f * rinv;
+      if (ALCH && alchPair && no_force<SOFT>(s, r2)) fr = 0.f;
     }
     // entries in turn (those that do not count add a zero)
     quad_add<0>(fr, dx, dy, dz, fx, fy, fz);

@@ -283,6 +283,8 @@ long nbdirect(const bm_topology *t, const bm_runparams *rp, const double *pos,
               double lj = lam(lambda, bj);
               double s = 1;
               bool sameSite = (bi & 0xFFFF0000) == (bj & 0xFFFF0000);
+              // two blocks of one site do not interact (and may coincide)
+              if (alch && sameSite && bi != bj) continue;
               if (alch) s = sameSite ? (bi == bj ? li : 0.0) : li * lj;
               Soft sc{r, 1, 0};
               if (useSoft && (bi || bj)) sc = soft_core(r, s);
@@ -299,7 +301,7 @@ long nbdirect(const bm_topology *t, const bm_runparams *rp, const double *pos,
                 }
               }
               fij *= sc.dredr;
-              fi = fi + (fij / r) * dr;
+              if (sc.dredr != 0) fi = fi + (fij / r) * dr;   // 0: a soft pair at r = 0
               eTot += 0.5 * s * p.e;
             }
           }
@@ -654,8 +656,10 @@ void nb14(const bm_topology *t, const bm_runparams *rp, const double *pos,
     double f = o.f * s.l0 * s.l1;
     scale_dudl(s, o.e + f * sc.dredll, dudl);
     f *= sc.dredr;
-    addf(force, n, i, (f / r) * dr);
-    addf(force, n, j, (-f / r) * dr);
+    if (sc.dredr != 0) {   // 0: a soft pair at r = 0
+      addf(force, n, i, (f / r) * dr);
+      addf(force, n, j, (-f / r) * dr);
+    }
     energy[BM_ENB14] += o.e * s.l0 * s.l1;
   }
 }

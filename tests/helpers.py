@@ -48,3 +48,20 @@ def lambdas0(s, name):
 
 def rel_rms(a, b):
     return float(np.sqrt(np.mean((a - b) ** 2)) / np.sqrt(np.mean(b ** 2)))
+
+
+def coincident(**kw):
+    """the small MSLD system with soft core and the last water's oxygen on a
+    heavy atom of substituent 3 (no constraint moves either); (spec, the
+    substituent atom, the oxygen)"""
+    import copy
+    sp = copy.copy(spec("msld_small"))
+    sp.pos = np.array(sp.pos)
+    sp.soft_core = True
+    for k, v in kw.items():
+        setattr(sp, k, v)
+    a = max(int(i) for i in np.flatnonzero(np.asarray(sp.atom_block) == 3) if sp.atoms[i][6] > 2)
+    o = sp.n - 3   # O, H, H
+    sp.pos[o:o + 3] += sp.pos[a] - sp.pos[o]
+    sp.pos[o] = sp.pos[a]
+    return sp, a, o

@@ -29,7 +29,7 @@ import pytest
 
 from blade_amd import synthetic, system
 from oracle import oracle as orc
-from tests.helpers import built, spec
+from tests.helpers import built, coincident, spec
 
 KE = 332.0716
 E_BOND, E_ANGLE, E_UREY, E_DIHE, E_IMPR, E_CMAP, E_NB14, E_NBDIRECT, E_NBRECIP, E_SELF, E_EXCL, E_LAMBDA = range(12)
@@ -912,6 +912,26 @@ def test_exclusion_correction_at_and_near_coincidence():
         h = 1e-4 * max(r, rs)
         dedr = (orc.nbex_pair(kqq, beta, r + h)[1] - orc.nbex_pair(kqq, beta, r - h)[1]) / (2 * h)
         assert fr * r == pytest.approx(dedr, rel=1e-6, abs=1e-9 * abs(kqq))
+
+
+def test_soft_core_pair_at_coincidence():
+    """An atom exactly on a soft-core atom: the pair's energy is that of half
+    its soft radius and its force vanishes (d r_eff/dr = 0 at r = 0), so the
+    forces, energies and dU/dlambda are the limits of a small displacement
+    (1e-7 A, where the atoms' other pairs vary on the scale of 0.1 A or more:
+    by 1e-6 of the largest value at most)."""
+    sp, a, o = coincident()
+    s = system.build(sp)
+    s.prepare()
+    top, rp = s.topology(), s.runparams()
+    lam = orc.theta_to_lambda(top, rp, np.array(sp.theta0, float))
+    x = system.soa(sp.pos)
+    f0, d0, e0, _ = orc.forces(top, rp, x, lam)
+    x[o] += 1e-7
+    f1, d1, e1, _ = orc.forces(top, rp, x, lam)
+    assert np.all(np.isfinite(f0)) and np.all(np.isfinite(e0)) and np.all(np.isfinite(d0))
+    for v0, v1 in ((f0, f1), (e0, e1), (d0, d1)):
+        assert np.max(np.abs(v1 - v0)) <= 1e-6 * np.max(np.abs(v0))
 
 
 # ---------------------------------------------------------------------------
