@@ -315,6 +315,7 @@ struct bm_system {
     if (evJoin) (void)hipEventDestroy(evJoin);
     if (evJoin3) (void)hipEventDestroy(evJoin3);
     for (void *p : allocs) (void)hipFree(p);
+    if (stage) (void)hipHostFree(stage);
     if (st3) (void)hipStreamDestroy(st3);
     if (st2) (void)hipStreamDestroy(st2);
     if (st) (void)hipStreamDestroy(st);
