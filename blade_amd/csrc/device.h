@@ -104,6 +104,8 @@ struct Dev {
   float rc, rs, beta;
   float rc2;
   double rcd, rsd, betad;        // FP64 copies for energy-step sums
+  double *erfct;                 // [erfcrows*kErfcTerms] erfc of the pair energies (energy64.h; PME)
+  int erfcrows;
   int vdwmethod, elecmethod;
   // PME
   int K[3], order;

@@ -24,6 +24,7 @@
 // atomics, and the result does not depend on the order in which the
 // chunks ran.
 #include "kernels.h"
+#include "energy64.h"
 #include "erfc_coef.h"
 
 namespace blade {
@@ -152,113 +153,6 @@ __device__ __forceinline__ void pair_ef(const NbConst &c, float qq, float c12, f
     eA = (float)(ri6 * ri6 + 2 * r6d * (double)c.rcinv18 - 3 * (double)c.rcinv12);
     eB = (float)(ri6 + r6d * (double)c.rcinv12 - 2 * (double)c.rcinv6);
   }
-}
-
-// ---- FP64 pair energies of energy steps ----------------------------------
-// The total potential is a small difference of large pair sums, so the sum
-// is built from FP64 pair energies.  1/x and 1/sqrt(x) are the hardware
-// approximation refined by Newton steps, and erfc is the fit of
-// fit_erfc.py times exp by range reduction and its Taylor series: about 90
-// FP64 instructions a pair without a branch, where the library's erfc walks
-// through three ranges, of which a wave takes all.  Relative error of erfc
-// below 4e-14 on [0, 6] (tests/test_erfc64.py).
-__device__ __forceinline__ double rcp_d(double x) {
-  double y = __builtin_amdgcn_rcp(x);
-  y = fma(fma(-x, y, 1.0), y, y);
-  return fma(fma(-x, y, 1.0), y, y);
-}
-__device__ __forceinline__ double rsqrt_d(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  y = fma(y, fma(-0.5 * x * y, y, 0.5), y);
-  return fma(y, fma(-0.5 * x * y, y, 0.5), y);
-}
-// (polynomial coefficients in constant memory: read into scalar registers;
-// as literals they are kept in two vector registers each)
-__constant__ double c_exp[13] = {1.0,        1.0,         1.0 / 2,      1.0 / 6,       1.0 / 24,       1.0 / 120,      1.0 / 720,
-                                 1.0 / 5040, 1.0 / 40320, 1.0 / 362880, 1.0 / 3628800, 1.0 / 39916800, 1.0 / 479001600};
-__constant__ double c_erfc[BM_ERFCD_DEG + 1] = {BM_ERFCD_COEF};
-__device__ __forceinline__ double exp_d(double v) {
-  const double n = rint(v * 1.4426950408889634);
-  // ln 2 as its float value and the rest
-  double r = fma(n, -(double)0.693147182464599609375f, v);
-  r = fma(n, 1.904654299957767878541823e-09, r);
-  double p = c_exp[12];   // sum r^k / k!, |r| <= ln 2 / 2
-#pragma unroll
-  for (int k = 11; k >= 0; k--) p = fma(p, r, c_exp[k]);
-  return ldexp(p, (int)n);
-}
-__device__ __forceinline__ double erfc_d(double x) {
-  const double xc = fmin(x, BM_ERFCD_XMAX);
-  const double y = fma(-2.0 * BM_ERFCD_A, rcp_d(xc + BM_ERFCD_A), 1.0);
-  double p = c_erfc[BM_ERFCD_DEG];
-#pragma unroll
-  for (int k = BM_ERFCD_DEG - 1; k >= 0; k--) p = fma(p, y, c_erfc[k]);
-  return p * exp_d(-x * x);
-}
-
-struct EnConst {
-  double rc, rs, beta, rcinv;
-  double rc3i, rc6i, k6, k12, dv6, dv12;   // VFSWITCH
-  double A, B, C, D, dvc, roff2;           // FSWITCH
-  double rul3i;                            // VSWITCH
-};
-
-__device__ __forceinline__ EnConst make_energy_const(const Dev &d) {
-  EnConst c;
-  c.rc = d.rcd; c.rs = d.rsd; c.beta = d.betad;
-  c.rcinv = 1.0 / c.rc;
-  const double rc3 = c.rc * c.rc * c.rc, rs3 = c.rs * c.rs * c.rs;
-  c.rc3i = 1 / rc3;
-  c.rc6i = c.rc3i * c.rc3i;
-  c.k6 = rc3 / (rc3 - rs3);
-  c.k12 = rc3 * rc3 / (rc3 * rc3 - rs3 * rs3);
-  c.dv6 = 1 / (rc3 * rs3);
-  c.dv12 = c.dv6 * c.dv6;
-  const double roff2 = c.rc * c.rc, ron2 = c.rs * c.rs;
-  const double g = 1 / ((roff2 - ron2) * (roff2 - ron2) * (roff2 - ron2));
-  c.roff2 = roff2;
-  c.rul3i = g;
-  c.A = roff2 * roff2 * (roff2 - 3 * ron2) * g;
-  c.B = 6 * roff2 * ron2 * g;
-  c.C = -(ron2 + roff2) * g;
-  c.D = 0.4 * g;
-  c.dvc = 8 * (ron2 * roff2 * (c.rc - c.rs) - (roff2 * roff2 * c.rc - ron2 * ron2 * c.rs) / 5) * g;
-  return c;
-}
-
-// energy of a pair at effective distance r (rinv = 1/r)
-template <int ELEC, int VDW>
-__device__ __forceinline__ double pair_energy_sum(const EnConst &c, double qq, double c12, double c6, double r,
-                                                double rinv) {
-  const double r2 = r * r;
-  double e;
-  if (ELEC == BM_PME) {
-    e = qq * erfc_d(c.beta * r) * rinv;
-  } else if (ELEC == BM_FSWITCH) {
-    const double r3 = r2 * r, r5 = r3 * r2;
-    const double in = rinv + c.dvc;
-    const double out = c.A * (rinv - c.rcinv) + c.B * (c.rc - r) + c.C * (c.roff2 * c.rc - r3) +
-                       c.D * (c.roff2 * c.roff2 * c.rc - r5);
-    e = qq * (r <= c.rs ? in : out);
-  } else {
-    e = qq * (rinv - 2 * c.rcinv + r * (c.rcinv * c.rcinv));
-  }
-  const double rinv3 = rinv * rinv * rinv, rinv6 = rinv3 * rinv3;
-  if (VDW == BM_VFSWITCH) {
-    const bool in = r < c.rs;
-    const double a3 = rinv3 - c.rc3i, a6 = rinv6 - c.rc6i;
-    const double rep = in ? rinv6 * rinv6 - c.dv12 : c.k12 * a6 * a6;
-    const double att = in ? rinv6 - c.dv6 : c.k6 * a3 * a3;
-    e += c12 * rep - c6 * att;
-  } else if (VDW == BM_VSWITCH) {
-    const double rijl = c.rs * c.rs - r2, riju = c.roff2 - r2;
-    const double sw = r < c.rs ? 1.0 : riju * riju * (riju - 3 * rijl) * c.rul3i;
-    e += sw * (c12 * rinv6 - c6) * rinv6;
-  } else {
-    const double r6 = r2 * r2 * r2, rc12i = c.rc6i * c.rc6i;
-    e += c12 * (rinv6 * rinv6 + 2 * r6 * rc12i * c.rc6i - 3 * rc12i) - c6 * (rinv6 + r6 * rc12i - 2 * c.rc6i);
-  }
-  return e;
 }
 
 // cull test between current block boxes (centre/half extent, fractional
@@ -390,11 +284,8 @@ __device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const
       const double ddy = (double)(int)(ia.p.y - pj.y) * d.ddscale[1];
       const double ddz = (double)(int)(ia.p.z - pj.z) * d.ddscale[2];
       const double dd2 = ddx * ddx + ddy * ddy + ddz * ddz;
-      double rid = rsqrt_d(dd2), rd = dd2 * rid;
-      if (!(dd2 > 0.0)) {   // (0 * inf in the Newton steps)
-        rid = HUGE_VAL;
-        rd = 0.0;
-      }
+      double rd = 0.0, rid = HUGE_VAL;
+      if (dd2 > 0.0) sqrt_rsqrt(dd2, __builtin_amdgcn_rsq(dd2), rd, rid);
       double sd = 1.0;
       if (ALCH && alchPair) {
         const double li_d = (bi & 0xFFFF) ? d.lambda[bi & 0xFFFF] : 1.0;
@@ -406,7 +297,7 @@ __device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const
           if (rd < rSoft) {
             const double q = rd / rSoft;
             rd = ((1.0 - 0.5 * q) * q * q * q + 0.5) * rSoft;
-            rid = rcp_d(rd);
+            rid = 1.0 / rd;
           }
         }
       }
@@ -797,20 +688,33 @@ __device__ __forceinline__ void nbdirect_kernel_body(const Dev &d, int bid, int 
   __shared__ int2 s_par[4][kBlockAtoms];
   __shared__ float s_lo[4][kBlockAtoms];
   __shared__ unsigned char s_jx[4][kBlockAtoms];
-  extern __shared__ float2 s_vdw_dyn[];
+  constexpr bool ERFC = ENERGY && ELEC == BM_PME;
+  // the erfc rows of energy steps, then the LJ table
+  extern __shared__ __attribute__((aligned(16))) double s_tab[];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int half = lane >> 5, li = lane & 31;
-  if (!GTABLE) {
-    const int nt2 = d.ntypes * d.ntypes;
-    for (int k = threadIdx.x; k < nt2; k += blockDim.x) s_vdw_dyn[k] = d.vdw[k];
-    __syncthreads();
-  }
-  const float2 *s_vdw = GTABLE ? d.vdw : s_vdw_dyn;
-  const NbConst c = make_const(d);
-  EnConst ec;
-  if (ENERGY) ec = make_energy_const(d);
   const bool fits = *d.ntiles <= d.maxtiles && *d.nchunks <= d.maxchunks;
   const int nchunks = fits ? *d.nchunks : 0;
+  if (bid * 4 >= nchunks) return;
+  float2 *s_lj = reinterpret_cast<float2 *>(s_tab + (ERFC ? d.erfcrows * kErfcTerms : 0));
+  if (ERFC) {
+    const double2 *src = reinterpret_cast<const double2 *>(d.erfct);
+#pragma unroll 2
+    for (int k = threadIdx.x; k < d.erfcrows * kErfcTerms / 2; k += 256) reinterpret_cast<double2 *>(s_tab)[k] = src[k];
+  }
+  if (!GTABLE) {
+    const int nt2 = d.ntypes * d.ntypes;
+    for (int k = threadIdx.x; k < nt2; k += blockDim.x) s_lj[k] = d.vdw[k];
+  }
+  if (ERFC || !GTABLE) __syncthreads();
+  const float2 *s_vdw = GTABLE ? d.vdw : s_lj;
+  const NbConst c = make_const(d);
+  EnConst ec;
+  if (ENERGY) ec = make_energy_const(d.rcd, d.rsd, d.betad);
+  if (ERFC) {
+    ec.erfct = s_tab;
+    ec.erfcrows = d.erfcrows;
+  }
   double eacc = 0.0;
   uint4 *sp = s_pos[w];
   int2 *spr = s_par[w];
@@ -1044,8 +948,9 @@ static void launch_t(const Dev &d, hipStream_t st) {
     return;
   }
   const unsigned grid = (unsigned)(d.maxchunks + 3) / 4;
-  if (lds) nbdirect_kernel<ELEC, VDW, ENERGY, ALCH, SOFT, false><<<grid, 256, lds, st>>>(d);
-  else nbdirect_kernel<ELEC, VDW, ENERGY, ALCH, SOFT, true><<<grid, 256, 0, st>>>(d);
+  const size_t rows = ENERGY && ELEC == BM_PME ? (size_t)d.erfcrows * kErfcTerms * sizeof(double) : 0;
+  if (lds) nbdirect_kernel<ELEC, VDW, ENERGY, ALCH, SOFT, false><<<grid, 256, rows + lds, st>>>(d);
+  else nbdirect_kernel<ELEC, VDW, ENERGY, ALCH, SOFT, true><<<grid, 256, rows, st>>>(d);
 }
 
 template <int ELEC, int VDW, bool ALCH, bool SOFT>

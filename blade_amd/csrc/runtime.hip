@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "kernels.h"
+#include "energy64.h"
 
 // bf16 of a float, rounded to nearest even (finite values), and back
 static uint16_t bf16_rne(float f) {
@@ -572,6 +573,12 @@ int bm_system_create(int device, const bm_topology *t, const bm_runparams *rp, c
   }
   // PME
   if (rp->elec_method == BM_PME) {
+    // erfc rows to the largest argument: the effective distance of a
+    // soft-core pair may exceed a cutoff shorter than the soft radius
+    d.erfcrows = erfc_rows(rp->beta_ewald * std::max(rp->rcut, (double)kSoftCoreRadius));
+    std::vector<double> ert((size_t)d.erfcrows * kErfcTerms);
+    erfc_table(ert.data(), d.erfcrows);
+    UPLOAD(d.erfct, ert);
     for (int k = 0; k < 3; k++) d.K[k] = rp->grid[k];
     d.order = rp->order;
     const size_t G = (size_t)d.K[0] * d.K[1] * d.K[2];

@@ -1,41 +1,32 @@
-"""The FP64 erfc of the pair energies (coefficients of erfc_coef.h, exp by
-range reduction and its Taylor series), restated here operation by operation
-in double precision, against scipy."""
+"""The FP64 pair energies of energy steps (blade_amd/csrc/energy64.h),
+compiled for the CPU and compared with long double: no larger an error than
+with IEEE square root and division and a library's erfc."""
 import os
-import re
-
-import numpy as np
-from scipy.special import erfcx
+import subprocess
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-HEADER = os.path.join(HERE, "..", "blade_amd", "csrc", "erfc_coef.h")
 
 
-def test_erfc64_fit():
-    src = open(HEADER).read()
-    a = float(re.search(r"BM_ERFCD_A\s+([\d.]+)", src).group(1))
-    xmax = float(re.search(r"BM_ERFCD_XMAX\s+([\d.]+)", src).group(1))
-    coef = [float(v) for v in re.findall(r"-?\d\.\d+e[+-]\d+(?=[, \n])", src.split("BM_ERFCD_COEF")[1])]
-    assert len(coef) == int(re.search(r"BM_ERFCD_DEG\s+(\d+)", src).group(1)) + 1
-    x = np.linspace(0.0, xmax, 60001)
-    y = 1.0 - 2.0 * a / (x + a)
-    p = np.zeros_like(x)
-    for c in reversed(coef):
-        p = p * y + c
-    # the polynomial's own error is 7e-15; Horner's roundings at |y| <= 1
-    # over coefficients summing below 1 add a few 1e-16 of erfcx(6) = 0.093
-    assert np.max(np.abs(p / erfcx(x) - 1.0)) < 4e-14
-    # exp(-x^2): |r| <= ln2/2, the series' next term is r^13/13! = 2e-16
-    v = -x * x
-    n = np.rint(v * 1.4426950408889634)
-    hi = float(np.float32(0.693147182464599609375))
-    r = (v - n * hi) + n * 1.904654299957767878541823e-09   # n*hi is exact: 24 + 6 bits
-    e = np.zeros_like(x)
-    f = 1.0
-    term = [1.0]
-    for k in range(1, 13):
-        f *= k
-        term.append(1.0 / f)
-    for c in reversed(term):
-        e = e * r + c
-    assert np.max(np.abs(np.ldexp(e, n.astype(int)) / np.exp(v) - 1.0)) < 2e-15
+def test_errors_against_long_double(tmp_path):
+    exe = str(tmp_path / "energy64_check")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-o", exe, os.path.join(HERE, "energy64_check.cpp")],
+                   check=True)
+    lines = [w.split() for w in subprocess.run([exe], check=True, capture_output=True, text=True).stdout.splitlines()]
+    print()
+    for w in lines:
+        print(*w)
+    # erfc: half an ulp (1.1e-16) each from the last sum and the row's first
+    # coefficient; the other terms, at most 0.38 of it, a rounding more
+    err, rms, lib, librms = map(float, lines[0][1:])
+    edge, far = float(lines[1][1]), float(lines[1][3])
+    assert err < 2.7e-16 and edge < 2.7e-16 and rms < librms
+    assert far < 2.2e-17 * 1e-6
+    # sqrt within 0.51 ulp; 1/sqrt as a division by the rounded root
+    s, sl, si, sil = (float(lines[2][k]) for k in (1, 2, 4, 5))
+    assert s < 1.02 * sl and si < 1.02 * sil
+    # energies: the rounding of r and 1/r, common to both, dominates
+    assert len(lines) == 3 + 6
+    for w in lines[3:]:
+        q, qp, qmax, qpmax, lj, ljp, ljmax, ljpmax = map(float, w[4:])
+        assert q < 1.02 * qp and lj < 1.02 * ljp
+        assert qmax < 1.2 * qpmax and ljmax < 1.2 * ljpmax
