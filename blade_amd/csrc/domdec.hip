@@ -257,71 +257,69 @@ __device__ __forceinline__ void dd_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-constexpr int kBoxLds = 3072;   // block boxes staged in LDS by the tile kernels (72 KB: two workgroups to a CU)
+// The tile kernels take the blocks J of a row in windows, whose boxes and
+// bitmaps they hold in LDS, so that neither grows with the system.  1,024
+// blocks (about 30,000 atoms of water to a window) take 27 KB for the counts
+// and 35 KB for the writer with its masks: five and four workgroups to a CU.
+// Counts and writer at 3,100 rows: 34 and 45 us, with windows of 2,048 blocks
+// 31 and 60 (two workgroups of the writer to a CU), with every row's bitmap
+// and 3,072 boxes in LDS 57 and 94 (one).  At 740 rows and fewer, one window
+// either way: 12 and 20 us.
+constexpr int kWindow = 1024;
+constexpr int kRowChunks = 64;   // chunks of a row counted one by one (later ones share the last count)
+constexpr int kRows = 4;         // rows (waves) of a workgroup
 
-// stage the first kBoxLds block boxes in LDS (every thread of the block
-// must call it); 16 bytes a load, four in flight: word by word this was most
-// of the tile kernels' time at 2,900 blocks
-__device__ __forceinline__ void dd_stage_boxes(const Dev &d, int nb, unsigned *lo, unsigned *hi) {
-  const int m = 3 * min(nb, kBoxLds), m4 = m / 4;
-  const uint4 *glo = reinterpret_cast<const uint4 *>(d.bblo), *ghi = reinterpret_cast<const uint4 *>(d.bbhi);
+// block boxes [W0, W0 + kWindow) into LDS (every thread of the block must
+// call it); 16 bytes a load, four in flight: word by word this was most of
+// the tile kernels' time at 2,900 blocks
+__device__ __forceinline__ void dd_stage_boxes(const Dev &d, int W0, int nb, unsigned *lo, unsigned *hi) {
+  if (W0) __syncthreads();   // the window before has been used
+  const int m = 3 * min(nb - W0, kWindow), m4 = m / 4;
+  const uint4 *glo = reinterpret_cast<const uint4 *>(d.bblo + 3 * (size_t)W0);
+  const uint4 *ghi = reinterpret_cast<const uint4 *>(d.bbhi + 3 * (size_t)W0);
 #pragma unroll 4
   for (int k = threadIdx.x; k < m4; k += 256) {
     reinterpret_cast<uint4 *>(lo)[k] = glo[k];
     reinterpret_cast<uint4 *>(hi)[k] = ghi[k];
   }
   if ((int)threadIdx.x < m - 4 * m4) {
-    lo[4 * m4 + threadIdx.x] = d.bblo[4 * m4 + threadIdx.x];
-    hi[4 * m4 + threadIdx.x] = d.bbhi[4 * m4 + threadIdx.x];
+    const size_t k = 4 * m4 + threadIdx.x;
+    lo[k] = d.bblo[3 * (size_t)W0 + k];
+    hi[k] = d.bbhi[3 * (size_t)W0 + k];
   }
   __syncthreads();
 }
 
-__device__ __forceinline__ bool dd_tile_keep(const Dev &d, const unsigned *lo, const unsigned *hi, int I,
-                                             const unsigned (&aLo)[3], const unsigned (&aHi)[3], int J, bool &core) {
-  core = true;
-  if (J == I) return true;
-  unsigned bLo[3], bHi[3];
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    bLo[k] = J < kBoxLds ? lo[3 * J + k] : d.bblo[3 * J + k];
-    bHi[k] = J < kBoxLds ? hi[3 * J + k] : d.bbhi[3 * J + k];
-  }
-  return dd_close(d, aLo, aHi, bLo, bHi, core);
-}
-
-// LDS of one row: the bitmap of its blocks J (64-bit words), a bit per tile
-// for exclusions, the tiles before each word of the bitmap, and the tiles
-// within rcut of each chunk
-__host__ __device__ inline int dd_row_words(int maxblocks) { return (maxblocks + 63) / 64; }
-constexpr int kRowChunks = 64;   // chunks of a row counted one by one (later ones share the last count)
-constexpr int kRows = 4;         // rows (waves) of a workgroup
-static size_t lds_rows(const Dev &d) {
-  return (size_t)kRows * (dd_row_words(d.maxblocks) * (8 + 8 + 4) + kRowChunks * 4);
-}
+// LDS of one row's window: the bitmap of its blocks J (64-bit words), the
+// tiles before each word, a bit per tile for exclusions; and the tiles within
+// rcut of each chunk of the row
+struct DdRowLds {
+  unsigned long long bits[kRows][kWindow / 64], ebits[kRows][kWindow / 64];
+  int pre[kRows][kWindow / 64], core[kRows][kRowChunks];
+};
 
 struct DdRow {
-  unsigned long long *bits, *ebits;   // kept blocks; tiles with exclusions
-  int *pre, *core;                    // tiles before a word of bits; tiles of a chunk within rcut
-  int cnt;                            // tiles of the row
+  unsigned long long *bits, *ebits;   // kept blocks; tiles with exclusions, by place in the window
+  int *pre, *core;                    // tiles of the window before a word of bits; tiles of a chunk within rcut
+  int W0, base, cnt;                  // the window; tiles of the row before it; tiles in it
 
-  __device__ __forceinline__ void place_lds(const Dev &d, unsigned long long *lds, int w) {
-    const int nw = dd_row_words(d.maxblocks);
-    bits = lds + w * nw;
-    ebits = lds + (kRows + w) * nw;
-    pre = reinterpret_cast<int *>(lds + 2 * kRows * nw) + w * nw;
-    core = reinterpret_cast<int *>(lds + 2 * kRows * nw) + kRows * nw + w * kRowChunks;
+  __device__ __forceinline__ DdRow(DdRowLds &l, int w)
+      : bits(l.bits[w]), ebits(l.ebits[w]), pre(l.pre[w]), core(l.core[w]), W0(0), base(0), cnt(0) {
+    core[threadIdx.x & 63] = 0;
   }
-  // place in the row of the tile to block J, -1 if the row has none
+  // place in the window of the tile to block J, -1 if it has none
   __device__ __forceinline__ int place(int J) const {
-    const unsigned long long m = bits[J >> 6], bit = 1ull << (J & 63);
-    return m & bit ? pre[J >> 6] + __popcll(m & (bit - 1)) : -1;
+    const unsigned j = J - W0;
+    if (j >= (unsigned)kWindow) return -1;
+    const unsigned long long m = bits[j >> 6], bit = 1ull << (j & 63);
+    return m & bit ? pre[j >> 6] + __popcll(m & (bit - 1)) : -1;
   }
   // chunk k has more than half its tiles within rcut
   __device__ __forceinline__ bool is_long(const Dev &d, int k) const {
     return 2 * core[min(k, kRowChunks - 1)] > d.tchunk;
   }
 };
+static_assert(kRowChunks == 64, "a lane clears each chunk's count");
 
 // Exclusions of slot lane % 32 of a block, two lanes to a slot on alternate
 // ones, eight loads in flight each (an atom of a chain has a dozen or more,
@@ -343,11 +341,11 @@ __device__ __forceinline__ void dd_exclusions(const Dev &d, int I, F f) {
   }
 }
 
-// One wave, row I: its blocks J within the list radius in ascending order
-// (tile(place, J) for each), its chunks' tiles within rcut, and the tiles
-// holding an excluded pair.
+// One wave, row I, window W0: the blocks J of the window within the list
+// radius in ascending order (tile(place in the row, J) for each), their
+// chunks' tiles within rcut, and the tiles holding an excluded pair.
 template <class F>
-__device__ __forceinline__ void dd_scan_row(const Dev &d, const unsigned *lo, const unsigned *hi, int nb, int I,
+__device__ __forceinline__ void dd_scan_row(const Dev &d, const unsigned *lo, const unsigned *hi, int W0, int nb, int I,
                                             DdRow &r, F tile) {
   const int lane = threadIdx.x & 63;
   unsigned aLo[3], aHi[3];
@@ -356,24 +354,30 @@ __device__ __forceinline__ void dd_scan_row(const Dev &d, const unsigned *lo, co
     aLo[k] = d.bblo[3 * I + k];
     aHi[k] = d.bbhi[3 * I + k];
   }
-  r.core[lane] = 0;
+  r.base += r.cnt;
+  r.W0 = W0;
   dd_wave_sync();
   const unsigned long long below = (1ull << lane) - 1;
+  const int n = min(nb - W0, kWindow);
   int run = 0;
-  for (int J0 = 0; J0 < nb; J0 += 64) {
-    const int J = J0 + lane;
-    bool core = false;
-    const bool keep = J < nb && dd_tile_keep(d, lo, hi, I, aLo, aHi, J, core);
+  for (int j0 = 0; j0 < n; j0 += 64) {
+    const int j = j0 + lane, J = W0 + j;
+    bool keep = j < n, core = true;
+    if (keep && J != I) {
+      const unsigned bLo[3] = {lo[3 * j], lo[3 * j + 1], lo[3 * j + 2]};
+      const unsigned bHi[3] = {hi[3 * j], hi[3 * j + 1], hi[3 * j + 2]};
+      keep = dd_close(d, aLo, aHi, bLo, bHi, core);
+    }
     const unsigned long long m = __ballot(keep);
     if (keep) {
-      const int q = run + __popcll(m & below);
+      const int q = r.base + run + __popcll(m & below);
       if (core) atomicAdd(&r.core[min(q / d.tchunk, kRowChunks - 1)], 1);
       tile(q, J);
     }
     if (lane == 0) {
-      r.bits[J0 >> 6] = m;
-      r.pre[J0 >> 6] = run;
-      r.ebits[J0 >> 6] = 0;
+      r.bits[j0 >> 6] = m;
+      r.pre[j0 >> 6] = run;
+      r.ebits[j0 >> 6] = 0;
     }
     run += __popcll(m);
   }
@@ -389,20 +393,24 @@ __device__ __forceinline__ void dd_scan_row(const Dev &d, const unsigned *lo, co
 // one wave per i-block: its tiles, those with exclusions and its long chunks
 __device__ __forceinline__ void dd_tile_count_body(const Dev &d, int bid) {
   if (halted_wg(d)) return;   // a halted step leaves the list as it is
-  __shared__ __attribute__((aligned(16))) unsigned s_lo[3 * kBoxLds], s_hi[3 * kBoxLds];
-  extern __shared__ unsigned long long s_row[];
+  __shared__ __attribute__((aligned(16))) unsigned s_lo[3 * kWindow], s_hi[3 * kWindow];
+  __shared__ DdRowLds s_row;
   const int nb = *d.nblocks;
-  dd_stage_boxes(d, nb, s_lo, s_hi);
+  if (bid * kRows >= nb) return;
   const int w = threadIdx.x >> 6, I = bid * kRows + w, lane = threadIdx.x & 63;
+  DdRow r(s_row, w);
+  int flagged = 0;
+  for (int W0 = 0; W0 < nb; W0 += kWindow) {
+    dd_stage_boxes(d, W0, nb, s_lo, s_hi);
+    if (I >= nb) continue;   // (the wave stages and waits with the others)
+    dd_scan_row(d, s_lo, s_hi, W0, nb, I, r, [](int, int) {});
+    for (int k = 0; 64 * k < r.cnt; k++) flagged += __popcll(r.ebits[k]);
+  }
   if (I >= nb) return;
-  DdRow r;
-  r.place_lds(d, s_row, w);
-  dd_scan_row(d, s_lo, s_hi, nb, I, r, [](int, int) {});
-  const int nchunk = (r.cnt + d.tchunk - 1) / d.tchunk;
-  int flagged = 0, lng = 0;
-  for (int k = 0; 64 * k < r.cnt; k++) flagged += __popcll(r.ebits[k]);
+  const int cnt = r.base + r.cnt, nchunk = (cnt + d.tchunk - 1) / d.tchunk;
+  int lng = 0;
   for (int k0 = 0; k0 < nchunk; k0 += 64) lng += __popcll(__ballot(k0 + lane < nchunk && r.is_long(d, k0 + lane)));
-  if (lane == 0) d.rowcount[I] = make_int4(r.cnt, nchunk, flagged, lng);
+  if (lane == 0) d.rowcount[I] = make_int4(cnt, nchunk, flagged, lng);
 }
 __global__ void __launch_bounds__(256) dd_tile_count(Dev d) { dd_tile_count_body(d, blockIdx.x); }
 __global__ void __launch_bounds__(256) dd_tile_count_multi(Multi m) {
@@ -420,11 +428,11 @@ __global__ void __launch_bounds__(256) dd_tile_count_multi(Multi m) {
 // touches the masks of the row.
 __device__ __forceinline__ void dd_tile_write_body(const Dev &d, int bid) {
   if (halted_wg(d)) return;   // a halted step leaves the list as it is
-  __shared__ __attribute__((aligned(16))) unsigned s_lo[3 * kBoxLds], s_hi[3 * kBoxLds];
+  __shared__ __attribute__((aligned(16))) unsigned s_lo[3 * kWindow], s_hi[3 * kWindow];
+  __shared__ DdRowLds s_row;
   __shared__ int s_sum[4 * 8];
   constexpr int kMaskTiles = 16;
   __shared__ unsigned s_mask[kRows][kMaskTiles * kBlockAtoms];
-  extern __shared__ unsigned long long s_row[];
   const int nb = *d.nblocks, I0 = bid * kRows;
   if (I0 >= nb) return;
   // tiles, chunks, masks, long chunks of all rows and of the rows before
@@ -452,33 +460,62 @@ __device__ __forceinline__ void dd_tile_write_body(const Dev &d, int bid) {
     if (over) atomicOr(d.errflag, 4);
   }
   if (over) return;
-  dd_stage_boxes(d, nb, s_lo, s_hi);
   const int w = threadIdx.x >> 6, I = I0 + w, lane = threadIdx.x & 63;
-  if (I >= nb) return;
-  int t0 = v[4], c0 = v[5], e0 = v[6], l0 = v[7];
-  for (int k = I0; k < I; k++) {
+  int t0 = v[4], c0 = v[5], e = v[6], l0 = v[7];
+  for (int k = I0; k < min(I, nb); k++) {
     const int4 c = d.rowcount[k];
     t0 += c.x;
     c0 += c.y;
-    e0 += c.z;
+    e += c.z;
     l0 += c.w;
   }
-  DdRow r;
-  r.place_lds(d, s_row, w);
-  dd_scan_row(d, s_lo, s_hi, nb, I, r, [&](int q, int J) {
-    d.tile_i[t0 + q] = I;
-    d.tile_j[t0 + q] = J;
-  });
-  const int tc = d.tchunk, nchunk = (r.cnt + tc - 1) / tc;
+  DdRow r(s_row, w);
+  const unsigned long long below = (1ull << lane) - 1;
+  for (int W0 = 0; W0 < nb; W0 += kWindow) {
+    dd_stage_boxes(d, W0, nb, s_lo, s_hi);
+    if (I >= nb) continue;   // (the wave stages and waits with the others)
+    dd_scan_row(d, s_lo, s_hi, W0, nb, I, r, [&](int q, int J) {
+      d.tile_i[t0 + q] = I;
+      d.tile_j[t0 + q] = J;
+    });
+    const int e0 = e;
+    for (int k = 0; 64 * k < r.cnt; k++) {
+      const unsigned long long m = r.ebits[k];
+      const int q = k * 64 + lane;
+      if (q < r.cnt) d.tile_ex[t0 + r.base + q] = (m >> lane) & 1ull ? e + __popcll(m & below) : -1;
+      e += __popcll(m);
+    }
+    // the masks, built in LDS some tiles at a time and stored whole (clearing
+    // them in memory and setting bits there takes a device-wide fence
+    // between, 25 us here)
+    unsigned *mask = s_mask[w];
+    for (int m0 = e0; m0 < e; m0 += kMaskTiles) {
+      const int words = min(kMaskTiles, e - m0) * kBlockAtoms;
+      for (int k = lane; k < words; k += 64) mask[k] = 0u;
+      dd_wave_sync();
+      dd_exclusions(d, I, [&](int sb) {
+        const int q = r.place(sb / kBlockAtoms);
+        if (q < 0) return;
+        int at = e0 - m0 + __popcll(r.ebits[q >> 6] & ((1ull << (q & 63)) - 1));
+        for (int i = 0; i < q >> 6; i++) at += __popcll(r.ebits[i]);
+        if (at >= 0 && at < kMaskTiles)
+          atomicOr(&mask[at * kBlockAtoms + (lane & (kBlockAtoms - 1))], 1u << (sb % kBlockAtoms));
+      });
+      dd_wave_sync();
+      for (int k = lane; k < words; k += 64) d.emask[(long long)m0 * kBlockAtoms + k] = mask[k];
+      dd_wave_sync();
+    }
+  }
+  if (I >= nb) return;
+  const int cnt = r.base + r.cnt, tc = d.tchunk, nchunk = (cnt + tc - 1) / tc;
   if (lane == 0) {
     d.tstart[I] = t0;
     d.cstart[I] = c0;
     if (I == nb - 1) {
-      d.tstart[nb] = t0 + r.cnt;
+      d.tstart[nb] = t0 + cnt;
       d.cstart[nb] = c0 + nchunk;
     }
   }
-  const unsigned long long below = (1ull << lane) - 1;
   // The chunks, and the order of the pair kernel's waves: first the long
   // chunks.  A SIMD serves about eight waves of 2 to 16 near tiles at this
   // list's usual sizes, so the last ones to start should be short.
@@ -488,38 +525,11 @@ __device__ __forceinline__ void dd_tile_write_body(const Dev &d, int bid) {
     const bool in = k < nchunk, lng = in && r.is_long(d, k);
     const unsigned long long ml = __ballot(lng), ms = __ballot(in && !lng);
     if (in) {
-      d.chunk[c0 + k] = make_int4(I, t0 + k * tc, min(tc, r.cnt - k * tc), 0);
+      d.chunk[c0 + k] = make_int4(I, t0 + k * tc, min(tc, cnt - k * tc), 0);
       d.corder[lng ? nl + __popcll(ml & below) : ns + __popcll(ms & below)] = c0 + k;
     }
     nl += __popcll(ml);
     ns += __popcll(ms);
-  }
-  int e = e0;
-  for (int k = 0; 64 * k < r.cnt; k++) {
-    const unsigned long long m = r.ebits[k];
-    const int q = k * 64 + lane;
-    if (q < r.cnt) d.tile_ex[t0 + q] = (m >> lane) & 1ull ? e + __popcll(m & below) : -1;
-    e += __popcll(m);
-  }
-  // the masks, built in LDS some tiles at a time and stored whole (clearing
-  // them in memory and setting bits there takes a device-wide fence between,
-  // 25 us here)
-  unsigned *mask = s_mask[w];
-  for (int m0 = e0; m0 < e; m0 += kMaskTiles) {
-    const int words = min(kMaskTiles, e - m0) * kBlockAtoms;
-    for (int k = lane; k < words; k += 64) mask[k] = 0u;
-    dd_wave_sync();
-    dd_exclusions(d, I, [&](int sb) {
-      const int q = r.place(sb / kBlockAtoms);
-      if (q < 0) return;
-      int at = e0 - m0 + __popcll(r.ebits[q >> 6] & ((1ull << (q & 63)) - 1));
-      for (int i = 0; i < q >> 6; i++) at += __popcll(r.ebits[i]);
-      if (at >= 0 && at < kMaskTiles)
-        atomicOr(&mask[at * kBlockAtoms + (lane & (kBlockAtoms - 1))], 1u << (sb % kBlockAtoms));
-    });
-    dd_wave_sync();
-    for (int k = lane; k < words; k += 64) d.emask[(long long)m0 * kBlockAtoms + k] = mask[k];
-    dd_wave_sync();
   }
 }
 __global__ void __launch_bounds__(256) dd_tile_write(Dev d) { dd_tile_write_body(d, blockIdx.x); }
@@ -626,8 +636,8 @@ void launch_domdec_rebuild(const Dev &d, int maxBlocks, hipStream_t st) {
   dd_wrap_count<<<grid_rebuild(d, 0), 256, 0, st>>>(d);
   dd_scatter<<<grid_rebuild(d, 1), 256, lds_rebuild(d, 1), st>>>(d);
   dd_sort_columns<<<grid_rebuild(d, 2), 256, 0, st>>>(d);
-  dd_tile_count<<<grid_rebuild(d, 3), 256, lds_rebuild(d, 3), st>>>(d);
-  dd_tile_write<<<grid_rebuild(d, 4), 256, lds_rebuild(d, 4), st>>>(d);
+  dd_tile_count<<<grid_rebuild(d, 3), 256, 0, st>>>(d);
+  dd_tile_write<<<grid_rebuild(d, 4), 256, 0, st>>>(d);
 }
 
 // The rebuild's kernels in order, for one launch each over several
@@ -645,16 +655,15 @@ int grid_rebuild(const Dev &d, int k) {
 }
 
 size_t lds_rebuild(const Dev &d, int k) {
-  if (k == 1) return ((size_t)d.ncol + 1) * sizeof(int);
-  return k >= 3 ? lds_rows(d) : 0;
+  return k == 1 ? ((size_t)d.ncol + 1) * sizeof(int) : 0;
 }
 
 void launch_domdec_rebuild_multi(const Multi *m, const size_t *lds, hipStream_t st) {
   dd_wrap_count_multi<<<m[0].nwg, 256, 0, st>>>(m[0]);
   dd_scatter_multi<<<m[1].nwg, 256, lds[1], st>>>(m[1]);
   dd_sort_columns_multi<<<m[2].nwg, 256, 0, st>>>(m[2]);
-  dd_tile_count_multi<<<m[3].nwg, 256, lds[3], st>>>(m[3]);
-  dd_tile_write_multi<<<m[4].nwg, 256, lds[4], st>>>(m[4]);
+  dd_tile_count_multi<<<m[3].nwg, 256, 0, st>>>(m[3]);
+  dd_tile_write_multi<<<m[4].nwg, 256, 0, st>>>(m[4]);
 }
 
 int grid_pack(const Dev &d) {
