@@ -4,13 +4,13 @@
 // fractional coordinates; orc_domdec in the oracle is the same rule set).
 //
 // Rebuild sequence (no host synchronisation, fixed grids, graph-capturable):
-//   dd_wrap_count -> dd_scatter -> dd_sort_columns -> dd_tile_count ->
-//   dd_tile_write
-// Five dependent launches: each one costs about 5 us beside its own work
+//   dd_wrap_count -> [dd_scan_columns] -> dd_scatter -> dd_sort_columns ->
+//   dd_tile_count -> dd_tile_write
+// Few dependent launches: each one costs about 5 us beside its own work
 // (start-up, drain, a dependent load chain), which is most of a rebuild at
-// any size this list serves, so prefix sums over columns and rows are
-// formed by every workgroup that needs them (a few KB from L2) instead of
-// in kernels of their own, and the exclusion masks are made by the wave
+// the usual sizes, so prefix sums over columns (up to kScanCols) and rows
+// are formed by every workgroup that needs them (a few KB from L2) instead
+// of in kernels of their own, and the exclusion masks are made by the wave
 // that writes the row.
 // Every step: dd_pack (slot positions, block boxes, accumulator reset).
 //
@@ -105,27 +105,55 @@ __global__ void __launch_bounds__(256) dd_wrap_count_multi(Multi m) {
   dd_wrap_count_body(d, b.bid, b.nblk);
 }
 
+// Column starts and, with ceil(count/32) blocks to a column, block starts;
+// start: [ncol+1] in LDS or global memory, all 256 threads.
+__device__ __forceinline__ void dd_column_starts(const Dev &d, int *start, int *s_sum) {
+  wg_scan256(d.ncol, [&](int c) { return d.colcount[c]; }, start, s_sum);
+  __syncthreads();
+}
+__device__ __forceinline__ void dd_block_starts(const Dev &d, int *s_sum) {
+  wg_scan256(d.ncol, [&](int c) { return (d.colcount[c] + kBlockAtoms - 1) / kBlockAtoms; }, d.blkstart, s_sum);
+  if (threadIdx.x == 0) *d.nblocks = d.blkstart[d.ncol];   // this thread's own store
+}
+
+// Most columns whose counts every workgroup of dd_scatter scans for itself
+// (16 KB of LDS); of more, a kernel of one workgroup stores the starts first.
+// A rebuild with and without that kernel: 49.3 and 47.8 us at 961 columns,
+// 104.1 and 102.2 at 3,025, 243 and 242 at 5,625.
+constexpr int kScanCols = 4096;
+
+__device__ __forceinline__ void dd_scan_columns_body(const Dev &d) {
+  if (halted_wg(d)) return;   // a halted step leaves the list as it is
+  __shared__ int s_sum[4];
+  dd_column_starts(d, d.colstart, s_sum);
+  dd_block_starts(d, s_sum);
+}
+__global__ void __launch_bounds__(256) dd_scan_columns(Dev d) { dd_scan_columns_body(d); }
+__global__ void __launch_bounds__(256) dd_scan_columns_multi(Multi m) {
+  const MultiBlk b = multi_block(m);
+  const Dev d = m.devs[b.sys];
+  dd_scan_columns_body(d);
+}
+
 // Atoms into column buckets (bucket order is arbitrary; the column sort
-// fixes the final order).  Every workgroup scans the column counts into LDS
-// (ncol+1 ints); the first also stores the column starts and, with
-// ceil(count/32) blocks to a column, the block starts.
+// fixes the final order).  Up to kScanCols columns, every workgroup scans
+// their counts into LDS, and the first also stores the starts.
 __device__ __forceinline__ void dd_scatter_body(const Dev &d, int bid) {
   if (halted_wg(d)) return;   // a halted step leaves the list as it is
-  extern __shared__ int s_start[];
-  __shared__ int s_sum[4];
-  wg_scan256(d.ncol, [&](int c) { return d.colcount[c]; }, s_start, s_sum);
-  __syncthreads();
+  __shared__ int s_start[kScanCols + 1], s_sum[4];
+  const bool own = d.ncol <= kScanCols;
+  if (own) dd_column_starts(d, s_start, s_sum);
   const int s = bid * blockDim.x + threadIdx.x;
   const int i = s < 32 * d.maxblocks ? d.l2g[s] : -1;
   if (i >= 0) {
     const unsigned cx = (unsigned)(((unsigned long long)d.ufrac[i] * (unsigned)d.ncx) >> 32);
     const unsigned cy = (unsigned)(((unsigned long long)d.ufrac[d.n + i] * (unsigned)d.ncy) >> 32);
-    d.bucket[s_start[cx * d.ncy + cy] + d.colrank[i]] = i;
+    const int c = cx * d.ncy + cy;
+    d.bucket[(own ? s_start[c] : d.colstart[c]) + d.colrank[i]] = i;
   }
-  if (bid == 0) {
+  if (own && bid == 0) {
     for (int c = threadIdx.x; c <= d.ncol; c += blockDim.x) d.colstart[c] = s_start[c];
-    wg_scan256(d.ncol, [&](int c) { return (d.colcount[c] + kBlockAtoms - 1) / kBlockAtoms; }, d.blkstart, s_sum);
-    if (threadIdx.x == 0) *d.nblocks = d.blkstart[d.ncol];   // this thread's own store
+    dd_block_starts(d, s_sum);
   }
 }
 __global__ void __launch_bounds__(256) dd_scatter(Dev d) { dd_scatter_body(d, blockIdx.x); }
@@ -634,36 +662,34 @@ __global__ void __launch_bounds__(256) dd_pack_multi(Multi m) {
 void launch_domdec_rebuild(const Dev &d, int maxBlocks, hipStream_t st) {
   (void)maxBlocks;
   dd_wrap_count<<<grid_rebuild(d, 0), 256, 0, st>>>(d);
-  dd_scatter<<<grid_rebuild(d, 1), 256, lds_rebuild(d, 1), st>>>(d);
-  dd_sort_columns<<<grid_rebuild(d, 2), 256, 0, st>>>(d);
-  dd_tile_count<<<grid_rebuild(d, 3), 256, 0, st>>>(d);
-  dd_tile_write<<<grid_rebuild(d, 4), 256, 0, st>>>(d);
+  if (grid_rebuild(d, 1)) dd_scan_columns<<<1, 256, 0, st>>>(d);
+  dd_scatter<<<grid_rebuild(d, 2), 256, 0, st>>>(d);
+  dd_sort_columns<<<grid_rebuild(d, 3), 256, 0, st>>>(d);
+  dd_tile_count<<<grid_rebuild(d, 4), 256, 0, st>>>(d);
+  dd_tile_write<<<grid_rebuild(d, 5), 256, 0, st>>>(d);
 }
 
-// The rebuild's kernels in order, for one launch each over several
-// systems: workgroups and dynamic LDS of kernel k for system d, and the
-// launches over the per-kernel plans m[kRebuildKernels] (lds: the largest
-// of their systems).
+// The rebuild's kernels in order, for one launch each over several systems:
+// workgroups of kernel k for system d (0 leaves d out of that launch), and the
+// launches over the per-kernel plans m[kRebuildKernels].
 int grid_rebuild(const Dev &d, int k) {
   const int slots = (int)((32LL * d.maxblocks + 255) / 256), rows = (d.maxblocks + kRows - 1) / kRows;
   switch (k) {
-    case 0: return slots;   // dd_wrap_count
-    case 1: return slots;   // dd_scatter
-    case 2: return d.ncol;  // dd_sort_columns
-    default: return rows;   // dd_tile_count, dd_tile_write: a wave per block
+    case 0: return slots;                // dd_wrap_count
+    case 1: return d.ncol > kScanCols;   // dd_scan_columns
+    case 2: return slots;                // dd_scatter
+    case 3: return d.ncol;               // dd_sort_columns
+    default: return rows;                // dd_tile_count, dd_tile_write: a wave per block
   }
 }
 
-size_t lds_rebuild(const Dev &d, int k) {
-  return k == 1 ? ((size_t)d.ncol + 1) * sizeof(int) : 0;
-}
-
-void launch_domdec_rebuild_multi(const Multi *m, const size_t *lds, hipStream_t st) {
+void launch_domdec_rebuild_multi(const Multi *m, hipStream_t st) {
   dd_wrap_count_multi<<<m[0].nwg, 256, 0, st>>>(m[0]);
-  dd_scatter_multi<<<m[1].nwg, 256, lds[1], st>>>(m[1]);
-  dd_sort_columns_multi<<<m[2].nwg, 256, 0, st>>>(m[2]);
-  dd_tile_count_multi<<<m[3].nwg, 256, 0, st>>>(m[3]);
-  dd_tile_write_multi<<<m[4].nwg, 256, 0, st>>>(m[4]);
+  if (m[1].nwg) dd_scan_columns_multi<<<m[1].nwg, 256, 0, st>>>(m[1]);
+  dd_scatter_multi<<<m[2].nwg, 256, 0, st>>>(m[2]);
+  dd_sort_columns_multi<<<m[3].nwg, 256, 0, st>>>(m[3]);
+  dd_tile_count_multi<<<m[4].nwg, 256, 0, st>>>(m[4]);
+  dd_tile_write_multi<<<m[5].nwg, 256, 0, st>>>(m[5]);
 }
 
 int grid_pack(const Dev &d) {

@@ -8,10 +8,9 @@ namespace blade {
 void launch_domdec_rebuild(const Dev &d, int maxBlocks, hipStream_t st);
 // the rebuild over several systems: kRebuildKernels launches, one per
 // rebuild kernel, each over the systems of its plan
-constexpr int kRebuildKernels = 5;
+constexpr int kRebuildKernels = 6;
 int grid_rebuild(const Dev &d, int k);
-size_t lds_rebuild(const Dev &d, int k);
-void launch_domdec_rebuild_multi(const Multi *m, const size_t *lds, hipStream_t st);
+void launch_domdec_rebuild_multi(const Multi *m, hipStream_t st);
 // bin: with the PME bins of this step
 void launch_domdec_pack(const Dev &d, int maxBlocks, hipStream_t st, bool bin = false);
 // the pair kernel over the list's chunks (the FP64 dU/dlambda of the

@@ -1448,12 +1448,8 @@ struct bm_batch {
     if (rebuild) {
       // the list rebuild of every member, one launch per rebuild kernel
       blade::Multi rm[blade::kRebuildKernels];
-      size_t lds[blade::kRebuildKernels];
-      for (int k = 0; k < blade::kRebuildKernels; k++) {
-        rm[k] = this->rebuild[k].m;
-        lds[k] = this->rebuild[k].lds;
-      }
-      blade::launch_domdec_rebuild_multi(rm, lds, st);
+      for (int k = 0; k < blade::kRebuildKernels; k++) rm[k] = this->rebuild[k].m;
+      blade::launch_domdec_rebuild_multi(rm, st);
     }
     blade::launch_pack_multi(pack.m, st);
     // the spread, bonded terms and normals of every member in one launch
@@ -1543,10 +1539,8 @@ static int build_plans(bm_batch *b) {
   if ((rc = make_plan(b, b->normals, all, blade::grid_normals))) return rc;
   if ((rc = make_plan(b, b->bonded, all, blade::grid_bonded))) return rc;
   if ((rc = make_plan(b, b->tail, all, blade::grid_tail))) return rc;
-  for (int r = 0; r < blade::kRebuildKernels; r++) {
+  for (int r = 0; r < blade::kRebuildKernels; r++)
     if ((rc = make_plan(b, b->rebuild[r], all, [r](const Dev &d) { return blade::grid_rebuild(d, r); }))) return rc;
-    for (int k : all) b->rebuild[r].lds = std::max(b->rebuild[r].lds, blade::lds_rebuild(D(k), r));
-  }
   if ((rc = make_groups(b, b->spread, pme, [&](int k) { return D(k).order; }, blade::grid_pme_spread))) return rc;
   for (MultiPlan &p : b->spread) {
     p.order = D(p.members[0]).order;
