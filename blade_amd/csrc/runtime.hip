@@ -126,7 +126,11 @@ struct StepGraphs {
     if (exec[k]) return BM_OK;
     HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
     int rc = BM_OK;
+    const bool clean = hipPeekAtLastError() == hipSuccess;   // (not an error of the caller's own)
     for (int i = 0; !rc && i < (k < 4 ? 1 : run_steps(k - 4)); i++) rc = k < 4 ? step(k >> 1, k & 1) : step(0, 0);
+    // a refused launch leaves no node in the graph, only the error
+    if (!rc && clean)
+      if (const hipError_t l = hipGetLastError()) rc = set_err(BM_EHIP, hipGetErrorString(l));
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(st, &g);
     if (rc) {
