@@ -54,9 +54,9 @@ void launch_set_step(const Dev &d, long long step, hipStream_t st);
 // the bins and the spread of launch_pme_grid alone
 void launch_pme_bin(const Dev &d, hipStream_t st);
 void launch_pme_spread(const Dev &d, hipStream_t st);
-// the FFT part of launch_pme_grid alone, or its first (kFftHead: of the MFMA
-// form the charge grid and the forward y-z transforms, of other forms what
-// precedes their first transform) or remaining kernels (kFftTail)
+// the FFT part of launch_pme_grid alone, or, of the MFMA form, its first
+// kernels (kFftHead: the charge grid and the forward y-z transforms) or the
+// others (kFftTail)
 constexpr int kFftAll = 0, kFftHead = 1, kFftTail = 2;
 void launch_pme_fft(const Dev &d, bool energy, hipStream_t st, int part = kFftAll);
 // the MFMA split-BF16x3 form of it (every grid edge fft_mfma_supported)

@@ -695,13 +695,11 @@ int grid_pme_sum(const Dev &d) { return (d.K[0] * d.K[1] * d.K[2] + 255) / 256; 
 void launch_pme_sum_multi(const Multi &m, hipStream_t st) { pme_sum_multi<<<m.nwg, 256, 0, st>>>(m); }
 
 void launch_pme_fft(const Dev &d, bool energy, hipStream_t st, int part) {
-  if (part != kFftTail && (d.fft_mode == 1 || !fft_plane_path(d)))
-    pme_sum<<<(unsigned)grid_pme_sum(d), 256, 0, st>>>(d);
   if (d.fft_mode == 1) {
+    if (part != kFftTail) pme_sum<<<(unsigned)grid_pme_sum(d), 256, 0, st>>>(d);
     launch_pme_fft_mfma(d, energy, st, part);
     return;
   }
-  if (part == kFftHead) return;
   if (fft_plane_path(d)) {
     // plane path: forward z+y per x-plane, x with convolution, inverse y+z
     const unsigned gx = (unsigned)grid_fft_x(d);
@@ -721,6 +719,7 @@ void launch_pme_fft(const Dev &d, bool energy, hipStream_t st, int part) {
 #undef BM_YZI
     }
   } else {
+    pme_sum<<<(unsigned)grid_pme_sum(d), 256, 0, st>>>(d);
     const int G = d.K[0] * d.K[1] * d.K[2];
     const float2 *tw[3] = {d.twiddle, d.twiddle + d.K[0], d.twiddle + d.K[0] + d.K[1]};
     FftArgs a;
