@@ -27,18 +27,26 @@ def _water(nwat):
     return system.relax(sp)
 
 
-@pytest.mark.parametrize("atoms,grid,fft", [
+CASES = [
     (5997, (40, 48, 40), 0),        # in line, line form
     (6000, (40, 48, 40), 0),        # pair kernel on the branch
     (6000, (40, 40, 40), 0),        # transforms on the branch, plane form
     (8997, (48, 48, 48), 1),        # MFMA in line
     (9000, (48, 48, 48), 1),        # MFMA: half of them before the fork
     (23558, (60, 64, 72), 0),       # pair kernel and dU/dlambda on branches
-])
-def test_branches(atoms, grid, fft):
+]
+
+
+def _spec(atoms, grid, fft):
     sp = copy.copy(relaxed("config2") if atoms == 23558 else _water(atoms // 3))
     assert len(sp.atoms) == atoms
     sp.grid, sp.fft_mode = grid, fft
+    return sp
+
+
+@pytest.mark.parametrize("atoms,grid,fft", CASES)
+def test_branches(atoms, grid, fft):
+    sp = _spec(atoms, grid, fft)
     runs = []
     for use_graph in (True, False):
         s = system.build(sp)
@@ -54,3 +62,27 @@ def test_branches(atoms, grid, fft):
     assert all(np.array_equal(a, b) for a, b in zip(*runs))
     assert rel_rms(fg, fo) <= 1e-5
     assert abs(eg[20] - eo[20]) <= 1e-6 * abs(eo[20])
+
+
+@pytest.mark.parametrize("atoms,grid,fft", CASES)
+def test_runs_of_steps_in_one_graph(atoms, grid, fft):
+    """stretches of 15 and 7 plain steps between rebuilds (every 16) and
+    energies (every 24), played in graphs of 8, 4, 2 and 1 steps, against the
+    steps launched one by one, to the bit; twice, the second time from the
+    state and graphs of the first"""
+    sp = _spec(atoms, grid, fft)
+    runs = []
+    for use_graph in (1, 0):
+        s = system.build(sp)
+        s.set_domdec_frequency(16)
+        s.run_energy()
+        L, dev = s.L, s.device()
+        if use_graph:
+            assert L.bm_capture_graphs(dev) == 0
+        for step in (0, 48):
+            assert L.bm_dynamics(dev, step, 48, 24, use_graph) == 0
+            runs.append((*system.state(s, sp.n, sp.nblocks), s.energy()))
+        s.close()
+    assert all(np.all(np.isfinite(a)) for a in runs[3])
+    for graph, eager in ((runs[0], runs[2]), (runs[1], runs[3])):
+        assert all(np.array_equal(a, b) for a, b in zip(graph, eager))

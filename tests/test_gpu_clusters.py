@@ -9,7 +9,8 @@ import numpy as np
 import pytest
 
 from blade_amd import system
-from tests.helpers import spec
+from oracle import oracle as orc
+from tests.helpers import rel_rms, spec
 
 pytestmark = pytest.mark.gpu
 
@@ -43,4 +44,39 @@ def test_cluster_and_wave_forms_are_bit_identical(base, kw):
     wave, cluster = forces(1), forces(0)
     assert np.any(wave)
     assert np.array_equal(wave, cluster)
+    s.close()
+
+
+@pytest.mark.parametrize("soft", [False, True])
+def test_lj_table_beyond_lds(soft):
+    """more than 78 atom types (a table of more than 6,144 entries): both
+    forms read it from global memory; against the oracle too (1e-5 relative
+    RMS, 1e-6 of the pair energy)"""
+    sp = copy.deepcopy(spec("msld_small"))
+    sp.soft_core = soft
+    oxygens = [i for i, a in enumerate(sp.atoms) if a[4] == "OT"][:90]
+    for k, i in enumerate(oxygens):
+        t = "O%02dX" % k
+        a = list(sp.atoms[i])
+        a[4] = t
+        sp.atoms[i] = tuple(a)
+        sp.types[t] = sp.types["OT"]
+        sp.bond_par[("HT", t)] = next(v for key, v in sp.bond_par.items() if set(key) == {"OT", "HT"})
+        sp.angle_par[("HT", t, "HT")] = sp.angle_par[("HT", "OT", "HT")]
+        eps, rmin, eps14, rmin14, e14, comb = sp.nb_par["OT"]
+        sp.nb_par[t] = (eps, rmin + 0.002 * k, eps14, rmin14, e14, comb)
+    s = system.build(sp)
+    s.run_energy()
+    top, rp = s.topology(), s.runparams()
+    assert top.contents.n_types ** 2 > 6144
+    lam = orc.theta_to_lambda(top, rp, np.array(sp.theta0, float))
+    fo, do, eo, pairs = orc.forces(top, rp, s.positions(), lam)
+    fe, eg = s.forces(), s.energy()
+    L, dev = s.L, s.device()
+    f = np.zeros(3 * sp.n + sp.nblocks, dtype=np.int64)
+    assert L.bm_domdec_update(dev, 0) == 0 and L.bm_calc_force(dev, 0, 0) == 0 and L.bm_sync(dev) == 0
+    assert L.bm_get_force_fixed(dev, f.ctypes.data_as(C.POINTER(C.c_longlong))) == 0
+    assert np.array_equal(fe, f[:3 * sp.n] / 2.0 ** 32)
+    assert rel_rms(fe, fo) <= 1e-5
+    assert abs(eg[7] - eo[7]) <= 1e-6 * abs(eo[7])
     s.close()
