@@ -213,19 +213,19 @@ struct IAtom {
 // kVdwLdsMax entries are read from global memory by a separate variant
 constexpr int kVdwLdsMax = 6144;
 
-// An alchemical pair without a force: one scaled to nothing, at whatever
-// distance, and a soft-core pair at r = 0, where dE/dr is zero.  Computed like
-// the others, 0 * inf would take the atom's whole sum with it.
-template <bool SOFT>
-__device__ __forceinline__ bool no_force(float s, float r2) {
-  return s == 0.f || (SOFT && !(r2 > 0.f));
+// 0 < r2 < rc2 in one comparison (non-negative floats order as integers)
+__device__ __forceinline__ bool apart_within(float r2, float rc2) {
+  return __float_as_uint(r2) - 1u < __float_as_uint(rc2) - 1u;
 }
 
 // The pairs of one tile for the lane's i-atom: the nj j-atoms near the
 // i-box, compacted into sp/spr/slo (sjx: their slot index in block J),
 // shared out between the halves (half 0 takes entries 0, 2, ..., half 1
 // entries 1, 3, ...).  CHK: the tile has exclusions or is the diagonal
-// tile (I == J), so the exclusion bit and j == i are tested.
+// tile (I == J), so the exclusion bit and j == i are tested.  Alchemical
+// atoms may coincide (alternative substituents, or a soft core): such a pair
+// has no force, and is left out, as 0 * inf would take the atom's whole sum
+// with it; its soft-core energy is finite.
 template <int ELEC, int VDW, bool ENERGY, bool ALCH, bool SOFT, bool CHK>
 __device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const EnConst &ec, const IAtom &ia, int li,
                                            int half, const uint4 *sp, const int2 *spr, const float *slo,
@@ -239,7 +239,7 @@ __device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const
     const float dy = fdisp(ia.p.y, pj.y, sy);
     const float dz = fdisp(ia.p.z, pj.z, sz);
     const float r2 = dx * dx + dy * dy + dz * dz;
-    bool ok = ia.t >= 0 && r2 < c.rc2;
+    bool ok = ia.t >= 0 && (ALCH && !ENERGY ? apart_within(r2, c.rc2) : r2 < c.rc2);
     if (CHK) {
       const int jo = sjx[jl];
       ok = ok && !((em >> jo) & 1u) && !(self && jo == li);
@@ -260,7 +260,6 @@ __device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const
       s = same ? (bi == bj ? ia.lam : 0.f) : ia.lam * lamj;
       if (SOFT) {
         const float rSoft = kSoftCoreRadius * (1.f - s);
-        if (!(r2 > 0.f)) r = 0.f;   // (0 * inf above)
         if (r < rSoft) {
           const float q = r / rSoft;
           float re = 1.f - 0.5f * q;
@@ -307,7 +306,7 @@ __device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const
     float fr;
     if (SOFT && alchPair) fr = f * dredr * __frsqrt_rn(r2);
     else fr = f * rinv;
-    if (ALCH && alchPair && no_force<SOFT>(s, r2)) fr = 0.f;
+    if (ALCH && ENERGY && !(r2 > 0.f)) fr = 0.f;
     fx += fr * dx;
     fy += fr * dy;
     fz += fr * dz;
@@ -508,7 +507,7 @@ __device__ __forceinline__ void cluster_pairs(const Dev &d, const NbConst &c, co
     const float dz = fdisp(ia.p.z, pj.z, sz);
     // (spelled out as the compiler contracts tile_pairs' sum)
     const float r2 = fmaf(dz, dz, fmaf(dx, dx, dy * dy));
-    bool ok = ia.t >= 0 && r2 < c.rc2 && p0 + q < nown;
+    bool ok = ia.t >= 0 && (ALCH ? apart_within(r2, c.rc2) : r2 < c.rc2) && p0 + q < nown;
     if (CHK) ok = ok && !((st.em[ic >> 5][is] >> (ic & 31)) & 1u);
     float fr = 0.f;
     if (ok) {
@@ -526,7 +525,6 @@ __device__ __forceinline__ void cluster_pairs(const Dev &d, const NbConst &c, co
         s = same ? (bi == bj ? ia.lam : 0.f) : ia.lam * lamj;
         if (SOFT) {
           const float rSoft = kSoftCoreRadius * (1.f - s);
-          if (!(r2 > 0.f)) r = 0.f;
           if (r < rSoft) {
             const float q1 = r / rSoft;
             float re = 1.f - 0.5f * q1;
@@ -543,7 +541,6 @@ __device__ __forceinline__ void cluster_pairs(const Dev &d, const NbConst &c, co
       (void)eq; (void)eA; (void)eB;
       if (SOFT && alchPair) fr = f * dredr * __frsqrt_rn(r2);
       else fr = f * rinv;
-      if (ALCH && alchPair && no_force<SOFT>(s, r2)) fr = 0.f;
     }
     // entries in turn (those that do not count add a zero)
     quad_add<0>(fr, dx, dy, dz, fx, fy, fz);
