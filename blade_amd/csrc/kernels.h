@@ -82,7 +82,9 @@ size_t lds_pme_spread(const Dev &d);
 bool fft_plane_path(const Dev &d);
 int grid_fft_planes(const Dev &d);
 int grid_fft_x(const Dev &d);
-bool nb_clusters(long long maxchunks);   // the form of a pair-kernel launch over lists of so many chunks
+// the form of a pair-kernel launch over lists of so many chunks; beside: the
+// PME transforms or a batch's other kernels run beside it
+bool nb_clusters(long long maxchunks, bool beside);
 int grid_nbdirect(const Dev &d, bool clusters);
 int grid_nb_dudl(const Dev &d);
 // FP64 dU/dlambda of the nonbonded pairs, by alchemical atom

@@ -918,11 +918,18 @@ void launch_nb_dudl_multi(const Multi &m, int elec, int vdw, bool soft, hipStrea
 // Which form sums the chunks of a launch, the same bits either way: clusters
 // (four waves to a chunk, each a quarter as long) where one wave to a chunk
 // would leave SIMDs idle, chunks counted by the lists' capacities (about 1.6
-// times their use).  One launch, one wave to a chunk against clusters: 53
-// and 21 us at 648 atoms, 88 and 117 us at 23,558 (the ordered adds of the
-// partial sums cost more than the pairs that clusters leave out once every
-// SIMD has work); the 11,121-atom cutoff box lies just below the line.
-bool nb_clusters(long long maxchunks) { return maxchunks <= 9500; }
+// times their use).  Beyond, the ordered adds of the partial sums cost more
+// than the pairs that clusters leave out: 21 us a launch against 53 at 648
+// atoms, 117 against 88 at 23,558.  us a step with clusters and without:
+//   alone on the chip: 9,000 atoms without PME (7,180 chunks) 68 and 79,
+//   14,100 (10,969) 83 and 87, 16,000 (12,259) 88 and 89, 18,000 (13,988) 96
+//   and 90;
+//   beside PME transforms, which take the idle SIMDs: 6,000 atoms (3,358)
+//   83 and 89, 6,900 (4,224) 88 and 90, 8,100 (6,038) 97 and 91, 11,121
+//   (8,934) 114 and 104;
+//   batches: 6 of 2,000 atoms (2,784) 117 and 124, 24 of 1,000 (4,344) 192 and
+//   194, 2 of 5,000 (5,026) 106 and 103, 3 of 5,000 (7,539) 124 and 124.
+bool nb_clusters(long long maxchunks, bool beside) { return maxchunks <= (beside ? 5000 : 12500); }
 
 // workgroups for every chunk slot of the list capacity; those past this
 // step's chunk count exit at once

@@ -180,7 +180,7 @@ struct StepGraphs {
 // 14,000 120 and 111.
 constexpr int kForkAtoms = 6000, kForkAtomsMfma = 9000;
 // most atoms of one whose line-form transforms take the step's own stream
-// and leave the branch to the pair kernel (see force_launches)
+// and leave the branch to the pair kernel (see lead())
 constexpr int kLeadAtoms = 64000;
 
 struct bm_system {
@@ -246,6 +246,14 @@ struct bm_system {
   // host time against 17 us for a linear one of as many kernels, which a
   // step of a small system cannot hide.
   bool forked() const { return d.elecmethod == BM_PME && d.n >= (d.fft_mode == 1 ? kForkAtomsMfma : kForkAtoms); }
+  // On the line form (six launches) the transforms outlast the pair kernel,
+  // as the first kernel of a branch waits for free slots: they keep the
+  // step's stream and the pair kernel takes the branch.  A step of 18,000
+  // atoms 182 -> 169 us, 24,000 215 -> 205, 40,000 259 -> 249, 50,000 294 ->
+  // 287; at 92,000 the pair kernel is the longer one and it gives 436 -> 427
+  // at order 6 but 484 -> 494 at order 8 with two sites.  The plane form
+  // (three launches) loses by it: 157 -> 163 at 23,558 atoms.
+  bool lead() const { return forked() && d.fft_mode == 0 && !blade::fft_plane_path(d) && d.n < kLeadAtoms; }
 
   // all force terms: the spread, the bonded slots and the step's normals in
   // one launch; the pair kernel's chunk partials; the PME transforms with
@@ -265,14 +273,7 @@ struct bm_system {
     // at 96^3, alone 20), so the first half runs before it.
     const bool head = pme && fork && d.fft_mode == 1;
     if (head) launch_pme_fft(d, energy, st, kFftHead);
-    // On the line form (six launches) the transforms outlast the pair
-    // kernel, as the first kernel of a branch waits for free slots: they keep
-    // this stream and the pair kernel takes the branch.  A step of 18,000
-    // atoms 182 -> 169 us, 24,000 215 -> 205, 40,000 259 -> 249, 50,000
-    // 294 -> 287; at 92,000 the pair kernel is the longer one and it gives
-    // 436 -> 427 at order 6 but 484 -> 494 at order 8 with two sites.  The
-    // plane form (three launches) loses by it: 157 -> 163 at 23,558 atoms.
-    const bool lead = fork && d.fft_mode == 0 && !fft_plane_path(d) && d.n < kLeadAtoms;
+    const bool lead = this->lead();
     hipStream_t sp = st, sn = st, sd = st;
     if (fork) {
       (void)hipEventRecord(evFork, st);
@@ -419,7 +420,6 @@ int bm_system_create(int device, const bm_topology *t, const bm_runparams *rp, c
   s->maxTiles0 = s->maxTiles;
   d.tchunk = rp->tile_chunk > 0 ? rp->tile_chunk : kTileChunk;
   d.maxchunks = (int)(s->maxTiles / d.tchunk + s->maxBlocks + 1);
-  d.clusters = nb_clusters(d.maxchunks);
   const int MB = s->maxBlocks;
   int rc = 0;
 #define ALLOC(p, c) \
@@ -704,6 +704,9 @@ int bm_system_create(int device, const bm_topology *t, const bm_runparams *rp, c
     d.pmefac = (float)d.pmefacd;
     d.pmeexp = (float)d.pmeexpd;
   }
+  // the pair kernel's form (on a branch of its own it takes one wave to a
+  // chunk: 6,000 atoms 122 us a step, with clusters 125)
+  d.clusters = !s->lead() && nb_clusters(d.maxchunks, s->forked());
   // bonded terms
   {
     d.nbond = t->n_bonds;
@@ -1579,7 +1582,7 @@ static int build_plans(bm_batch *b) {
     chunks += D(k).maxchunks;
     clusters = clusters && D(k).clusters;
   }
-  clusters = clusters && blade::nb_clusters(chunks);
+  clusters = clusters && blade::nb_clusters(chunks, true);
   if ((rc = make_groups(b, b->nb, all, nkey, [=](const Dev &d) { return blade::grid_nbdirect(d, clusters); })))
     return rc;
   auto dkey = [&](int k) {
