@@ -814,7 +814,8 @@ __global__ void __launch_bounds__(256) side_kernel(Dev d, BondedLaunch L, bool e
 }
 
 // the same over several systems; the spread's plan holds the PME members of
-// spline order N
+// spline order N.  (The systems' Dev by value spill 220 bytes a lane, by
+// reference 44, at the same time: 9.17 and 9.22 ms for 40 steps of 8 replicas.)
 template <int N>
 __global__ void __launch_bounds__(256, 3) side_multi(Multi ms, Multi mb, Multi mn, bool energy) {
   int b = blockIdx.x;

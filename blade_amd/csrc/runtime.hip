@@ -174,7 +174,7 @@ struct StepGraphs {
 
 // least atoms of a system whose PME transforms run on a branch of their own.
 // us a step of a water box, linear and forked: 3,500 atoms 75 and 79, 4,500
-// 79 and 80, 6,000 86 and 83, 9,000 100 and 97, 12,000 122 and 105, 16,000
+// 79 and 80, 6,000 86 and 83, 9,000 100 and 94, 12,000 122 and 105, 16,000
 // 139 and 110.  MFMA transforms, which start half of theirs before the
 // fork, cross later: 6,500 atoms 92 and 96, 9,000 (one site) 127 and 124,
 // 14,000 120 and 111.
