@@ -9,6 +9,7 @@
 #include <stdint.h>
 
 #include "../../include/blade_mi355x.h"
+#include "energy64.h"
 
 namespace blade {
 
@@ -106,6 +107,7 @@ struct Dev {
   double rcd, rsd, betad;        // FP64 copies for energy-step sums
   double *erfct;                 // [erfcrows*kErfcTerms] erfc of the pair energies (energy64.h; PME)
   int erfcrows;
+  EnConst en;                    // constants of the FP64 pair energies
   int vdwmethod, elecmethod;
   // PME
   int K[3], order;

@@ -5,8 +5,8 @@
 // is built from FP64 pair energies.  They are formed without branches and
 // without a division per pair, each with no larger an error than the plain
 // form with IEEE division, square root and the library's erfc:
-//   * r and 1/r from the hardware's approximation of 1/sqrt by two Newton
-//     steps and one correction each, within 0.51 ulp;
+//   * r and 1/r from the hardware's approximation of 1/sqrt by a Newton
+//     step and one correction each, within 0.51 ulp;
 //   * division by constants of the system as a product and one correction;
 //   * erfc by rows of 1/16 in its argument, each a Taylor series about the
 //     row's middle.  Its error is below 2.5e-16 of erfc(x) to x = 6 (the
@@ -68,10 +68,12 @@ BM_HD double erfc_d(const double *table, int rows, double x) {
 }
 
 // ---- 1/sqrt, division ----------------------------------------------------
-// sqrt(x) and its reciprocal from an approximation y of 1/sqrt(x) (relative
-// error below 2^-20); x > 0
+// sqrt(x) and its reciprocal from an approximation y of 1/sqrt(x), x > 0: one
+// Newton step takes a relative error of 2^-20 (the hardware's is below 2^-23)
+// to 2^-39, and the correction of each result squares that
+// (1/sqrt from the rounded root, so that the two belong together: the switched
+// and shifted energies cancel)
 BM_HD void sqrt_rsqrt(double x, double y, double &s, double &si) {
-  y = fma(y, fma(-0.5 * x * y, y, 0.5), y);
   y = fma(y, fma(-0.5 * x * y, y, 0.5), y);
   const double s0 = x * y;
   s = fma(fma(-s0, s0, x), 0.5 * y, s0);
@@ -84,6 +86,9 @@ BM_HD double div_by(double x, double y, double yi) {
 }
 
 // ---- pair energy ---------------------------------------------------------
+// constants of a system's methods, formed on the host: as kernel arguments
+// they are scalar operands, computed in the kernel they took up to 30 vector
+// registers
 struct EnConst {
   double rc, rs, beta, rcinv;
   double rc3i, rc6i, k6, k12, dv6, dv12;         // VFSWITCH
@@ -91,11 +96,9 @@ struct EnConst {
   double rul3, rul3i;                            // VSWITCH
   double rc2, rc2i;                              // FSHIFT
   double rc12, rc12i, rc18, rc18i, sh12, sh6;    // VSHIFT
-  const double *erfct;                           // PME: erfc rows
-  int erfcrows;
 };
 
-BM_HD EnConst make_energy_const(double rc, double rs, double beta) {
+inline EnConst make_energy_const(double rc, double rs, double beta) {
   EnConst c;
   c.rc = rc;
   c.rs = rs;
@@ -127,18 +130,18 @@ BM_HD EnConst make_energy_const(double rc, double rs, double beta) {
   c.rc18i = 1 / c.rc18;
   c.sh12 = 3 / c.rc12;
   c.sh6 = 2 / rc6;
-  c.erfct = nullptr;
-  c.erfcrows = 0;
   return c;
 }
 
-// energy of a pair at effective distance r (rinv = 1/r)
+// energy of a pair at effective distance r (rinv = 1/r); erfct: the erfc rows
+// (PME)
 template <int ELEC, int VDW>
-BM_HD double pair_energy_sum(const EnConst &c, double qq, double c12, double c6, double r, double rinv) {
+BM_HD double pair_energy_sum(const EnConst &c, const double *erfct, int erfcrows, double qq, double c12, double c6,
+                             double r, double rinv) {
   const double r2 = r * r;
   double e;
   if (ELEC == BM_PME) {
-    e = qq * erfc_d(c.erfct, c.erfcrows, c.beta * r) * rinv;
+    e = qq * erfc_d(erfct, erfcrows, c.beta * r) * rinv;
   } else if (ELEC == BM_FSWITCH) {
     const double r3 = r2 * r, r5 = r3 * r2;
     const double in = rinv + c.dvc;

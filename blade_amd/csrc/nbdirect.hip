@@ -24,7 +24,6 @@
 // atomics, and the result does not depend on the order in which the
 // chunks ran.
 #include "kernels.h"
-#include "energy64.h"
 #include "erfc_coef.h"
 
 namespace blade {
@@ -227,7 +226,7 @@ __device__ __forceinline__ bool apart_within(float r2, float rc2) {
 // has no force, and is left out, as 0 * inf would take the atom's whole sum
 // with it; its soft-core energy is finite.
 template <int ELEC, int VDW, bool ENERGY, bool ALCH, bool SOFT, bool CHK>
-__device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const EnConst &ec, const IAtom &ia, int li,
+__device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const double *erfct, const IAtom &ia, int li,
                                            int half, const uint4 *sp, const int2 *spr, const float *slo,
                                            const unsigned char *sjx, const float2 *svdw, int nj,
                                            unsigned em, bool self, float &fx, float &fy, float &fz,
@@ -239,7 +238,7 @@ __device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const
     const float dy = fdisp(ia.p.y, pj.y, sy);
     const float dz = fdisp(ia.p.z, pj.z, sz);
     const float r2 = dx * dx + dy * dy + dz * dz;
-    bool ok = ia.t >= 0 && (ALCH && !ENERGY ? apart_within(r2, c.rc2) : r2 < c.rc2);
+    bool ok = ALCH && !ENERGY ? (ia.t >= 0) & apart_within(r2, c.rc2) : ia.t >= 0 && r2 < c.rc2;
     if (CHK) {
       const int jo = sjx[jl];
       ok = ok && !((em >> jo) & 1u) && !(self && jo == li);
@@ -273,7 +272,8 @@ __device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const
     float f, eq, eA, eB;
     pair_ef<ELEC, VDW>(c, qq, lj.x, lj.y, r, rinv, f, eq, eA, eB);
     if (ALCH) f *= s;
-    const bool none = ALCH && alchPair && s == 0.f;
+    // (without a soft core a pair scaled to nothing may be infinite at r = 0)
+    const bool none = ALCH && !SOFT && s == 0.f;
     if (ENERGY && !none) {
       // FP64 pair energy from the exact integer displacement and FP64
       // charges / LJ parameters
@@ -284,7 +284,7 @@ __device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const
       const double ddz = (double)(int)(ia.p.z - pj.z) * d.ddscale[2];
       const double dd2 = ddx * ddx + ddy * ddy + ddz * ddz;
       double rd = 0.0, rid = HUGE_VAL;
-      if (dd2 > 0.0) sqrt_rsqrt(dd2, __builtin_amdgcn_rsq(dd2), rd, rid);
+      if (r2 > 0.f) sqrt_rsqrt(dd2, __builtin_amdgcn_rsq(dd2), rd, rid);
       double sd = 1.0;
       if (ALCH && alchPair) {
         const double li_d = (bi & 0xFFFF) ? d.lambda[bi & 0xFFFF] : 1.0;
@@ -300,7 +300,7 @@ __device__ __forceinline__ void tile_pairs(const Dev &d, const NbConst &c, const
           }
         }
       }
-      etile += sd * pair_energy_sum<ELEC, VDW>(ec, ia.qd * qjd, ljd.x, ljd.y, rd, rid);
+      etile += sd * pair_energy_sum<ELEC, VDW>(d.en, erfct, d.erfcrows, ia.qd * qjd, ljd.x, ljd.y, rd, rid);
     }
     (void)eq; (void)eA; (void)eB;
     float fr;
@@ -322,7 +322,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 // One chunk of the list: the tiles of row I it holds, against the 32
 // i-atoms in registers; the i-force partials go to the chunk's slot.
 template <int ELEC, int VDW, bool ENERGY, bool ALCH, bool SOFT>
-__device__ __forceinline__ void chunk_pairs(const Dev &d, const NbConst &c, const EnConst &ec, const float2 *s_vdw, int ch, int lane,
+__device__ __forceinline__ void chunk_pairs(const Dev &d, const NbConst &c, const double *erfct, const float2 *s_vdw, int ch, int lane,
                                             int half, int li, uint4 *sp, int2 *spr, float *slo,
                                             unsigned char *sjx, double &eacc) {
   const int4 cr = d.chunk[ch];
@@ -398,7 +398,7 @@ __device__ __forceinline__ void chunk_pairs(const Dev &d, const NbConst &c, cons
     const bool alchTile = ALCH && (hi.w | alchJc);
     const bool self = I == Jc, chk = self || ex >= 0;
 #define BM_TILE(EN, AL, SO, CK)                                                                       \
-  tile_pairs<ELEC, VDW, EN, AL, SO, CK>(d, c, ec, ia, li, half, sp, spr, slo, sjx, s_vdw, nj, emc, self, \
+  tile_pairs<ELEC, VDW, EN, AL, SO, CK>(d, c, erfct, ia, li, half, sp, spr, slo, sjx, s_vdw, nj, emc, self, \
                                         fx, fy, fz, etile)
 #define BM_TILE_CHK(EN)                  \
   if (alchTile) {                        \
@@ -507,7 +507,8 @@ __device__ __forceinline__ void cluster_pairs(const Dev &d, const NbConst &c, co
     const float dz = fdisp(ia.p.z, pj.z, sz);
     // (spelled out as the compiler contracts tile_pairs' sum)
     const float r2 = fmaf(dz, dz, fmaf(dx, dx, dy * dy));
-    bool ok = ia.t >= 0 && (ALCH ? apart_within(r2, c.rc2) : r2 < c.rc2) && p0 + q < nown;
+    bool ok = ALCH ? (ia.t >= 0) & apart_within(r2, c.rc2) & (p0 + q < nown)
+                   : ia.t >= 0 && r2 < c.rc2 && p0 + q < nown;
     if (CHK) ok = ok && !((st.em[ic >> 5][is] >> (ic & 31)) & 1u);
     float fr = 0.f;
     if (ok) {
@@ -690,9 +691,8 @@ __device__ __forceinline__ void nbdirect_kernel_body(const Dev &d, int bid, int 
   extern __shared__ __attribute__((aligned(16))) double s_tab[];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int half = lane >> 5, li = lane & 31;
-  const bool fits = *d.ntiles <= d.maxtiles && *d.nchunks <= d.maxchunks;
-  const int nchunks = fits ? *d.nchunks : 0;
-  if (bid * 4 >= nchunks) return;
+  auto chunks = [&] { return *d.ntiles <= d.maxtiles && *d.nchunks <= d.maxchunks ? *d.nchunks : 0; };
+  if (ERFC && bid * 4 >= chunks()) return;   // before its rows are staged
   float2 *s_lj = reinterpret_cast<float2 *>(s_tab + (ERFC ? d.erfcrows * kErfcTerms : 0));
   if (ERFC) {
     const double2 *src = reinterpret_cast<const double2 *>(d.erfct);
@@ -706,12 +706,7 @@ __device__ __forceinline__ void nbdirect_kernel_body(const Dev &d, int bid, int 
   if (ERFC || !GTABLE) __syncthreads();
   const float2 *s_vdw = GTABLE ? d.vdw : s_lj;
   const NbConst c = make_const(d);
-  EnConst ec;
-  if (ENERGY) ec = make_energy_const(d.rcd, d.rsd, d.betad);
-  if (ERFC) {
-    ec.erfct = s_tab;
-    ec.erfcrows = d.erfcrows;
-  }
+  const int nchunks = chunks();
   double eacc = 0.0;
   uint4 *sp = s_pos[w];
   int2 *spr = s_par[w];
@@ -723,7 +718,7 @@ __device__ __forceinline__ void nbdirect_kernel_body(const Dev &d, int bid, int 
   // count exit
   const int k = bid * 4 + w;
   if (k >= nchunks) return;
-  chunk_pairs<ELEC, VDW, ENERGY, ALCH, SOFT>(d, c, ec, s_vdw, d.corder[k], lane, half, li, sp, spr, slo, sjx, eacc);
+  chunk_pairs<ELEC, VDW, ENERGY, ALCH, SOFT>(d, c, s_tab, s_vdw, d.corder[k], lane, half, li, sp, spr, slo, sjx, eacc);
   if (ENERGY) {
     long long v = (long long)__double2ll_rn(eacc * kFixScaleD);
     wave_atomic_fix(&d.energy[BM_ENBDIRECT], v);
@@ -731,7 +726,7 @@ __device__ __forceinline__ void nbdirect_kernel_body(const Dev &d, int bid, int 
 }
 
 template <int ELEC, int VDW, bool ENERGY, bool ALCH, bool SOFT, bool GTABLE>
-__global__ void __launch_bounds__(256) nbdirect_kernel(Dev d) { nbdirect_kernel_body<ELEC, VDW, ENERGY, ALCH, SOFT, GTABLE>(d, blockIdx.x, gridDim.x); }
+__global__ void __launch_bounds__(256, ENERGY ? 4 : 1) nbdirect_kernel(Dev d) { nbdirect_kernel_body<ELEC, VDW, ENERGY, ALCH, SOFT, GTABLE>(d, blockIdx.x, gridDim.x); }
 
 template <int ELEC, int VDW, bool ENERGY, bool ALCH, bool SOFT, bool GTABLE>
 __global__ void __launch_bounds__(256) nbdirect_kernel_multi(Multi m) {

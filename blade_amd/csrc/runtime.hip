@@ -27,7 +27,6 @@
 #include <vector>
 
 #include "kernels.h"
-#include "energy64.h"
 
 // bf16 of a float, rounded to nearest even (finite values), and back
 static uint16_t bf16_rne(float f) {
@@ -516,6 +515,7 @@ int bm_system_create(int device, const bm_topology *t, const bm_runparams *rp, c
   d.rcd = rp->rcut;
   d.rsd = rp->rswitch;
   d.betad = rp->beta_ewald;
+  d.en = make_energy_const(d.rcd, d.rsd, d.betad);
   d.vdwmethod = rp->vdw_method;
   d.elecmethod = rp->elec_method;
   // domdec buffers

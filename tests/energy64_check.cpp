@@ -57,6 +57,10 @@ T plain(int elec, int vdw, T rc, T rs, T beta, T qq, T c12, T c6, T r) {
   return e;
 }
 
+// a worse approximation of 1/sqrt(x) than the hardware's (2^-23): off by up to
+// 2^-20
+double seed(double x, double w) { return (1.0 + (2 * w - 1) * 0x1p-20) / std::sqrt(x); }
+
 struct Err {
   double max = 0, sum2 = 0;
   long n = 0;
@@ -71,9 +75,7 @@ struct Err {
 
 template <int ELEC, int VDW>
 void energies(double rc, double rs, double beta, std::mt19937_64 &rng, const std::vector<double> &table, int rows) {
-  EnConst c = make_energy_const(rc, rs, beta);
-  c.erfct = table.data();
-  c.erfcrows = rows;
+  const EnConst c = make_energy_const(rc, rs, beta);
   std::uniform_real_distribution<double> u(0, 1);
   Err mine, ieee, qmine, qieee;
   for (int k = 0; k < 200000; k++) {
@@ -82,16 +84,15 @@ void energies(double rc, double rs, double beta, std::mt19937_64 &rng, const std
     if (!(d2 < rc * rc)) continue;
     const double q = 332.0716 * (u(rng) - 0.5), c12 = 6e5 * u(rng), c6 = 600 * u(rng);
     double r, ri;
-    // the hardware's approximation is good to 2^-24 or better: a float
-    sqrt_rsqrt(d2, (double)(float)(1.0 / std::sqrt(d2)), r, ri);
+    sqrt_rsqrt(d2, seed(d2, u(rng)), r, ri);
     const real R = std::sqrt((real)d2);
     // errors relative to the pair's 1/r, the size of what a sum cancels
     const real qref = plain<real>(ELEC, VDW, rc, rs, beta, q, 0, 0, R), ref = plain<real>(ELEC, VDW, rc, rs, beta, 0, c12, c6, R);
     const real qs = std::fabs(q) / R, ls = c12 / std::pow(R, (real)12) + c6 / std::pow(R, (real)6);
     const double rp = std::sqrt(d2);
-    qmine.add(pair_energy_sum<ELEC, VDW>(c, q, 0, 0, r, ri), qref, qs);
+    qmine.add(pair_energy_sum<ELEC, VDW>(c, table.data(), rows, q, 0, 0, r, ri), qref, qs);
     qieee.add(plain<double>(ELEC, VDW, rc, rs, beta, q, 0, 0, rp), qref, qs);
-    mine.add(pair_energy_sum<ELEC, VDW>(c, 0, c12, c6, r, ri), ref, ls);
+    mine.add(pair_energy_sum<ELEC, VDW>(c, table.data(), rows, 0, c12, c6, r, ri), ref, ls);
     ieee.add(plain<double>(ELEC, VDW, rc, rs, beta, 0, c12, c6, rp), ref, ls);
   }
   printf("energy %d %d %g %.4g %.4g %.4g %.4g %.4g %.4g %.4g %.4g\n", ELEC, VDW, rc, qmine.rms(), qieee.rms(), qmine.max,
@@ -125,7 +126,7 @@ int main() {
   for (int k = 0; k < 1000000; k++) {
     const double x = std::exp(12 * u(rng) - 6) ;
     double r, ri;
-    sqrt_rsqrt(x, (double)(float)(1.0 / std::sqrt(x)), r, ri);
+    sqrt_rsqrt(x, seed(x, u(rng)), r, ri);
     const real R = std::sqrt((real)x);
     s.add(r, R, R);
     si.add(ri, 1 / R, 1 / R);
